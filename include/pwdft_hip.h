@@ -68,10 +68,10 @@ enum {
   PW_TUNE_GEMM_CN_WG = 2,     /* A^H B split-K target workgroup count (0 = default 1024) */
   PW_TUNE_GEMM_NN_WG = 3,     /* A B split-K target workgroup count (0 = default 512) */
   PW_TUNE_BAND_BATCH = 4,     /* bands per fused FFT launch (same as pw_set_band_batch) */
-  PW_TUNE_PLANE_COMPRESSED = 5, /* 1: always use the compressed z-plane kernels (they are used
-                                   anyway when the padded plane does not fit in LDS); 2: always
-                                   the global-plane pass (compressed planes in HBM, used anyway
-                                   when even the compressed plane exceeds LDS) */
+  PW_TUNE_PLANE_COMPRESSED = 5, /* 1: always use the general compressed z-plane kernels (they are
+                                   used anyway for line lengths without a two-pass plan); 2:
+                                   always the global-plane pass (compressed planes in HBM, used
+                                   anyway when even the compressed plane exceeds LDS) */
   PW_TUNE_OVERLAP = 6,          /* 1 (default): op_H runs its nonlocal products on a second
                                    stream beside the FFT passes; 0: one stream, in sequence */
   PW_TUNE_COL_CHUNK = 7,        /* z-columns per workgroup of the column FFT kernels (0: the
@@ -109,7 +109,8 @@ enum {
                                    accesses, each producer waiting for its stores before the
                                    flag (n = 480: 10.8 ms, n = 960: 21.4 ms); 0 two exchanges
                                    ordered by agent-scope fences (12.2, 33.4 ms) */
-  PW_TUNE_FFT_ORDER = 15,       /* radix plan of the FFT lines: 0 (default) largest radices
+  PW_TUNE_FFT_ORDER = 15,       /* radix plan of the FFT lines outside the plane kernels, which
+                                   have their own plans: 0 (default) largest radices
                                    first (72 = 9 x 8, compile-time specialised); 1 the same
                                    radices in reverse order; 2 radices 5, 4, 3, 2 only */
   PW_TUNE_BATCH_GEMM_SMALL = 16, /* pw_zgemm_batch_dev and the batched solvers: 1 (default) the

@@ -9,6 +9,7 @@
 #include <new>
 
 #include "pw_internal.h"
+#include "pw_fft_core.h"
 
 namespace pw {
 
@@ -101,6 +102,7 @@ void free_k(KData& k) {
   hipFree(k.d_col_ij);
   hipFree(k.d_col_cy);
   hipFree(k.d_xact);
+  hipFree(k.d_ctab);
   hipFree(k.d_gk2);
   hipFree(k.d_gk);
   hipFree(k.d_gpos);
@@ -526,7 +528,7 @@ int build_kdata(pw_ctx* c, KData& k, int ngw, const int64_t* idx, int base, cons
   free_k(k);
   const int n1 = c->n1, n2 = c->n2, n3 = c->n3;
   struct Ent { int col; int z; int igw; };
-  std::map<int, int> colmap;  // plane offset -> column id (ordered by offset)
+  std::map<int, int> colmap;  // y + n2 x -> column id: the columns of one x are consecutive
   std::vector<int> keys(ngw), zs(ngw);
   std::vector<char> seen(c->N, 0);
   for (int g = 0; g < ngw; ++g) {
@@ -535,7 +537,7 @@ int build_kdata(pw_ctx* c, KData& k, int ngw, const int64_t* idx, int base, cons
     if (seen[ip]) return set_error(c, PW_ERR_ARG, std::string(who) + ": duplicate grid index");
     seen[ip] = 1;
     const int i = (int)(ip % n1), j = (int)((ip / n1) % n2), z = (int)(ip / ((int64_t)n1 * n2));
-    keys[g] = i + n1 * j;
+    keys[g] = j + n2 * i;
     zs[g] = z;
     colmap[keys[g]] = 0;
   }
@@ -545,7 +547,7 @@ int build_kdata(pw_ctx* c, KData& k, int ngw, const int64_t* idx, int base, cons
   for (auto& kv : colmap) {
     kv.second = ncol++;
     col_ij.push_back(kv.first);
-    xs.push_back(kv.first % n1);
+    xs.push_back(kv.first / n2);
   }
   std::vector<Ent> ent(ngw);
   for (int g = 0; g < ngw; ++g) ent[g] = Ent{colmap[keys[g]], zs[g], g};
@@ -559,18 +561,20 @@ int build_kdata(pw_ctx* c, KData& k, int ngw, const int64_t* idx, int base, cons
     e_pos[e] = ent[e].col * cs + ent[e].z;
     col_ptr[ent[e].col + 1]++;
   }
-  for (int cc = 0; cc < ncol; ++cc) col_ij[cc] = (col_ij[cc] % n1) + ps * (col_ij[cc] / n1);
+  for (int cc = 0; cc < ncol; ++cc) col_ij[cc] = (col_ij[cc] / n2) + ps * (col_ij[cc] % n2);
   for (int cc = 0; cc < ncol; ++cc) col_ptr[cc + 1] += col_ptr[cc];
   std::sort(xs.begin(), xs.end());
   xs.erase(std::unique(xs.begin(), xs.end()), xs.end());
-  std::vector<int> col_cy(ncol);
+  std::vector<int> col_cy(ncol), apos(n1, -1), ctab(xs.size() * n2, -1);
+  bool half = true;
   {
-    std::vector<int> apos(n1, -1);
     for (int a = 0; a < (int)xs.size(); ++a) apos[xs[a]] = a;
     const int ys = odd_stride(n2);
     int cc = 0;
     for (auto& kv : colmap) {
-      const int x = kv.first % n1, y = kv.first / n1;
+      const int x = kv.first / n2, y = kv.first % n2;
+      half = half && line_window_holds(n1, x) && line_window_holds(n2, y);
+      ctab[apos[x] * n2 + y] = cc;
       col_cy[cc++] = apos[x] * ys + y;
     }
   }
@@ -591,6 +595,7 @@ int build_kdata(pw_ctx* c, KData& k, int ngw, const int64_t* idx, int base, cons
   k.ncol = ncol;
   k.nxact = (int)xs.size();
   k.h_xact = xs;
+  k.half = half;
   int rc;
   if ((rc = upload(c, &k.d_ent_igw, e_igw.data(), ngw))) return rc;
   if ((rc = upload(c, &k.d_ent_pos, e_pos.data(), ngw))) return rc;
@@ -598,6 +603,10 @@ int build_kdata(pw_ctx* c, KData& k, int ngw, const int64_t* idx, int base, cons
   if ((rc = upload(c, &k.d_col_ij, col_ij.data(), ncol))) return rc;
   if ((rc = upload(c, &k.d_col_cy, col_cy.data(), ncol))) return rc;
   if ((rc = upload(c, &k.d_xact, xs.data(), xs.size()))) return rc;
+  const size_t ntab = ctab.size();
+  ctab.insert(ctab.end(), apos.begin(), apos.end());
+  if ((rc = upload(c, &k.d_ctab, ctab.data(), ctab.size()))) return rc;
+  k.d_apos = k.d_ctab + ntab;
   if ((rc = upload(c, &k.d_gk2, gk2.data(), ngw))) return rc;
   if ((rc = upload(c, &k.d_gk, gk, 3 * (size_t)ngw))) return rc;
   if ((rc = upload(c, &k.d_gpos, gpos.data(), ngw))) return rc;

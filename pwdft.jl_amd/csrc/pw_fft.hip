@@ -8,25 +8,24 @@
 // Three kernels per batch of bands:
 //   1. col_ifft  : scatter sphere entries into their z-columns (LDS), inverse z-FFT,
 //                  write W[b][z][col]                      (work array, in place below)
-//   2. plane_vloc: per (z-plane, band): inverse y-FFT on active x lines, inverse x-FFT on
+//   2. plane     : per (z-plane, band): inverse y-FFT on active x lines, inverse x-FFT on
 //                  all rows, * V(r)/N, forward x-FFT, forward y-FFT on active x lines,
-//                  write W[b][z][col] back                 (whole plane in LDS)
+//                  write W[b][z][col] back                 (pw_plane.h; general forms here)
 //   3. col_fft   : forward z-FFT of each column, gather the sphere entries, add the
 //                  kinetic term and write/accumulate Hpsi.
-// For calc_rhoe, kernel 2 is replaced by plane_rhoe (inverse y/x FFT, |.|^2 weighted
-// accumulation over a group of bands in registers) and a deterministic group reduction.
+// For calc_rhoe, kernel 2 ends at the weighted |.|^2 of a group of bands, with a
+// deterministic group reduction.
 //
-// Every 1-D FFT runs as Stockham radix passes (radices 2,3,4,5,8,9) on lines held in LDS;
+// The 1-D FFTs of this file run as Stockham radix passes (radices 2,3,4,5,8,9) on lines held in LDS;
 // each thread keeps its butterflies in registers across the pass barrier, so a pass is
 // done in place.  Backward (G->R) uses exp(+i), forward exp(-i), as FFTW's
 // plan_ifft!/plan_fft! (wrappers_fft.jl:42-62); the 1/N of plan_ifft! is folded into V.
 #include "pw_internal.h"
+#include "pw_fft_core.h"
+#include "pw_plane.h"
 
 namespace pw {
 
-// Launch shapes: column kernels run 512 threads holding up to COL_ME elements each across
-// a pass barrier; plane kernels run 1024 threads (16 waves on one CU, whose LDS the plane
-// fills) holding up to PLANE_ME elements each.
 #ifndef PW_COL_NT
 #define PW_COL_NT 512
 #endif
@@ -39,146 +38,13 @@ namespace pw {
 // Launch shapes: workgroups of COL_NT / PLANE_NT threads; a lane holds at most FFT_ME
 // elements of a line across one radix pass (FftDim::L lanes per line).
 constexpr int COL_NT = PW_COL_NT;
-constexpr int PLANE_NT = PW_PLANE_NT;  // FP32 planes (~41 KiB of LDS at 72^2): several workgroups per CU
-constexpr int PLANE_NT64 = PW_PLANE_NT64;  // FP64 planes fill one CU's LDS: one wide workgroup
+constexpr int PLANE_NT = PW_PLANE_NT;      // FP32 compressed planes
+constexpr int PLANE_NT64 = PW_PLANE_NT64;  // FP64 compressed planes fill one CU's LDS: one wide workgroup
 template <typename T>
 struct PlaneNT {
   static constexpr int value = sizeof(T) == 8 ? PLANE_NT64 : PLANE_NT;
 };
 constexpr int FFT_ME = 12;
-
-// ----------------------------------------------------------------------------- butterflies
-
-template <typename T, int S, int R>
-struct DFT;
-
-template <typename T, int S>
-struct DFT<T, S, 2> {
-  __device__ static inline void run(cplx<T>* v) {
-    cplx<T> a = v[0], b = v[1];
-    v[0] = a + b;
-    v[1] = a - b;
-  }
-};
-
-template <typename T, int S>
-struct DFT<T, S, 3> {
-  __device__ static inline void run(cplx<T>* v) {
-    const T c = (T)-0.5;
-    const T d = (T)(S * 0.86602540378443864676);
-    cplx<T> t1 = v[1] + v[2], t2 = v[1] - v[2];
-    cplx<T> m = v[0] + scal(c, t1);
-    cplx<T> q = mk(-d * t2.y, d * t2.x);  // i*d*t2
-    v[0] = v[0] + t1;
-    v[1] = m + q;
-    v[2] = m - q;
-  }
-};
-
-template <typename T, int S>
-struct DFT<T, S, 4> {
-  __device__ static inline void run(cplx<T>* v) {
-    cplx<T> s02 = v[0] + v[2], d02 = v[0] - v[2];
-    cplx<T> s13 = v[1] + v[3], d13 = mul_i<S>(v[1] - v[3]);
-    v[0] = s02 + s13;
-    v[2] = s02 - s13;
-    v[1] = d02 + d13;
-    v[3] = d02 - d13;
-  }
-};
-
-template <typename T, int S>
-struct DFT<T, S, 5> {
-  __device__ static inline void run(cplx<T>* v) {
-    const T c1 = (T)0.30901699437494742410, c2 = (T)-0.80901699437494742410;
-    const T s1 = (T)(S * 0.95105651629515357212), s2 = (T)(S * 0.58778525229247312917);
-    cplx<T> t1 = v[1] + v[4], t2 = v[2] + v[3], t3 = v[1] - v[4], t4 = v[2] - v[3];
-    cplx<T> a1 = v[0] + scal(c1, t1) + scal(c2, t2);
-    cplx<T> a2 = v[0] + scal(c2, t1) + scal(c1, t2);
-    cplx<T> b1 = scal(s1, t3) + scal(s2, t4);
-    cplx<T> b2 = scal(s2, t3) - scal(s1, t4);
-    cplx<T> ib1 = mk(-b1.y, b1.x), ib2 = mk(-b2.y, b2.x);
-    v[0] = v[0] + t1 + t2;
-    v[1] = a1 + ib1;
-    v[4] = a1 - ib1;
-    v[2] = a2 + ib2;
-    v[3] = a2 - ib2;
-  }
-};
-
-template <typename T, int S>
-struct DFT<T, S, 8> {
-  __device__ static inline void run(cplx<T>* v) {
-    cplx<T> e[4] = {v[0], v[2], v[4], v[6]};
-    cplx<T> o[4] = {v[1], v[3], v[5], v[7]};
-    DFT<T, S, 4>::run(e);
-    DFT<T, S, 4>::run(o);
-    const T h = (T)0.70710678118654752440;
-    // w^1 = (1 + S i)/sqrt2, w^2 = S i, w^3 = (-1 + S i)/sqrt2
-    cplx<T> o1 = mk(h * (o[1].x - S * o[1].y), h * (o[1].y + S * o[1].x));
-    cplx<T> o2 = mul_i<S>(o[2]);
-    cplx<T> o3 = mk(h * (-o[3].x - S * o[3].y), h * (-o[3].y + S * o[3].x));
-    v[0] = e[0] + o[0];
-    v[4] = e[0] - o[0];
-    v[1] = e[1] + o1;
-    v[5] = e[1] - o1;
-    v[2] = e[2] + o2;
-    v[6] = e[2] - o2;
-    v[3] = e[3] + o3;
-    v[7] = e[3] - o3;
-  }
-};
-
-template <typename T, int S>
-struct DFT<T, S, 9> {
-  __device__ static inline void run(cplx<T>* v) {
-    // 9 = 3 x 3: inner DFT3 over p (r = 3p + q), twiddle w9^(q k1), outer DFT3 over q.
-    cplx<T> y[3][3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      cplx<T> t[3] = {v[q], v[3 + q], v[6 + q]};
-      DFT<T, S, 3>::run(t);
-      y[q][0] = t[0];
-      y[q][1] = t[1];
-      y[q][2] = t[2];
-    }
-    const T c1 = (T)0.76604444311897803520, s1 = (T)(S * 0.64278760968653932632);  // w9^1
-    const T c2 = (T)0.17364817766693034885, s2 = (T)(S * 0.98480775301220805936);  // w9^2
-    const T c4 = (T)-0.93969262078590838405, s4 = (T)(S * 0.34202014332566873304); // w9^4
-    y[1][1] = cmul(y[1][1], mk(c1, s1));
-    y[1][2] = cmul(y[1][2], mk(c2, s2));
-    y[2][1] = cmul(y[2][1], mk(c2, s2));
-    y[2][2] = cmul(y[2][2], mk(c4, s4));
-#pragma unroll
-    for (int k1 = 0; k1 < 3; ++k1) {
-      cplx<T> t[3] = {y[0][k1], y[1][k1], y[2][k1]};
-      DFT<T, S, 3>::run(t);
-      v[k1] = t[0];
-      v[k1 + 3] = t[1];
-      v[k1 + 6] = t[2];
-    }
-  }
-};
-
-// Wave-local Stockham FFT.  One line (length n, element r at lds[base + r*es]) is owned by
-// a group of d.L lanes of one wavefront; a wavefront holds d.gpw groups.  Lane q of a group
-// takes butterflies q, q + L, ... of each radix pass, so no workgroup barrier is needed
-// between passes: the LDS operations of one wavefront complete in issue order, and the
-// wavefront fence keeps the compiler from moving the next pass's reads above this pass's
-// writes.  In-place: every lane reads all of its butterflies before any lane writes.
-// Ns = product of the radices already applied; tw[t] = exp(+2 pi i t / n).
-__device__ inline void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// LDS pointers keep their address space across the (non-inlined) pass so that accesses
-// compile to ds_read/ds_write rather than flat instructions.
-#if defined(__HIP_DEVICE_COMPILE__)
-#define LDS_AS __attribute__((address_space(3)))
-#else
-#define LDS_AS
-#endif
 
 template <typename T, int S, int R, int ME>
 __device__ __attribute__((noinline)) void wave_pass(LDS_AS cplx<T>* lds, int base, int es, int n, int Ns,
@@ -468,59 +334,10 @@ k_col_ifft(const cplx<double>* __restrict__ psi, long ldpsi, int b0, cplx<T>* __
                    c0, dz, twz);
 }
 
-// 2. per (z-plane, band): inverse y-FFT on the active x lines, then per x-row one wavefront
-// does inverse x-FFT, * V/N (read from L2 inside the first forward pass) and forward
-// x-FFT, then forward y-FFT on the active x lines.  In place on the plane w (ncol entries).
-template <typename T>
-__device__ inline void plane_vloc_body(cplx<T>* __restrict__ w, const T* __restrict__ V, int z,
-                                       const int* __restrict__ col_ij, int ncol, const int* __restrict__ xact,
-                                       int nxact, FftDim dx, FftDim dy, const cplx<T>* __restrict__ twx,
-                                       const cplx<T>* __restrict__ twy) {
-  extern __shared__ char smem_raw[];
-  cplx<T>* lds = reinterpret_cast<cplx<T>*>(smem_raw);
-  const int n1 = dx.n, n2 = dy.n, np = n1 * n2, ps = odd_stride(n1);
-  cplx<T>* tx = lds + ps * n2;
-  cplx<T>* ty = tx + n1;
-  int* xl = reinterpret_cast<int*>(ty + n2);
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  for (int i = tid; i < ps * n2; i += nthr) lds[i] = mk((T)0, (T)0);
-  stage(tx, twx, n1);
-  stage(ty, twy, n2);
-  stage(xl, xact, nxact);
-  __syncthreads();
-  for (int c = tid; c < ncol; c += nthr) lds[col_ij[c]] = w[c];
-  __syncthreads();
-  wave_lines<T, +1, FFT_ME>(lds, nxact, xl, 0, ps, dy, ty);
-  __syncthreads();
-  {
-    const T* v = V + (long)z * np;
-    const int lane = tid & 63, wave = tid >> 6, nwave = nthr >> 6;
-    const int g = lane / dx.L, q = lane - g * dx.L;
-    for (int t0 = wave * dx.gpw; t0 < n2; t0 += nwave * dx.gpw) {
-      const int row = t0 + g;
-      const bool active = g < dx.gpw && row < n2;
-      const int base = active ? row * ps : 0;
-      wave_row_vloc<T>(lds, base, dx, tx, q, active, v + (long)(active ? row : 0) * n1);
-    }
-  }
-  __syncthreads();
-  wave_lines<T, -1, FFT_ME>(lds, nxact, xl, 0, ps, dy, ty);
-  __syncthreads();
-  for (int c = tid; c < ncol; c += nthr) w[c] = lds[col_ij[c]];
-}
-
-template <typename T>
-__global__ void __launch_bounds__(PlaneNT<T>::value)
-k_plane_vloc(cplx<T>* __restrict__ W, const T* __restrict__ V, const int* __restrict__ col_ij,
-             int ncol, const int* __restrict__ xact, int nxact, FftDim dx, FftDim dy,
-             const cplx<T>* __restrict__ twx, const cplx<T>* __restrict__ twy, int n3) {
-  const int z = blockIdx.x, bl = blockIdx.y;
-  plane_vloc_body<T>(W + ((long)bl * n3 + z) * ncol, V, z, col_ij, ncol, xact, nxact, dx, dy, twx, twy);
-}
-
-// 2c. The plane pass for planes whose padded form does not fit in LDS (FP64 at 108^2):
-// only the active x lines are kept, compressed (Yc: nxact lines of n2, stride ys; column c
-// sits at slot col_cy[c] = a*ys + y for x = xact[a]).  The x-transform of each row runs in a
+// 2c. The plane pass where the line lengths have no two-pass plan (125, 162, ...) or
+// PW_TUNE_PLANE_COMPRESSED asks for it; otherwise pw_plane.h runs.  Only the active x lines are
+// kept, compressed (Yc: nxact lines of n2, stride ys; column c sits at slot col_cy[c] =
+// a*ys + y for x = xact[a]).  The x-transform of each row runs in a
 // per-wavefront row buffer of n1 entries: the row is expanded from Yc (zero at inactive x),
 // transformed (inverse, * V/N, forward) and its active entries gathered back.  rl rows are
 // in flight per wavefront (rl <= gpw, sized to the LDS left after Yc).
@@ -648,39 +465,6 @@ k_plane_rhoe_c(const cplx<T>* __restrict__ W, const double* __restrict__ wts, in
 // G->R of real fields on a sphere (FP64), after k_col_ifft: per (z-plane, field) the inverse
 // y-FFT of the active x lines and the inverse x-FFT of every row, then
 // out[f N + r] = scale Re f(r) (added to out when acc is set).
-__global__ void __launch_bounds__(PlaneNT<double>::value)
-k_plane_g2r(const cplx<double>* __restrict__ W, double* __restrict__ out, long N, double scale, int acc,
-            const int* __restrict__ col_ij, int ncol, const int* __restrict__ xact, int nxact, FftDim dx, FftDim dy,
-            const cplx<double>* __restrict__ twx, const cplx<double>* __restrict__ twy, int n3) {
-  extern __shared__ char smem_raw[];
-  cplx<double>* lds = reinterpret_cast<cplx<double>*>(smem_raw);
-  const int n1 = dx.n, n2 = dy.n, np = n1 * n2, ps = odd_stride(n1);
-  cplx<double>* tx = lds + ps * n2;
-  cplx<double>* ty = tx + n1;
-  int* xl = reinterpret_cast<int*>(ty + n2);
-  const int z = blockIdx.x, f = blockIdx.y;
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  for (int i = tid; i < ps * n2; i += nthr) lds[i] = mk(0.0, 0.0);
-  stage(tx, twx, n1);
-  stage(ty, twy, n2);
-  stage(xl, xact, nxact);
-  __syncthreads();
-  const cplx<double>* w = W + ((long)f * n3 + z) * ncol;
-  for (int c = tid; c < ncol; c += nthr) lds[col_ij[c]] = w[c];
-  __syncthreads();
-  wave_lines<double, +1, FFT_ME>(lds, nxact, xl, 0, ps, dy, ty);
-  __syncthreads();
-  wave_lines<double, +1, FFT_ME>(lds, n2, nullptr, ps, 1, dx, tx);
-  __syncthreads();
-  double* o = out + (long)f * N + (long)z * np;
-  for (int i = tid; i < np; i += nthr) {
-    const int j = i / n1, x = i - j * n1;
-    const double v = scale * lds[x + ps * j].x;
-    o[i] = acc ? o[i] + v : v;
-  }
-}
-
-// The same for planes beyond LDS, in the compressed form of k_plane_vloc_c.
 __global__ void __launch_bounds__(PlaneNT<double>::value)
 k_plane_g2r_c(const cplx<double>* __restrict__ W, double* __restrict__ out, long N, double scale, int acc,
               const int* __restrict__ col_cy, int ncol, const int* __restrict__ xact, int nxact, FftDim dx,
@@ -862,17 +646,6 @@ k_col_ifft_batch(const KBatch* __restrict__ kb, int nk, int nb, cplx<T>* __restr
 }
 
 template <typename T>
-__global__ void __launch_bounds__(PlaneNT<T>::value)
-k_plane_vloc_batch(const KBatch* __restrict__ kb, int nb, cplx<T>* __restrict__ W, const T* __restrict__ V,
-                   FftDim dx, FftDim dy, const cplx<T>* __restrict__ twx, const cplx<T>* __restrict__ twy,
-                   int n3) {
-  const int z = blockIdx.x, kk = blockIdx.y / nb, bl = blockIdx.y - kk * nb;
-  const KBatch& d = kb[kk];
-  plane_vloc_body<T>(W + d.woff + ((long)bl * n3 + z) * d.ncol, V, z, d.col_ij, d.ncol, d.xact, d.nxact, dx, dy,
-                     twx, twy);
-}
-
-template <typename T>
 __global__ void __launch_bounds__(COL_NT)
 k_col_fft_batch(const KBatch* __restrict__ kb, int nk, int nb, const cplx<T>* __restrict__ W, int C, FftDim dz,
                 const cplx<T>* __restrict__ twz, int kin, int acc) {
@@ -882,62 +655,6 @@ k_col_fft_batch(const KBatch* __restrict__ kb, int nk, int nb, const cplx<T>* __
   if (!batch_col_block(d, C, nb, w - d.blk0, c0, bl)) return;
   col_fft_body<T>(W + d.woff + (long)bl * dz.n * d.ncol, d.psi + (long)bl * d.ldpsi, d.hpsi + (long)bl * d.ldh,
                   d.ent_igw, d.ent_pos, d.col_ptr, d.ncol, C, c0, dz, twz, d.gk2, kin, acc);
-}
-
-// rho planes: per (z-plane, band group): y/x inverse FFT of each band and
-// sum_b w_b |psi_b(r)|^2 accumulated in registers (plane point tid + r * blockDim.x in
-// register r, NR <= RHO_REGS per thread: the launch picks the smallest NR that covers the
-// plane, so no accumulator registers go unused); one partial plane per group.
-constexpr int RHO_REGS = 16;
-template <typename T, int NR>
-__global__ void __launch_bounds__(PlaneNT<T>::value)
-k_plane_rhoe(const cplx<T>* __restrict__ W, const double* __restrict__ wts, int nb, int bpg,
-             double* __restrict__ rpart, long N, const int* __restrict__ col_ij, int ncol,
-             const int* __restrict__ xact, int nxact, FftDim dx, FftDim dy,
-             const cplx<T>* __restrict__ twx, const cplx<T>* __restrict__ twy, int n3) {
-  extern __shared__ char smem_raw[];
-  cplx<T>* lds = reinterpret_cast<cplx<T>*>(smem_raw);
-  const int n1 = dx.n, n2 = dy.n, np = n1 * n2, ps = odd_stride(n1);
-  cplx<T>* tx = lds + ps * n2;
-  cplx<T>* ty = tx + n1;
-  int* xl = reinterpret_cast<int*>(ty + n2);
-  const int z = blockIdx.x, g = blockIdx.y;
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  stage(tx, twx, n1);
-  stage(ty, twy, n2);
-  stage(xl, xact, nxact);
-  double acc[NR];
-#pragma unroll
-  for (int r = 0; r < NR; ++r) acc[r] = 0.0;
-  const int bend = min(nb, (g + 1) * bpg);
-  for (int b = g * bpg; b < bend; ++b) {
-    for (int i = tid; i < ps * n2; i += nthr) lds[i] = mk((T)0, (T)0);
-    __syncthreads();
-    const cplx<T>* w = W + ((long)b * n3 + z) * ncol;
-    for (int c = tid; c < ncol; c += nthr) lds[col_ij[c]] = w[c];
-    __syncthreads();
-    wave_lines<T, +1, FFT_ME>(lds, nxact, xl, 0, ps, dy, ty);
-    __syncthreads();
-    wave_lines<T, +1, FFT_ME>(lds, n2, nullptr, ps, 1, dx, tx);
-    __syncthreads();
-    const double wb = wts[b];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const int i = tid + r * nthr;
-      if (i < np) {
-        const int j = i / n1, x = i - j * n1;
-        const double re = (double)lds[x + ps * j].x, im = (double)lds[x + ps * j].y;
-        acc[r] += wb * (re * re + im * im);
-      }
-    }
-    __syncthreads();
-  }
-  double* out = rpart + (long)g * N + (long)z * np;
-#pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    const int i = tid + r * nthr;
-    if (i < np) out[i] = acc[r];
-  }
 }
 
 __global__ void k_rho_reduce(double* __restrict__ rho, const double* __restrict__ rpart, int ng,
@@ -988,18 +705,6 @@ static bool lanes_ok(const FftDim& d) { return d.L >= 1 && d.L <= 64 && d.gpw >=
 static size_t plane_lds(const pw_ctx* c, size_t esz, int nxact) {
   return ((size_t)odd_stride(c->n1) * c->n2 + c->n1 + c->n2) * esz + (size_t)nxact * sizeof(int);
 }
-// Threads of a padded-plane workgroup (the kernels index by blockDim.x): wavefronts for one
-// pass over the plane's lines, max(nxact y lines, n2 x rows) / lines per wavefront, when that
-// is at most half of PlaneNT.  Small planes (20^2: one wavefront) then fit many workgroups
-// per CU instead of one or two mostly idle ones; large planes keep PlaneNT.
-template <typename T>
-static int plane_threads(const pw_ctx* c, int nxact) {
-  const FftDim& dx = c->dim[0];
-  const FftDim& dy = c->dim[1];
-  const int waves = std::max(1, std::max((nxact + dy.gpw - 1) / dy.gpw, (c->n2 + dx.gpw - 1) / dx.gpw));
-  return 2 * 64 * waves <= PlaneNT<T>::value ? 64 * waves : PlaneNT<T>::value;
-}
-
 // Threads of a column workgroup holding C columns: wavefronts for one pass over its C lines
 // when that is at most half of COL_NT, else COL_NT (the column kernels index by blockDim.x).
 static int col_threads(const pw_ctx* c, int C) {
@@ -1051,9 +756,9 @@ static int vloc_run(pw_ctx* c, KData& k, const T* V, int nb, const cplx<double>*
   // an XCD at once and Hpsi's scattered rows merge in L2 (Si64: 151 -> 87 MB written per
   // launch); W's layout does not depend on the chunk
   const int Cf = (sizeof(T) == 4 && c->tune_col_chunk <= 0) ? std::min(C, 32) : C;
-  size_t plane_bytes = plane_lds(c, esz, k.nxact);
+  size_t plane_bytes = 0;
   int rl = 0;
-  const bool compressed = plane_bytes > 160 * 1024 || c->plane_compressed != 0;
+  const bool compressed = !plane_applies<T>(c, k.nxact, k.half);
   PlaneGP gp;
   bool global_plane = false;
   if (compressed) {
@@ -1108,8 +813,7 @@ static int vloc_run(pw_ctx* c, KData& k, const T* V, int nb, const cplx<double>*
         hipLaunchKernelGGL(k_plane_vloc_c<T>, g2, dim3(PlaneNT<T>::value), plane_bytes, c->stream, W, V,
                            k.d_col_cy, k.ncol, k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0], tw[1], c->n3, rl);
       else
-        hipLaunchKernelGGL(k_plane_vloc<T>, g2, dim3(plane_threads<T>(c, k.nxact)), plane_bytes, c->stream, W, V,
-                           k.d_col_ij, k.ncol, k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0], tw[1], c->n3);
+        plane_vloc<T>(c, k, W, V, nbb);
     }
     if (join && b0 == 0) {
       hipError_t e = hipStreamWaitEvent(c->stream, join, 0);
@@ -1159,14 +863,15 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
   long woff = 0;
   long blk = 0;
   int maxx = 0;
+  bool half = true;
   for (int kk = 0; kk < nk; ++kk) {
     const KData& k = c->kd[iks[kk]];
     KBatch d{};
     d.ent_igw = k.d_ent_igw;
     d.ent_pos = k.d_ent_pos;
     d.col_ptr = k.d_col_ptr;
-    d.col_ij = k.d_col_ij;
-    d.xact = k.d_xact;
+    d.ctab = k.d_ctab;
+    d.apos = k.d_apos;
     d.gk2 = k.d_gk2;
     d.psi = psi[kk];
     d.hpsi = hpsi[kk];
@@ -1180,11 +885,16 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
     woff += (long)nb * c->n3 * k.ncol;
     blk += (long)((k.ncol + C - 1) / C) * nb8;
     maxx = std::max(maxx, k.nxact);
+    half = half && k.half;
   }
   if (blk > 0x7fffffffL) return set_error(c, PW_ERR_ARG, "op_H batch too large for one launch");
-  const size_t plane_bytes = plane_lds(c, esz, maxx);
-  if (plane_bytes > 160 * 1024)
+  if (plane_lds(c, esz, maxx) > 160 * 1024)
     return set_error(c, PW_ERR_ARG, "z-plane does not fit in LDS for this precision");
+  // without a plane kernel for these lengths, the compressed planes k-point after k-point
+  const bool planes = plane_applies<T>(c, maxx, half);
+  size_t plane_bytes = 0;
+  const int rl = planes ? 0 : plane_c_rows(c, esz, maxx, PlaneNT<T>::value, &plane_bytes);
+  if (!planes && rl < 1) return set_error(c, PW_ERR_ARG, "z-plane does not fit in LDS for this precision");
   int rc = ensure(c, &c->d_work, &c->work_bytes, (size_t)woff * esz);
   if (rc) return rc;
   const void* dptr = nullptr;
@@ -1197,8 +907,15 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
     tw[d] = reinterpret_cast<const cplx<T>*>(sizeof(T) == 8 ? c->d_tw64[d] : c->d_tw32[d]);
   hipLaunchKernelGGL(k_col_ifft_batch<T>, dim3((unsigned)blk), dim3(cnt), col_lds(c, C, esz), c->stream, dkb,
                      nk, nb, W, C, c->dim[2], tw[2]);
-  hipLaunchKernelGGL(k_plane_vloc_batch<T>, dim3(c->n3, nk * nb), dim3(plane_threads<T>(c, maxx)), plane_bytes, c->stream,
-                     dkb, nb, W, V, c->dim[0], c->dim[1], tw[0], tw[1], c->n3);
+  if (planes)
+    plane_vloc_batch<T>(c, dkb, nk, nb, maxx, half, W, V);
+  else
+    for (int kk = 0; kk < nk; ++kk) {
+      const KData& k = c->kd[iks[kk]];
+      hipLaunchKernelGGL(k_plane_vloc_c<T>, dim3(c->n3, nb), dim3(PlaneNT<T>::value), plane_bytes, c->stream,
+                         W + kb[kk].woff, V, k.d_col_cy, k.ncol, k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0], tw[1],
+                         c->n3, rl);
+    }
   hipLaunchKernelGGL(k_col_fft_batch<T>, dim3((unsigned)blk), dim3(cnt), col_lds(c, C, esz), c->stream, dkb, nk,
                      nb, W, C, c->dim[2], tw[2], kin, acc);
   return hip_check(c, hipGetLastError(), "batched vloc kernels");
@@ -1727,13 +1444,9 @@ static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldp
   KData& k = c->kd[ik];
   const size_t esz = sizeof(cplx<T>);
   const int C = cols_per_block(c, esz);
-  const int np = c->n1 * c->n2;
-  size_t plane_bytes = plane_lds(c, esz, k.nxact);
+  size_t plane_bytes = 0;
   int rl = 0;
-  // the padded-plane kernel keeps each thread's share of the plane (<= RHO_REGS points) in
-  // registers; planes beyond that take the compressed kernel, which accumulates in HBM
-  const bool compressed = plane_bytes > 160 * 1024 || c->plane_compressed != 0 ||
-                          np > RHO_REGS * PlaneNT<T>::value;
+  const bool compressed = !(k.half && plane_applies<T>(c, k.nxact, true));
   if (compressed) {
     rl = plane_c_rows(c, esz, k.nxact, PlaneNT<T>::value, &plane_bytes);
     if (rl < 1) return set_error(c, PW_ERR_ARG, "z-plane too large for calc_rhoe kernel");
@@ -1765,17 +1478,8 @@ static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldp
       hipLaunchKernelGGL(k_plane_rhoe_c<T>, dim3(c->n3, ngu), dim3(PlaneNT<T>::value), plane_bytes, c->stream, W,
                          d_w + b0, nbb, bpg, reinterpret_cast<double*>(c->d_rpart), c->N, k.d_col_cy, k.ncol,
                          k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0], tw[1], c->n3, rl);
-    else {
-      // the plane's points over the threads, at most RHO_REGS each (np <= RHO_REGS * PlaneNT here)
-      int nt = plane_threads<T>(c, k.nxact);
-      while ((np + nt - 1) / nt > RHO_REGS) nt += 64;
-      const int nr = (np + nt - 1) / nt;
-      auto kern = nr <= 4 ? k_plane_rhoe<T, 4> : nr <= 6 ? k_plane_rhoe<T, 6> : nr <= 8 ? k_plane_rhoe<T, 8>
-                : nr <= 12 ? k_plane_rhoe<T, 12> : k_plane_rhoe<T, RHO_REGS>;
-      hipLaunchKernelGGL(kern, dim3(c->n3, ngu), dim3(nt), plane_bytes, c->stream, W, d_w + b0, nbb,
-                         bpg, reinterpret_cast<double*>(c->d_rpart), c->N, k.d_col_ij, k.ncol, k.d_xact, k.nxact,
-                         c->dim[0], c->dim[1], tw[0], tw[1], c->n3);
-    }
+    else
+      plane_rho<T>(c, k, W, nbb, bpg, ngu, d_w + b0, reinterpret_cast<double*>(c->d_rpart));
     hipLaunchKernelGGL(k_rho_reduce, dim3(1024), dim3(256), 0, c->stream, c->d_rho,
                        reinterpret_cast<const double*>(c->d_rpart), ngu, c->N, 1.0 / c->omega);
   }
@@ -1786,9 +1490,9 @@ int g2r_apply(pw_ctx* c, KData& k, int nf, const cplx<double>* fG, long ldf, dou
               int acc) {
   const size_t esz = sizeof(cplx<double>);
   const int C = cols_per_block(c, esz);
-  size_t plane_bytes = plane_lds(c, esz, k.nxact);
+  size_t plane_bytes = 0;
   int rl = 0;
-  const bool compressed = plane_bytes > 160 * 1024 || c->plane_compressed != 0;
+  const bool compressed = !plane_applies<double>(c, k.nxact, false);
   PlaneGP gp;
   bool global_plane = false;
   if (compressed) {
@@ -1836,9 +1540,7 @@ int g2r_apply(pw_ctx* c, KData& k, int nf, const cplx<double>* fG, long ldf, dou
                          o, c->N, scale, acc, k.d_col_cy, k.ncol, k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0],
                          tw[1], c->n3, rl);
     else
-      hipLaunchKernelGGL(k_plane_g2r, dim3(c->n3, nbb), dim3(plane_threads<double>(c, k.nxact)), plane_bytes, c->stream, W, o,
-                         c->N, scale, acc, k.d_col_ij, k.ncol, k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0],
-                         tw[1], c->n3);
+      plane_real(c, k, W, nbb, o, scale, acc);
   }
   return hip_check(c, hipGetLastError(), "G->R kernels");
 }

@@ -77,10 +77,10 @@ inline void plan_lanes(FftDim& d, int me) {
 }
 
 // LDS strides: odd line lengths keep strided butterfly reads off a single bank group.
-__host__ __device__ inline int odd_stride(int n) { return (n % 2 == 0) ? n + 1 : n; }
+__host__ __device__ constexpr int odd_stride(int n) { return (n % 2 == 0) ? n + 1 : n; }
 
 // Sphere bookkeeping of one k-point.  Sphere entries are sorted by (column, z);
-// a column is one (x, y) pair that holds at least one entry.
+// a column is one (x, y) pair that holds at least one entry, columns sorted by (x, y).
 struct KData {
   int ngw = 0;
   int ncol = 0;
@@ -92,6 +92,9 @@ struct KData {
   int* d_col_ij = nullptr;    // [ncol]  i + pstride * j (LDS slot inside a padded z-plane)
   int* d_col_cy = nullptr;    // [ncol]  a * ystride + j, x = xact[a] (slot in a compressed plane)
   int* d_xact = nullptr;      // [nxact] distinct x of the columns
+  int* d_ctab = nullptr;      // [nxact * n2] column of (a, y), x = xact[a], or -1
+  int* d_apos = nullptr;      // [n1]    a of x, or -1 (in d_ctab's allocation)
+  bool half = false;          // every x and y lies in the half-sphere window of its line plan (pw_plane.h)
   double* d_gk2 = nullptr;    // [ngw]   |G+k|^2
   double* d_gk = nullptr;     // [3*ngw] G+k (x,y,z per entry, column-major 3 x ngw)
   int* d_gpos = nullptr;      // [ngw]   psi row -> x + ps (y + n2 z), ps = odd_stride(n1): slot in a whole padded grid
@@ -108,8 +111,8 @@ struct KBatch {
   const int* ent_igw;
   const int* ent_pos;
   const int* col_ptr;
-  const int* col_ij;
-  const int* xact;
+  const int* ctab;
+  const int* apos;
   const double* gk2;
   const cplx<double>* psi;
   cplx<double>* hpsi;

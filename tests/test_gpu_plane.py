@@ -1,0 +1,98 @@
+"""The plane kernels (csrc/pw_plane.h) through the C ABI against numpy's FFT: every line
+length with a two-pass plan, lengths without one, unequal lengths, index sets inside and
+outside the half-sphere window, and density groups of several bands.  Tolerances are those
+of the operator tests: 1e-12 (FP64) and 2e-5 (mixed) of the largest value."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+PLANS = [12, 15, 16, 18, 20, 24, 25, 27, 30, 32, 36, 40, 45, 48, 50, 54, 60, 64, 72, 75, 80, 81, 90, 96, 100, 108,
+         120, 128, 135, 144, 150, 160, 180, 192]
+
+
+def index_set(ns, radius, shift=0.3):
+    """Grid points of an ellipsoid of the given half axes, off centre by `shift` points."""
+    m = [np.where(np.arange(n) > n // 2, np.arange(n) - n, np.arange(n)) for n in ns]
+    r2 = sum((((a - shift) / max(r, 0.5)) ** 2).reshape([-1 if d == i else 1 for i in range(3)])
+             for d, (a, r) in enumerate(zip(m, radius)))
+    x, y, z = np.nonzero(r2 <= 1.0)
+    idx = np.sort(x + ns[0] * (y + ns[1] * z))
+    return np.random.default_rng(5).permutation(idx).astype(np.int64)
+
+
+def context(ns, idx, omega=3.7):
+    import pwdft_hip as ph
+    from pwdft_hip._lib import ptr
+    c = ph.Context()
+    c.call("pw_set_grid", *ns, omega)
+    c.call("pw_set_band_batch", 64)
+    gk = np.random.default_rng(6).standard_normal((idx.size, 3))
+    c.call("pw_set_kpoint", 0, idx.size, ptr(idx), 0, ptr(gk))
+    return c
+
+
+def apply_v(c, ns, idx, V, psi, mixed):
+    from pwdft_hip._lib import PW_MIXED, PW_TERM_VLOC, ptr
+    c.call("pw_set_vloc", 0, ptr(V))
+    out = np.zeros_like(psi)
+    c.call("pw_op_H", 0, 0, psi.shape[1], ptr(psi), psi.shape[0], ptr(out), out.shape[0],
+           PW_TERM_VLOC | (PW_MIXED if mixed else 0))
+    f = np.zeros((psi.shape[1], ns[2], ns[1], ns[0]), dtype=complex)
+    f.reshape(psi.shape[1], -1)[:, idx] = psi.T
+    f = np.fft.fftn(np.fft.ifftn(f, axes=(1, 2, 3)) * V.reshape(ns[2], ns[1], ns[0]), axes=(1, 2, 3))
+    return out, f.reshape(psi.shape[1], -1)[:, idx].T
+
+
+def rand(rng, n, nb):
+    return np.asfortranarray(rng.standard_normal((n, nb)) + 1j * rng.standard_normal((n, nb)))
+
+
+VLOC = [((n, n, 12), "half", m) for n in PLANS for m in (False, True)]
+VLOC += [((n, n, 12), "full", False) for n in (12, 20, 27, 45, 72, 75, 96)]
+VLOC += [((n, n, 12), "full", True) for n in (27, 72)]
+VLOC += [((40, 75, 12), "half", m) for m in (False, True)] + [((75, 40, 12), "half", m) for m in (False, True)]
+VLOC += [((108, 64, 16), "half", False), ((27, 160, 12), "half", True), ((45, 36, 12), "full", False)]
+VLOC += [((125, 8, 12), "half", False), ((10, 125, 12), "half", True), ((5, 6, 4), "full", False)]
+
+
+@pytest.mark.parametrize("ns,extent,mixed", VLOC)
+def test_vloc_plane(ns, extent, mixed):
+    idx = index_set(ns, [((n - 1) // 4) if extent == "half" else n // 2 - 0.6 for n in ns])
+    c = context(ns, idx)
+    rng = np.random.default_rng(1)
+    V = rng.standard_normal(int(np.prod(ns)))
+    print(f"case {ns} {extent} mixed={mixed}", flush=True)
+    got, ref = apply_v(c, ns, idx, V, rand(rng, idx.size, 3), mixed)
+    assert np.abs(got - ref).max() <= (2e-5 if mixed else 1e-12) * np.abs(ref).max()
+    c.close()
+
+
+RHO = [((n, n, 120), m) for n in (15, 24, 27, 45, 72, 75) for m in (False, True)]
+RHO += [((108, 108, 120), False), ((135, 135, 150), True), ((40, 75, 120), True), ((75, 27, 120), False)]
+
+
+@pytest.mark.parametrize("ns,mixed", RHO)
+def test_rho_groups(ns, mixed):
+    """More bands than groups, so a workgroup carries its plane state over several bands."""
+    from pwdft_hip._lib import PW_MIXED, ptr
+    idx = index_set(ns, [(n - 1) // 4 for n in ns])
+    c = context(ns, idx)
+    rng = np.random.default_rng(2)
+    nb = 16
+    psi = rand(rng, idx.size, nb)
+    w = rng.random(nb)
+    N = int(np.prod(ns))
+    print(f"case rho {ns} mixed={mixed}", flush=True)
+    c.call("pw_rhoe_zero")
+    c.call("pw_rhoe_accum", 0, nb, ptr(psi), idx.size, ptr(w), PW_MIXED if mixed else 0)
+    got = np.empty(N)
+    c.call("pw_rhoe_get", ptr(got))
+    ref = np.zeros(N)
+    for b in range(nb):
+        f = np.zeros(N, dtype=complex)
+        f[idx] = psi[:, b]
+        ref += w[b] * np.abs(np.fft.ifftn(f.reshape(ns[2], ns[1], ns[0])).reshape(-1)) ** 2
+    ref *= float(N) ** 2 / 3.7
+    assert np.abs(got - ref).max() <= (2e-5 if mixed else 1e-12) * np.abs(ref).max()
+    c.close()
