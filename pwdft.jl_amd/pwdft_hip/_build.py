@@ -20,7 +20,7 @@ OUT = os.path.join(HERE, "libpwdft_hip.so")
 EXTRA_FLAGS = {s: ["-fno-signed-zeros"] for s in SOURCES if s.startswith("pw_plane_")}
 
 HIPCC_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
     "-Wno-unused-value", "-Wno-unused-result",
     # keep hipcc from emitting packed FP32 instructions
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -43,11 +43,11 @@ def build_library(verbose=False):
     # one object per source, compiled side by side
     with tempfile.TemporaryDirectory() as td:
         objs = [os.path.join(td, s.replace(".hip", ".o")) for s in SOURCES]
-        jobs = [[hipcc] + HIPCC_FLAGS + EXTRA_FLAGS.get(s, []) + ["-c", "-o", o, os.path.join(CSRC, s)]
+        jobs = [[hipcc] + [f for f in HIPCC_FLAGS if f != "-shared"] + EXTRA_FLAGS.get(s, []) + ["-c", "-o", o, os.path.join(CSRC, s)]
                 for s, o in zip(SOURCES, objs)]
         with ThreadPoolExecutor(max_workers=max(1, min(8, os.cpu_count() or 1))) as pool:
             list(pool.map(run, sorted(jobs, key=lambda j: "pw_plane_" not in j[-1])))
-        run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp] + objs + LIBS)
+        run([hipcc] + HIPCC_FLAGS + ["-o", tmp] + objs + LIBS)
     n = check_no_packed_fp32(tmp)
     os.replace(tmp, OUT)
     if verbose:
