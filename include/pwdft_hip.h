@@ -213,6 +213,11 @@ int pw_rhoe_accum(pw_ctx* ctx, int ik, int nb, const void* psi, int64_t ldpsi, c
                   unsigned flags);
 int pw_rhoe_accum_dev(pw_ctx* ctx, int ik, int nb, const void* psi, int64_t ldpsi, const double* w,
                       unsigned flags);
+/* pw_rhoe_accum_dev for several k-points (the k loop of calc_rhoe.jl:38-80): k-point iks[i] adds
+ * the nb bands psi[i] (Ngw[iks[i]] x nb, leading dimension ldpsi[i]) with weights w[i nb + ist]
+ * (host array).  The bands of as many k-points as 256 MiB of transforms hold share each launch. */
+int pw_rhoe_accum_batch_dev(pw_ctx* ctx, int nk, const int* iks, int nb, void* const* psi, const int64_t* ldpsi,
+                            const double* w, unsigned flags);
 int pw_rhoe_get(pw_ctx* ctx, double* rho);
 /* Copy of the accumulated density into a device array (N doubles). */
 int pw_rhoe_get_dev(pw_ctx* ctx, double* rho);

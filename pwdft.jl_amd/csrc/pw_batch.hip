@@ -369,7 +369,7 @@ using namespace pw;
 #define CTX_CHECK(c) \
   if (!(c)) return PW_ERR_ARG
 
-static int check_batch_k(pw_ctx* c, int nk, const int* iks) {
+int pw::check_batch_k(pw_ctx* c, int nk, const int* iks) {
   if (c->N == 0) return set_error(c, PW_ERR_STATE, "pw_set_grid has not been called");
   if (nk < 0 || (nk > 0 && !iks)) return set_error(c, PW_ERR_ARG, "batch: bad k-point list");
   for (int kk = 0; kk < nk; ++kk)

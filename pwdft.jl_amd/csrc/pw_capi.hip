@@ -779,6 +779,29 @@ int pw_rhoe_accum_dev(pw_ctx* c, int ik, int nb, const void* psi, int64_t ldpsi,
   return hip_check(c, hipStreamSynchronize(c->stream), "rhoe");
 }
 
+int pw_rhoe_accum_batch_dev(pw_ctx* c, int nk, const int* iks, int nb, void* const* psi, const int64_t* ldpsi,
+                            const double* w, unsigned flags) {
+  CTX_CHECK(c);
+  hipSetDevice(c->device);
+  int rc = check_batch_k(c, nk, iks);
+  if (rc) return rc;
+  if (nb < 0) return set_error(c, PW_ERR_ARG, "rhoe batch: nb < 0");
+  if (nk == 0 || nb == 0) return PW_OK;
+  if (!psi || !ldpsi || !w) return set_error(c, PW_ERR_ARG, "rhoe batch: null argument");
+  for (int kk = 0; kk < nk; ++kk)
+    if (!psi[kk] || ldpsi[kk] < c->kd[iks[kk]].ngw)
+      return set_error(c, PW_ERR_ARG, "rhoe batch: bad pointer or leading dimension");
+  const size_t wb = (size_t)nk * nb * sizeof(double);
+  rc = ensure(c, &c->d_wts, &c->wts_bytes, wb);
+  if (rc) return rc;
+  double* dw = reinterpret_cast<double*>(c->d_wts);
+  hipError_t e = hipMemcpyAsync(dw, w, wb, hipMemcpyHostToDevice, c->stream);
+  if (e != hipSuccess) return hip_check(c, e, "rhoe weights upload");
+  rc = rhoe_accum_batch(c, nk, iks, nb, reinterpret_cast<const cplx<double>* const*>(psi), ldpsi, dw, flags);
+  if (rc) return rc;
+  return hip_check(c, hipStreamSynchronize(c->stream), "rhoe batch");
+}
+
 int pw_rhoe_accum(pw_ctx* c, int ik, int nb, const void* psi, int64_t ldpsi, const double* w, unsigned flags) {
   CTX_CHECK(c);
   hipSetDevice(c->device);

@@ -661,6 +661,7 @@ __global__ void k_rho_reduce(double* __restrict__ rho, const double* __restrict_
                              long N, double scale) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) {
     double s = 0.0;
+#pragma unroll 8
     for (int g = 0; g < ng; ++g) s += rpart[(long)g * N + i];
     rho[i] += scale * s;
   }
@@ -1439,6 +1440,12 @@ int kprec_apply(pw_ctx* c, int ik, int nb, const cplx<double>* in, long ldin, cp
   return hip_check(c, hipGetLastError(), "k_kprec");
 }
 
+// Groups that the bands of a density launch are split into: one round of workgroups, per_cu of
+// them on each of the 256 CUs, over the n3 planes.
+static int rho_groups(const pw_ctx* c, int per_cu, int nb) {
+  return std::max(1, std::min(nb, (256 * per_cu + c->n3 - 1) / c->n3));
+}
+
 template <typename T>
 static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldpsi, const double* d_w) {
   KData& k = c->kd[ik];
@@ -1456,9 +1463,9 @@ static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldp
   const int bb = std::max(1, std::min(nb, c->band_batch));
   int rc = ensure(c, &c->d_work, &c->work_bytes, (size_t)bb * c->n3 * k.ncol * esz);
   if (rc) return rc;
-  // band groups: about one round of resident plane workgroups (3 per CU on 256 CUs) over the
-  // n3 planes; each group's partial plane is reduced afterwards in a fixed order
-  int ngroup = std::max(1, std::min(bb, (768 + c->n3 - 1) / c->n3));
+  // band groups: about one round of resident plane workgroups over the n3 planes; each group's
+  // partial plane is reduced afterwards in a fixed order
+  const int ngroup = rho_groups(c, compressed ? 3 : plane_rho_resident<T>(c, k.nxact), bb);
   rc = ensure(c, &c->d_rpart, &c->rpart_bytes, (size_t)ngroup * c->N * sizeof(double));
   if (rc) return rc;
   cplx<T>* W = reinterpret_cast<cplx<T>*>(c->d_work);
@@ -1484,6 +1491,83 @@ static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldp
                        reinterpret_cast<const double*>(c->d_rpart), ngu, c->N, 1.0 / c->omega);
   }
   return hip_check(c, hipGetLastError(), "rhoe kernels");
+}
+
+// Every band of the k-points iks: one column launch, one plane launch and one reduction for as
+// many k-points as 256 MiB of W hold (at least two; else k-point after k-point).  A k-point of a
+// metal's mesh is a few bands on a small grid, so its three launches and the wait after them
+// took ~32 us whatever their work (Al fcc, 20^3, 8 bands, 182 k-points: 5.8 -> 0.2 ms).
+template <typename T>
+static int rhoe_batch_run(pw_ctx* c, int nk, const int* iks, int nb, const cplx<double>* const* psi,
+                          const int64_t* ldpsi, const double* d_w) {
+  const size_t esz = sizeof(cplx<T>);
+  int maxcol = 1, maxx = 1;
+  bool half = true;
+  for (int kk = 0; kk < nk; ++kk) {
+    const KData& k = c->kd[iks[kk]];
+    maxcol = std::max(maxcol, k.ncol);
+    maxx = std::max(maxx, k.nxact);
+    half = half && k.half;
+  }
+  const size_t kbytes = (size_t)nb * c->n3 * maxcol * esz;
+  const int kc = (int)std::min<size_t>(nk, (256u << 20) / kbytes);
+  if (kc < 2 || !half || !plane_applies<T>(c, maxx, true) || !lanes_ok(c->dim[2])) {
+    for (int kk = 0; kk < nk; ++kk) {
+      int rc = rhoe_run<T>(c, iks[kk], nb, psi[kk], ldpsi[kk], d_w + (size_t)kk * nb);
+      if (rc) return rc;
+    }
+    return PW_OK;
+  }
+  const int C = std::min(cols_per_block(c, esz), maxcol), cnt = col_threads(c, C), nb8 = (nb + 7) / 8 * 8;
+  const int ngroup = rho_groups(c, plane_rho_resident<T>(c, maxx), kc * nb);
+  int rc = ensure(c, &c->d_work, &c->work_bytes, kc * kbytes);
+  if (rc) return rc;
+  rc = ensure(c, &c->d_rpart, &c->rpart_bytes, (size_t)ngroup * c->N * sizeof(double));
+  if (rc) return rc;
+  cplx<T>* W = reinterpret_cast<cplx<T>*>(c->d_work);
+  double* rpart = reinterpret_cast<double*>(c->d_rpart);
+  const cplx<T>* twz = reinterpret_cast<const cplx<T>*>(sizeof(T) == 8 ? c->d_tw64[2] : c->d_tw32[2]);
+  for (int k0 = 0; k0 < nk; k0 += kc) {
+    const int kn = std::min(kc, nk - k0);
+    std::vector<KBatch> kb(kn);
+    long woff = 0, blk = 0;
+    for (int i = 0; i < kn; ++i) {
+      const KData& k = c->kd[iks[k0 + i]];
+      KBatch d{};
+      d.ent_igw = k.d_ent_igw;
+      d.ent_pos = k.d_ent_pos;
+      d.col_ptr = k.d_col_ptr;
+      d.ctab = k.d_ctab;
+      d.apos = k.d_apos;
+      d.psi = psi[k0 + i];
+      d.ldpsi = ldpsi[k0 + i];
+      d.woff = woff;
+      d.ncol = k.ncol;
+      d.nxact = k.nxact;
+      d.blk0 = (int)blk;
+      kb[i] = d;
+      woff += (long)nb * c->n3 * k.ncol;
+      blk += (long)((k.ncol + C - 1) / C) * nb8;
+    }
+    if (blk > 0x7fffffffL) return set_error(c, PW_ERR_ARG, "rhoe batch too large for one launch");
+    const void* dptr = nullptr;
+    rc = desc_get(c, kb.data(), kb.size() * sizeof(KBatch), &dptr);
+    if (rc) return rc;
+    const KBatch* dkb = reinterpret_cast<const KBatch*>(dptr);
+    hipLaunchKernelGGL(k_col_ifft_batch<T>, dim3((unsigned)blk), dim3(cnt), col_lds(c, C, esz), c->stream, dkb, kn, nb,
+                       W, C, c->dim[2], twz);
+    const int tot = kn * nb, bpg = (tot + std::min(ngroup, tot) - 1) / std::min(ngroup, tot);
+    const int ngu = (tot + bpg - 1) / bpg;
+    plane_rho_batch<T>(c, dkb, nb, tot, maxx, W, bpg, ngu, d_w + (size_t)k0 * nb, rpart);
+    hipLaunchKernelGGL(k_rho_reduce, dim3(1024), dim3(256), 0, c->stream, c->d_rho, rpart, ngu, c->N, 1.0 / c->omega);
+  }
+  return hip_check(c, hipGetLastError(), "batched rhoe kernels");
+}
+
+int rhoe_accum_batch(pw_ctx* c, int nk, const int* iks, int nb, const cplx<double>* const* psi, const int64_t* ldpsi,
+                     const double* d_w, unsigned flags) {
+  if (flags & PW_MIXED) return rhoe_batch_run<float>(c, nk, iks, nb, psi, ldpsi, d_w);
+  return rhoe_batch_run<double>(c, nk, iks, nb, psi, ldpsi, d_w);
 }
 
 int g2r_apply(pw_ctx* c, KData& k, int nf, const cplx<double>* fG, long ldf, double* out, double scale,

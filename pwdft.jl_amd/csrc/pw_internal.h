@@ -318,6 +318,9 @@ int kinetic_apply(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldpsi
                   long ldh, unsigned flags);
 int rhoe_accum(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldpsi, const double* d_w,
                unsigned flags);
+// The same over the k-points iks, nb bands each, weights d_w[kk nb + band].
+int rhoe_accum_batch(pw_ctx* c, int nk, const int* iks, int nb, const cplx<double>* const* psi, const int64_t* ldpsi,
+                     const double* d_w, unsigned flags);
 int kprec_apply(pw_ctx* c, int ik, int nb, const cplx<double>* in, long ldin, cplx<double>* out,
                 long ldout);
 // out = FFT[ V(r) * IFFT[psi] ] restricted to the sphere k (FP64, no kinetic term, overwrite);
@@ -345,6 +348,8 @@ int zero_fill(pw_ctx* c, double* out, long n);
 int op_H_fused_batch(pw_ctx* c, int nk, const int* iks, int ispin, int nb, const cplx<double>* const* psi,
                      const int64_t* ldpsi, cplx<double>* const* hpsi, const int64_t* ldh, unsigned flags);
 bool op_H_fused_fits(const pw_ctx* c, bool mixed);
+// Argument check of the batched entry points (pw_batch.hip).
+int check_batch_k(pw_ctx* c, int nk, const int* iks);
 // Batched op_V_loc (+ kinetic) over the k-points iks (pw_fft.hip); psi / hpsi per k-point.
 int vloc_apply_batch(pw_ctx* c, int nk, const int* iks, int ispin, int nb, const cplx<double>* const* psi,
                      const int64_t* ldpsi, cplx<double>* const* hpsi, const int64_t* ldh, unsigned flags);

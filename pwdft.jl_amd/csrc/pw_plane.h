@@ -611,9 +611,16 @@ template <typename T>
 void plane_vloc(pw_ctx* c, const KData& k, cplx<T>* W, const T* V, int nb);
 template <typename T>
 void plane_vloc_batch(pw_ctx* c, const KBatch* dkb, int nk, int nb, int maxx, bool half, cplx<T>* W, const T* V);
-// ngroup partial planes (A.out), bpg bands each, weights d_w per band
+// ngroup partial planes (rpart), bpg bands each, weights d_w per band; the batched form takes
+// nb / nbk k-points of nbk bands each
 template <typename T>
 void plane_rho(pw_ctx* c, const KData& k, cplx<T>* W, int nb, int bpg, int ngroup, const double* d_w, double* rpart);
+template <typename T>
+void plane_rho_batch(pw_ctx* c, const KBatch* dkb, int nbk, int nb, int maxx, cplx<T>* W, int bpg, int ngroup,
+                     const double* d_w, double* rpart);
+// Workgroups of the density kernel that a CU holds at once, for at most maxx active x.
+template <typename T>
+int plane_rho_resident(const pw_ctx* c, int maxx);
 void plane_real(pw_ctx* c, const KData& k, cplx<double>* W, int nf, double* out, double scale, int acc);
 
 }  // namespace pw

@@ -97,22 +97,51 @@ void plane_vloc_batch(pw_ctx* c, const KBatch* dkb, int nk, int nb, int maxx, bo
 }
 
 template <typename T>
-void plane_rho(pw_ctx* c, const KData& k, cplx<T>* W, int nb, int bpg, int ngroup, const double* d_w, double* rpart) {
+static int rho_waves(const pw_ctx* c, size_t lds) {
+  const int reg = c->n1 == c->n2 ? rho_waves_of(c->n1) : 0;
+  return reg ? reg : plane_waves(c, lds);
+}
+
+template <typename T>
+int plane_rho_resident(const pw_ctx* c, int maxx) {
   PlaneArgs<T> A{};
-  const size_t lds = plane_args<T>(c, k.nxact, A);
-  const PlaneKernel<T> kern = lds && k.half ? plane_kernel<T, MODE_RHO, true>(c->n1, c->n2) : nullptr;
+  const size_t lds = plane_args<T>(c, maxx, A);
+  if (!lds) return 1;
+  // by LDS, and by registers about 12 wavefronts
+  return std::max(1, std::min((int)(160 * 1024 / lds), 12 / rho_waves<T>(c, lds)));
+}
+
+template <typename T>
+static void rho_launch(pw_ctx* c, PlaneArgs<T>& A, int maxx, cplx<T>* W, int nb, int bpg, int ngroup, const double* d_w,
+                       double* rpart) {
+  const size_t lds = plane_args<T>(c, maxx, A);
+  const PlaneKernel<T> kern = lds ? plane_kernel<T, MODE_RHO, true>(c->n1, c->n2) : nullptr;
   if (!kern) return;
   A.W = W;
-  A.ctab = k.d_ctab;
-  A.apos = k.d_apos;
-  A.ncol = k.ncol;
-  A.nxact = k.nxact;
   A.nb = nb;
   A.bpg = bpg;
   A.wts = d_w;
   A.out = rpart;
-  const int reg = c->n1 == c->n2 ? rho_waves_of(c->n1) : 0;
-  hipLaunchKernelGGL(kern, dim3(c->n3, ngroup), dim3(64 * (reg ? reg : plane_waves(c, lds))), lds, c->stream, A);
+  hipLaunchKernelGGL(kern, dim3(c->n3, ngroup), dim3(64 * rho_waves<T>(c, lds)), lds, c->stream, A);
+}
+
+template <typename T>
+void plane_rho(pw_ctx* c, const KData& k, cplx<T>* W, int nb, int bpg, int ngroup, const double* d_w, double* rpart) {
+  PlaneArgs<T> A{};
+  A.ctab = k.d_ctab;
+  A.apos = k.d_apos;
+  A.ncol = k.ncol;
+  A.nxact = k.nxact;
+  rho_launch<T>(c, A, k.nxact, W, nb, bpg, ngroup, d_w, rpart);
+}
+
+template <typename T>
+void plane_rho_batch(pw_ctx* c, const KBatch* dkb, int nbk, int nb, int maxx, cplx<T>* W, int bpg, int ngroup,
+                     const double* d_w, double* rpart) {
+  PlaneArgs<T> A{};
+  A.kb = dkb;
+  A.nbk = nbk;
+  rho_launch<T>(c, A, maxx, W, nb, bpg, ngroup, d_w, rpart);
 }
 
 void plane_real(pw_ctx* c, const KData& k, cplx<double>* W, int nf, double* out, double scale, int acc) {
@@ -137,5 +166,9 @@ template void plane_vloc_batch<double>(pw_ctx*, const KBatch*, int, int, int, bo
 template void plane_vloc_batch<float>(pw_ctx*, const KBatch*, int, int, int, bool, cplx<float>*, const float*);
 template void plane_rho<double>(pw_ctx*, const KData&, cplx<double>*, int, int, int, const double*, double*);
 template void plane_rho<float>(pw_ctx*, const KData&, cplx<float>*, int, int, int, const double*, double*);
+template void plane_rho_batch<double>(pw_ctx*, const KBatch*, int, int, int, cplx<double>*, int, int, const double*, double*);
+template void plane_rho_batch<float>(pw_ctx*, const KBatch*, int, int, int, cplx<float>*, int, int, const double*, double*);
+template int plane_rho_resident<double>(const pw_ctx*, int);
+template int plane_rho_resident<float>(const pw_ctx*, int);
 
 }  // namespace pw

@@ -61,6 +61,7 @@ _PROTOS = {
     "pw_rhoe_zero": [_vp],
     "pw_rhoe_accum": [_vp, _i, _i, _vp, _i64, _vp, _c.c_uint],
     "pw_rhoe_accum_dev": [_vp, _i, _i, _vp, _i64, _vp, _c.c_uint],
+    "pw_rhoe_accum_batch_dev": [_vp, _i, _vp, _i, _vp, _vp, _vp, _c.c_uint],
     "pw_rhoe_get": [_vp, _vp],
     "pw_op_H_batch_dev": [_vp, _i, _vp, _i, _i, _vp, _vp, _vp, _vp, _c.c_uint],
     "pw_kprec_batch_dev": [_vp, _i, _vp, _i, _vp, _vp, _vp, _vp],

@@ -96,3 +96,40 @@ def test_rho_groups(ns, mixed):
     ref *= float(N) ** 2 / 3.7
     assert np.abs(got - ref).max() <= (2e-5 if mixed else 1e-12) * np.abs(ref).max()
     c.close()
+
+
+@pytest.mark.parametrize("ns,nk,nb,mixed", [((20, 20, 20), 9, 3, False), ((27, 27, 27), 5, 7, True),
+                                            ((36, 24, 45), 3, 5, False), ((24, 36, 20), 4, 40, True),
+                                            ((125, 12, 12), 2, 2, False)])
+def test_rho_batch(ns, nk, nb, mixed):
+    """k-points with different index sets in the same launches (and, without a plan, one by one)."""
+    from pwdft_hip._lib import PW_MIXED, DeviceMatrix, ptr
+    rng = np.random.default_rng(3)
+    sets = [index_set(ns, [(n - 1) // 4 - (ik % 2) for n in ns], shift=0.2 * ik / nk) for ik in range(nk)]
+    c = context(ns, sets[0])
+    for ik in range(1, nk):
+        gk = rng.standard_normal((sets[ik].size, 3))
+        c.call("pw_set_kpoint", ik, sets[ik].size, ptr(sets[ik]), 0, ptr(gk))
+    psi = [rand(rng, s.size, nb) for s in sets]
+    dev = [DeviceMatrix.from_host(c, p) for p in psi]
+    w = np.ascontiguousarray(rng.random((nk, nb)))
+    ld = np.array([p.shape[0] for p in psi], dtype=np.int64)
+    pp = np.array([d.p.value for d in dev], dtype=np.uint64)
+    N = int(np.prod(ns))
+    got = np.empty(N)
+    print(f"case rho batch {ns} nk={nk} nb={nb} mixed={mixed}", flush=True)
+    c.call("pw_rhoe_zero")
+    c.call("pw_rhoe_accum_batch_dev", nk, ptr(np.arange(nk, dtype=np.int32)), nb, ptr(pp), ptr(ld), ptr(w),
+           PW_MIXED if mixed else 0)
+    c.call("pw_rhoe_get", ptr(got))
+    ref = np.zeros(N)
+    for ik in range(nk):
+        f = np.zeros((nb, N), dtype=complex)
+        f[:, sets[ik]] = psi[ik].T
+        g = np.fft.ifftn(f.reshape(nb, ns[2], ns[1], ns[0]), axes=(1, 2, 3)).reshape(nb, N)
+        ref += (w[ik][:, None] * np.abs(g) ** 2).sum(0)
+    ref *= float(N) ** 2 / 3.7
+    assert np.abs(got - ref).max() <= (2e-5 if mixed else 1e-12) * np.abs(ref).max()
+    for d in dev:
+        d.free()
+    c.close()
