@@ -62,11 +62,15 @@ int pw_set_band_batch(pw_ctx* ctx, int nb);
 
 /* Tuning knobs set by the autotuner (pwdft_hip/autotune.py); no reference counterpart. */
 enum {
-  PW_TUNE_GEMM_CN_SHAPE = 0,  /* A^H B products: -1 = chosen by N (default), 0 = 64x64 tile, 1 = 128x64,
-                                 2 = 64x128, 3 = 128x128, 4 = 128x32, 5 = 64x32 */
+  PW_TUNE_GEMM_CN_SHAPE = 0,  /* A^H B products: -1 = chosen by size (default); a 32x32 tile per
+                                 wavefront in workgroups covering 0 = 64x64, 1 = 128x64, 2 = 64x128,
+                                 3 = 128x128, 4 = 128x32, 5 = 64x32; wavefronts sharing the K of one
+                                 tile: 6 = eight on 16x16, 7 = four on 32x32 (FP32 MFMA in the mixed
+                                 path also where PW_TUNE_GEMM_SPLIT_BF16 asks for the split) */
   PW_TUNE_GEMM_NN_SHAPE = 1,  /* A B products: same codes */
-  PW_TUNE_GEMM_CN_WG = 2,     /* A^H B split-K target workgroup count (0 = default 1024) */
-  PW_TUNE_GEMM_NN_WG = 3,     /* A B split-K target workgroup count (0 = default 512) */
+  PW_TUNE_GEMM_CN_WG = 2,     /* A^H B split-K target workgroup count (0 = default: 512, 1024 for
+                                 shape 5, 256 for shapes 2 and 3) */
+  PW_TUNE_GEMM_NN_WG = 3,     /* A B split-K target workgroup count (0 = default, the same) */
   PW_TUNE_BAND_BATCH = 4,     /* bands per fused FFT launch (same as pw_set_band_batch) */
   PW_TUNE_PLANE_COMPRESSED = 5, /* 1: always use the general compressed z-plane kernels (they are
                                    used anyway for line lengths without a two-pass plan); 2:

@@ -4,17 +4,14 @@
 //
 //   C (M x N) = alpha * op(A) * B + beta * C,  op(A) = A (M x K) or A^H (A is K x M)
 //
-// The complex product is the real product  C_raw (2M x N) = At (2M x 2K) * B_raw (2K x N)
-// where B_raw / C_raw are the interleaved (re, im) storage of B / C and At replaces each
-// complex entry a of op(A) by the 2x2 block [[re a, -im a], [im a, re a]].  Every element of
-// At is a signed copy of one element of A, so one MFMA stream computes 8 real flops per
-// complex multiply-add with no wasted lanes.
+// The 16x16x4 MFMA takes from lane l the A element of row l % 16 and the B element of column
+// l % 16 at k = l / 16, so a lane's operands are whole complex numbers of A and B as they lie in
+// memory: one 16-byte load per 16 x 4 complex entries of each, no LDS, no barrier.  A complex
+// 16 x 16 tile is four real MFMAs per four k (re re, im im, re im, im re), 8 real flops per
+// complex multiply-add with no wasted lanes.  Every wavefront runs on its own, its loads a ring
+// of RING k-steps ahead of the MFMAs that use them.  What bounds it is MFMA issue (64 cycles per
+// FP64 MFMA, 32 in FP32): a 32 x 32 tile needs four loads per 16 MFMAs.
 //
-// Tiles: a workgroup of WM x WN waves owns 32 WM complex rows (64 WM real rows) x 32 WN
-// columns of C; each wave owns 64 real rows x 32 columns as 4 x 2 MFMA 16x16 accumulators.
-// K is consumed in stages of 16 (FP32) or 8 (FP64) complex k staged through k-contiguous,
-// padded LDS rows in two buffers: the next stage's global loads are issued before the
-// current stage's MFMAs and written to the other buffer after them, one barrier per stage.
 // Long K (the Ngw-long inner products) is split into chunks; partial tiles are reduced by a
 // second kernel in a fixed order, so results are bitwise repeatable.
 #include "pw_internal.h"
@@ -32,10 +29,8 @@ struct Mfma<double> {
   __device__ static inline acc_t run(double a, double b, acc_t c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-  // f64 16x16x4 leaves D[(l/16) + 4r][l%16] in register r of lane l; A-row i is fed with
-  // logical real row 2*(2*(i%4) + (i/4)/2) + (i/4)%2 so that registers (0,1) and (2,3) of
-  // lane group g hold the (re, im) pairs of complex rows 2g and 2g+1.
-  __device__ static inline int row(int i) { return 2 * (2 * (i & 3) + ((i >> 2) >> 1)) + ((i >> 2) & 1); }
+  // row of D in register r of lane group g = l / 16 (the column is l % 16)
+  __device__ static inline int row(int g, int r) { return g + 4 * r; }
 };
 template <>
 struct Mfma<float> {
@@ -43,238 +38,204 @@ struct Mfma<float> {
   __device__ static inline acc_t run(float a, float b, acc_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
-  // f32 16x16x4 leaves D[4*(l/16) + r][l%16] in register r of lane l: identity row map.
-  __device__ static inline int row(int i) { return i; }
+  __device__ static inline int row(int g, int r) { return 4 * g + r; }
 };
 
-// Workgroup of WM x WN wavefronts; each wavefront owns 64 real rows (32 complex) x 32
-// columns of C as 4 x 2 MFMA 16x16 accumulators, so the workgroup tile is
-// (32 WM complex rows) x (32 WN columns) while per-lane registers stay fixed.
 constexpr int GBK = 16;           // split-K chunks are multiples of this (and of every stage)
 
-// Workgroup id -> (m tile, n tile, k chunk).  Consecutive workgroup ids land on different
-// XCDs (round-robin over 8), so the mapping sends every tile of one k chunk (which share
-// the chunk of A^H / B rows) to one XCD and its L2.  Without split-K the n tiles of one
-// m tile (which share the rows of A) go to one XCD.
-__device__ inline void tile_of(int w, int tm, int tn, int nz, int& mt, int& nt, int& z) {
-  const int xcd = w & 7, idx = w >> 3;
+// Workgroup id -> (m tile, n tile, k chunk).  Consecutive workgroup ids land on different XCDs
+// (round-robin over 8); XCD x takes the x-th contiguous eighth of the (chunk, n, m) order with
+// split-K (the tiles of a chunk, which share its rows of A^H and B, meet in one L2) and of the
+// (m, n) order without (the n tiles of one m tile, which share the rows of A).
+__device__ inline bool tile_of(int w, int tm, int tn, int nz, int& mt, int& nt, int& z) {
+  const int tiles = tm * tn, tot = tiles * nz, per = (tot + 7) >> 3;
+  const int t = (w & 7) * per + (w >> 3);
+  if ((w >> 3) >= per || t >= tot) return false;
   if (nz > 1) {
-    const int tiles = tm * tn;
-    const int zq = idx / tiles, t = idx - zq * tiles;
-    z = zq * 8 + xcd;
-    mt = t % tm;
-    nt = t / tm;
+    z = t / tiles;
+    const int r = t - z * tiles;
+    nt = r / tm;
+    mt = r - nt * tm;
   } else {
-    // the tn tiles of one m tile run back to back on one XCD; m tiles rotate over XCDs
-    const int mq = idx / tn;
-    nt = idx - mq * tn;
-    mt = mq * 8 + xcd;
     z = 0;
+    mt = t / tn;
+    nt = t - mt * tn;
+  }
+  return true;
+}
+
+// A wavefront's T x T tiles of 16 x 16 complex outputs at (m0, n0), over the k-steps (4 k each)
+// k0 + 4 (first + stride i) that lie wholly before kend, and the masked rest of K, which belongs
+// to the wavefront with `tail`.
+template <typename TC, typename TA, typename TB, int TRANSA, int TM, int TN>
+struct WaveTile {
+  typedef typename Mfma<TC>::acc_t acc_t;
+  static constexpr int RING = TM * TN > 1 ? 4 : 8;   // k-steps in flight
+  acc_t re[TM][TN], im[TM][TN];
+
+  __device__ inline void mma(const cplx<TA> (&a)[TM], const cplx<TB> (&b)[TN]) {
+    TC ar[TM], ai[TM], na[TM], br[TN], bi[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      ar[i] = (TC)a[i].x;
+      ai[i] = (TC)a[i].y;
+      na[i] = -ai[i];
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      br[j] = (TC)b[j].x;
+      bi[j] = (TC)b[j].y;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        re[i][j] = Mfma<TC>::run(ar[i], br[j], re[i][j]);
+        im[i][j] = Mfma<TC>::run(ar[i], bi[j], im[i][j]);
+      }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        // A^H: re += im im, im -= im re; A: re -= im im, im += im re
+        re[i][j] = Mfma<TC>::run(TRANSA ? ai[i] : na[i], bi[j], re[i][j]);
+        im[i][j] = Mfma<TC>::run(TRANSA ? na[i] : ai[i], br[j], im[i][j]);
+      }
+  }
+
+  __device__ inline void run(int M, int N, const cplx<TA>* __restrict__ A, long lda, const cplx<TB>* __restrict__ B,
+                             long ldb, int m0, int n0, int kbeg, int kend, int first, int stride, bool tail) {
+    const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) re[i][j][r] = im[i][j][r] = (TC)0;
+    // rows and columns past the matrices take a valid one's data; their outputs are not stored
+    const cplx<TA>* pa[TM];
+    const cplx<TB>* pb[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const int m = min(m0 + 16 * i + li, M - 1);
+      pa[i] = TRANSA ? A + (long)m * lda + kbeg + lg : A + (long)(kbeg + lg) * lda + m;
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) pb[j] = B + (long)min(n0 + 16 * j + li, N - 1) * ldb + kbeg + lg;
+    const long sa = TRANSA ? 4 : 4 * lda;
+    const int full = (kend - kbeg) >> 2;
+    const int n = full > first ? (full - first + stride - 1) / stride : 0;
+    cplx<TA> a[RING][TM];
+    cplx<TB> b[RING][TN];
+    auto load = [&](int d, int s) {
+      const int k = first + s * stride;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[d][i] = pa[i][k * sa];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[d][j] = pb[j][4 * k];
+    };
+#pragma unroll
+    for (int d = 0; d < RING; ++d)
+      if (d < n) load(d, d);
+    int s = 0;
+    for (; s + 2 * RING <= n; s += RING) {
+#pragma unroll
+      for (int d = 0; d < RING; ++d) {
+        mma(a[d], b[d]);
+        load(d, s + RING + d);
+      }
+    }
+    for (; s < n; s += RING) {
+#pragma unroll
+      for (int d = 0; d < RING; ++d) {
+        if (s + d < n) mma(a[d], b[d]);
+        if (s + RING + d < n) load(d, s + RING + d);
+      }
+    }
+    if (tail && (kend - kbeg) & 3) {
+      const bool ok = 4 * full + lg < kend - kbeg;
+      cplx<TA> ta[TM];
+      cplx<TB> tb[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) ta[i] = ok ? pa[i][full * sa] : mk((TA)0, (TA)0);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) tb[j] = ok ? pb[j][4 * full] : mk((TB)0, (TB)0);
+      mma(ta, tb);
+    }
+  }
+};
+
+struct GemmOut {
+  cplx<double>* C;
+  long ldc;
+  cplx<double> alpha, beta;
+  int direct, use_beta;
+  cplx<double>* part;   // !direct: partial sums [z][n][m]
+};
+__device__ inline void gemm_store(const GemmOut& o, int M, int N, int z, int m, int n, cplx<double> v) {
+  if (m >= M || n >= N) return;
+  if (o.direct) {
+    cplx<double> r = cmul(o.alpha, v);
+    if (o.use_beta) r = r + cmul(o.beta, o.C[(long)n * o.ldc + m]);
+    o.C[(long)n * o.ldc + m] = r;
+  } else {
+    o.part[((long)z * N + n) * M + m] = v;
   }
 }
 
+// WM x WN wavefronts, each with a 32 x 32 tile of its own.
 template <typename TC, typename TA, typename TB, int TRANSA, int WM, int WN>
 __global__ void __launch_bounds__(64 * WM * WN)
 k_zgemm(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const cplx<TB>* __restrict__ B,
-        long ldb, int kchunk, cplx<double>* __restrict__ C, long ldc, cplx<double> alpha,
-        cplx<double> beta, int direct, int use_beta, cplx<double>* __restrict__ part, int tm, int tn,
-        int nz) {
-  constexpr int NT = 64 * WM * WN;
-  constexpr int BMC = 32 * WM;   // complex rows per workgroup
-  constexpr int BNC = 32 * WN;   // columns per workgroup
-  // complex k per LDS stage: two stages (double buffer) of 16 (FP32) or 8 (FP64) complex k
-  // keep the LDS of a 64 x 64 tile at 36 KiB, so four workgroups fit a CU
-  constexpr int SBK = sizeof(TC) == 8 ? 8 : 16;
-  constexpr int SKS = 2 * SBK + 4;  // LDS row stride (reals): k-contiguous rows, padded
-  constexpr int NA = (BMC * SBK) / NT, NB = (BNC * SBK) / NT;
-  static_assert(NA >= 1 && NB >= 1 && (BMC * SBK) % NT == 0 && (BNC * SBK) % NT == 0, "tile");
-  __shared__ TC As[2][BMC][SKS];   // [buffer][complex row m][real k'] raw (re, im) pairs along k
-  __shared__ TC Bs[2][BNC][SKS];   // [buffer][column n][real k']
-  typedef typename Mfma<TC>::acc_t acc_t;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = wave % WM, wn = wave / WM;
+        long ldb, int kchunk, GemmOut o, int tm, int tn, int nz) {
   int mt, nt, z;
-  tile_of(blockIdx.x, tm, tn, nz, mt, nt, z);
-  if (z >= nz || mt >= tm || nt >= tn) return;
-  const int m0 = mt * BMC, n0 = nt * BNC;
-  const int kbeg = z * kchunk;
-  const int kend = min(K, kbeg + kchunk);
-  acc_t acc[4][2];
+  if (!tile_of(blockIdx.x, tm, tn, nz, mt, nt, z)) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m0 = mt * 32 * WM + 32 * (wave % WM), n0 = nt * 32 * WN + 32 * (wave / WM);
+  if (m0 >= M || n0 >= N) return;
+  WaveTile<TC, TA, TB, TRANSA, 2, 2> t;
+  t.run(M, N, A, lda, B, ldb, m0, n0, z * kchunk, min(K, (z + 1) * kchunk), 0, 1, true);
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[i][j][r] = (TC)0;
-  const int li = lane & 15, lg = lane >> 4;
+      for (int r = 0; r < 4; ++r)
+        gemm_store(o, M, N, z, m0 + 16 * i + Mfma<TC>::row(lane >> 4, r), n0 + 16 * j + (lane & 15),
+                   mk((double)t.re[i][j][r], (double)t.im[i][j][r]));
+}
 
-  // global -> register staging: NA complex of A and NB of B per thread per stage, held in
-  // their storage type and converted only when written to LDS, so the loads of the next
-  // stage stay in flight during the MFMA phase.  Out-of-range elements load a valid
-  // address (element 0) and are zeroed at the LDS write through the valid mask.
-  cplx<TA> ra[NA];
-  cplx<TB> rb[NB];
-  unsigned va = 0, vb = 0;
-  auto a_idx = [&](int s, int& mm, int& kk) {
-    if (TRANSA == 0) { mm = tid % BMC; kk = tid / BMC + (NT / BMC) * s; }
-    else { kk = tid % SBK; mm = tid / SBK + (NT / SBK) * s; }
-  };
-  auto b_idx = [&](int s, int& kb, int& nn) { kb = tid % SBK; nn = tid / SBK + (NT / SBK) * s; };
-  // a stage wholly inside the matrices (every stage of an interior tile but the last of its
-  // K chunk) is loaded and stored without per-element checks, in workgroups of at most four
-  // wavefronts except FP32-MFMA A^H B: measured 2-5 % faster there at the Si64 projector
-  // shapes, but 6-10 % slower for FP32-MFMA A^H B and ~10 % slower in the 8-wavefront tiles
-  // of the Si216 shapes (the extra path's registers)
-  constexpr bool FAST = WM * WN <= 4 && !(sizeof(TC) == sizeof(float) && TRANSA == 1);
-  bool sfull = false;
-  auto load_stage = [&](int k0) {
-    sfull = FAST && m0 + BMC <= M && n0 + BNC <= N && k0 + SBK <= kend;
-    if (sfull) {
+// WK wavefronts on one tile of (16 T) x (16 T) outputs, their k-steps interleaved, the partial
+// tiles summed through LDS in wavefront order: products too small to fill the chip with 32 x 32
+// tiles of their own.
+template <typename TC, typename TA, typename TB, int TRANSA, int T, int WK>
+__global__ void __launch_bounds__(64 * WK)
+k_zgemm_wk(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const cplx<TB>* __restrict__ B,
+           long ldb, int kchunk, GemmOut o, int tm, int tn, int nz) {
+  __shared__ cplx<TC> red[WK][16][17];
+  int mt, nt, z;
+  if (!tile_of(blockIdx.x, tm, tn, nz, mt, nt, z)) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m0 = mt * 16 * T, n0 = nt * 16 * T;
+  WaveTile<TC, TA, TB, TRANSA, T, T> t;
+  t.run(M, N, A, lda, B, ldb, m0, n0, z * kchunk, min(K, (z + 1) * kchunk), wave, WK, wave == 0);
 #pragma unroll
-      for (int s = 0; s < NA; ++s) {
-        int mm, kk;
-        a_idx(s, mm, kk);
-        const int gm = m0 + mm, gk = k0 + kk;
-        ra[s] = A[TRANSA == 0 ? (long)gk * lda + gm : (long)gm * lda + gk];
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int j = 0; j < T; ++j) {
+      if (i + j > 0) __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[wave][lane & 15][Mfma<TC>::row(lane >> 4, r)] = mk(t.re[i][j][r], t.im[i][j][r]);
+      __syncthreads();
+      for (int e = threadIdx.x; e < 256; e += 64 * WK) {
+        const int n = e >> 4, m = e & 15;
+        cplx<double> v = cvt<double>(red[0][n][m]);
+#pragma unroll
+        for (int w = 1; w < WK; ++w) v = v + cvt<double>(red[w][n][m]);
+        gemm_store(o, M, N, z, m0 + 16 * i + m, n0 + 16 * j + n, v);
       }
-#pragma unroll
-      for (int s = 0; s < NB; ++s) {
-        int kb, nn;
-        b_idx(s, kb, nn);
-        rb[s] = B[(long)(n0 + nn) * ldb + k0 + kb];
-      }
-      return;
     }
-    va = 0;
-    vb = 0;
-#pragma unroll
-    for (int s = 0; s < NA; ++s) {
-      int mm, kk;
-      a_idx(s, mm, kk);
-      const int gm = m0 + mm, gk = k0 + kk;
-      const bool ok = gm < M && gk < kend;
-      const long off = ok ? (TRANSA == 0 ? (long)gk * lda + gm : (long)gm * lda + gk) : 0;
-      ra[s] = A[off];
-      va |= (unsigned)ok << s;
-    }
-#pragma unroll
-    for (int s = 0; s < NB; ++s) {
-      int kb, nn;
-      b_idx(s, kb, nn);
-      const int gkb = k0 + kb, gn = n0 + nn;
-      const bool ok = gkb < kend && gn < N;
-      rb[s] = B[ok ? (long)gn * ldb + gkb : 0];
-      vb |= (unsigned)ok << s;
-    }
-  };
-  auto store_stage = [&](int buf) {
-    if (sfull) {
-#pragma unroll
-      for (int s = 0; s < NA; ++s) {
-        int mm, kk;
-        a_idx(s, mm, kk);
-        *reinterpret_cast<cplx<TC>*>(&As[buf][mm][2 * kk]) = cvt<TC>(ra[s]);
-      }
-#pragma unroll
-      for (int s = 0; s < NB; ++s) {
-        int kb, nn;
-        b_idx(s, kb, nn);
-        *reinterpret_cast<cplx<TC>*>(&Bs[buf][nn][2 * kb]) = cvt<TC>(rb[s]);
-      }
-      return;
-    }
-#pragma unroll
-    for (int s = 0; s < NA; ++s) {
-      int mm, kk;
-      a_idx(s, mm, kk);
-      const cplx<TC> v = ((va >> s) & 1u) ? cvt<TC>(ra[s]) : mk((TC)0, (TC)0);
-      *reinterpret_cast<cplx<TC>*>(&As[buf][mm][2 * kk]) = v;
-    }
-#pragma unroll
-    for (int s = 0; s < NB; ++s) {
-      int kb, nn;
-      b_idx(s, kb, nn);
-      const cplx<TC> v = ((vb >> s) & 1u) ? cvt<TC>(rb[s]) : mk((TC)0, (TC)0);
-      *reinterpret_cast<cplx<TC>*>(&Bs[buf][nn][2 * kb]) = v;
-    }
-  };
-
-  int buf = 0;
-  if (kbeg < kend) {
-    load_stage(kbeg);
-    store_stage(0);
-  }
-  __syncthreads();
-  for (int k0 = kbeg; k0 < kend; k0 += SBK) {
-    const bool more = k0 + SBK < kend;
-    if (more) load_stage(k0 + SBK);  // in flight during the MFMA phase
-    // operand fragments of k-step q: read from LDS one step ahead of the MFMAs that use
-    // them (two register sets), so the LDS latency overlaps the previous step's MFMAs
-    // Ã's sign pattern depends on the lane and the row tile only (k-step parity is lg's)
-    constexpr int NQ = (2 * SBK) / 4;
-    TC a[2][4], b[2][2];
-    auto frag = [&](int q, int p) {
-      const int kp = 4 * q + lg;
-      const int kc = kp >> 1, t = kp & 1;
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        const int ip = wm * 64 + rt * 16 + Mfma<TC>::row(li);
-        a[p][rt] = As[buf][ip >> 1][2 * kc + ((ip & 1) ^ t)];
-      }
-#pragma unroll
-      for (int ct = 0; ct < 2; ++ct) b[p][ct] = Bs[buf][wn * 32 + ct * 16 + li][kp];
-    };
-    bool neg[4];
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-      const int sgn = (wm * 64 + rt * 16 + Mfma<TC>::row(li)) & 1, t = lg & 1;
-      neg[rt] = (TRANSA == 0) ? (sgn == 0 && t == 1) : (sgn == 1 && t == 0);
-    }
-    frag(0, 0);
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      const int p = q & 1;
-      if (q + 1 < NQ) frag(q + 1, p ^ 1);
-      // keep the next step's LDS reads ahead of this step's MFMAs (the scheduler would
-      // otherwise sink them to their use), so their latency overlaps these MFMAs
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        const TC av = neg[rt] ? -a[p][rt] : a[p][rt];
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct) acc[rt][ct] = Mfma<TC>::run(av, b[p][ct], acc[rt][ct]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // one barrier per stage: the other buffer is written while this one is read, and no
-    // wave writes this buffer again before every wave has passed this barrier
-    if (more) store_stage(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-  // with the row maps above, registers (0, 1) and (2, 3) of lane group lg hold the
-  // (re, im) pairs of complex rows 2*lg and 2*lg + 1 of each 16-row tile.
-#pragma unroll
-  for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-    for (int ct = 0; ct < 2; ++ct)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const int ip = wm * 64 + rt * 16 + 4 * lg + 2 * p;
-        const int m = m0 + (ip >> 1);
-        const int n = n0 + wn * 32 + ct * 16 + li;
-        if (m < M && n < N) {
-          cplx<double> v = mk((double)acc[rt][ct][2 * p], (double)acc[rt][ct][2 * p + 1]);
-          if (direct) {
-            cplx<double> r = cmul(alpha, v);
-            if (use_beta) r = r + cmul(beta, C[(long)n * ldc + m]);
-            C[(long)n * ldc + m] = r;
-          } else {
-            part[((long)z * N + n) * M + m] = v;
-          }
-        }
-      }
 }
 
 // FP32-accurate complex GEMM on BF16 MFMA (the mixed path's alternative to the FP32 MFMA
@@ -300,8 +261,7 @@ __device__ inline void split3(float x, __bf16& h0, __bf16& h1, __bf16& h2) {
 template <typename TA, typename TB, int TRANSA, int WM, int WN>
 __global__ void __launch_bounds__(64 * WM * WN)
 k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const cplx<TB>* __restrict__ B,
-           long ldb, int kchunk, cplx<double>* __restrict__ C, long ldc, cplx<double> alpha, cplx<double> beta,
-           int direct, int use_beta, cplx<double>* __restrict__ part, int tm, int tn, int nz) {
+           long ldb, int kchunk, GemmOut o, int tm, int tn, int nz) {
   constexpr int NT = 64 * WM * WN;
   constexpr int BMC = 32 * WM, BNC = 32 * WN;
   constexpr int NA = (BMC * HBK) / NT, NB = (BNC * HBK) / NT;
@@ -312,8 +272,7 @@ k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave % WM, wn = wave / WM;
   int mt, nt, z;
-  tile_of(blockIdx.x, tm, tn, nz, mt, nt, z);
-  if (z >= nz || mt >= tm || nt >= tn) return;
+  if (!tile_of(blockIdx.x, tm, tn, nz, mt, nt, z)) return;
   const int m0 = mt * BMC, n0 = nt * BNC;
   const int kbeg = z * kchunk;
   const int kend = min(K, kbeg + kchunk);
@@ -444,18 +403,8 @@ k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         const int ip = wm * 64 + rt * 16 + 4 * lg + 2 * p;
-        const int m = m0 + (ip >> 1);
-        const int n = n0 + wn * 32 + ct * 16 + li;
-        if (m < M && n < N) {
-          cplx<double> v = mk((double)acc[rt][ct][2 * p], (double)acc[rt][ct][2 * p + 1]);
-          if (direct) {
-            cplx<double> r = cmul(alpha, v);
-            if (use_beta) r = r + cmul(beta, C[(long)n * ldc + m]);
-            C[(long)n * ldc + m] = r;
-          } else {
-            part[((long)z * N + n) * M + m] = v;
-          }
-        }
+        gemm_store(o, M, N, z, m0 + (ip >> 1), n0 + wn * 32 + ct * 16 + li,
+                   mk((double)acc[rt][ct][2 * p], (double)acc[rt][ct][2 * p + 1]));
       }
 }
 
@@ -473,109 +422,161 @@ __global__ void k_zgemm_reduce(int M, int N, int nz, const cplx<double>* __restr
   }
 }
 
-// Launch one (WM x WN) instance: tiles, split-K chunks, optional ordered reduction.
+// Complex multiply-adds from which the split-BF16 kernel takes FP32 products by default: it pays
+// off on large ones (Si216's projector and Gram products, 4e10), not beside the FFT passes at
+// Si64 (1.2e9).
+constexpr double GEMM_SPLIT_MIN = 8589934592.0;
+
+// Split of K over `nz` chunks for about `slots` workgroups on `tiles` tiles (no chunk shorter
+// than `kmin`), the partial-sum workspace and the epilogue.
+struct GemmSplit {
+  int nz = 1, kchunk = GBK;
+  long nwg = 0;
+  GemmOut o{};
+};
+static int gemm_split(pw_ctx* c, int M, int N, int K, long tiles, long slots, int kmin, cplx<double> alpha,
+                      cplx<double> beta, cplx<double>* C, long ldc, GemmSplit& g) {
+  const int ksteps = (K + GBK - 1) / GBK;
+  long nz = std::min<long>(slots / std::max<long>(tiles, 1), K / std::max(kmin, GBK));
+  nz = std::max<long>(nz, 1);
+  // a no-allocation call splits K only as far as its fixed partial-sum array holds
+  if (c->no_alloc && nz > 1) nz = std::max<long>(1, std::min<long>(nz, (long)(c->gpart_bytes / ((size_t)M * N * 16))));
+  if (K > 0) {
+    g.kchunk = (int)((ksteps + nz - 1) / nz) * GBK;
+    nz = (K + g.kchunk - 1) / g.kchunk;
+  }
+  g.nz = (int)nz;
+  g.nwg = 8 * ((tiles * nz + 7) / 8);   // ids past the work return at once
+  g.o.C = C;
+  g.o.ldc = ldc;
+  g.o.alpha = alpha;
+  g.o.beta = beta;
+  g.o.use_beta = (beta.x != 0.0 || beta.y != 0.0) ? 1 : 0;
+  g.o.direct = nz == 1 ? 1 : 0;
+  if (nz > 1) {
+    int rc = ensure(c, &c->d_gpart, &c->gpart_bytes, (size_t)nz * M * N * sizeof(cplx<double>));
+    if (rc) return rc;
+    g.o.part = reinterpret_cast<cplx<double>*>(c->d_gpart);
+  }
+  return PW_OK;
+}
+static int gemm_finish(pw_ctx* c, int M, int N, const GemmSplit& g) {
+  if (g.nz > 1) {
+    const long tot = (long)M * N;
+    const int blocks = (int)std::min<long>((tot + 255) / 256, 2048);
+    hipLaunchKernelGGL(k_zgemm_reduce, dim3(blocks), dim3(256), 0, c->stream, M, N, g.nz, g.o.part, g.o.C, g.o.ldc,
+                       g.o.alpha, g.o.beta, g.o.use_beta);
+  }
+  return hip_check(c, hipGetLastError(), "zgemm");
+}
+
+// One (WM x WN) instance of the kernels with 32 x 32 tiles per wavefront.
 template <typename TC, typename TA, typename TB, int WM, int WN>
 static int zgemm_launch(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alpha, const cplx<TA>* A,
                         long lda, const cplx<TB>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc,
                         int target_wg) {
   constexpr int BMC = 32 * WM, BNC = 32 * WN;
-  const int use_beta = (beta.x != 0.0 || beta.y != 0.0) ? 1 : 0;
   const int tm = (M + BMC - 1) / BMC, tn = (N + BNC - 1) / BNC;
-  const long tiles = (long)tm * tn;
-  const int ksteps = (K + GBK - 1) / GBK;
-  int nz = 1;
-  if (tiles < target_wg && ksteps > 8) {
-    nz = (int)std::min<long>((target_wg + tiles - 1) / tiles, ksteps / 8);
-    nz = std::max(8, (nz + 7) / 8 * 8);  // whole rounds over the 8 XCDs
-    // a no-allocation call splits K only as far as its fixed partial-sum array holds
-    if (c->no_alloc) nz = std::max<int>(1, std::min<long>(nz, (long)(c->gpart_bytes / ((size_t)M * N * 16))));
-  }
-  int kchunk = GBK;
-  if (K > 0) {
-    kchunk = ((ksteps + nz - 1) / nz) * GBK;
-    nz = (K + kchunk - 1) / kchunk;
-  } else {
-    nz = 1;
-  }
-  cplx<double>* part = nullptr;
-  if (nz > 1) {
-    int rc = ensure(c, &c->d_gpart, &c->gpart_bytes, (size_t)nz * M * N * sizeof(cplx<double>));
-    if (rc) return rc;
-    part = reinterpret_cast<cplx<double>*>(c->d_gpart);
-  }
-  const int direct = nz == 1 ? 1 : 0;
-  // ids past the work (the last partial round of 8) return at once
-  const long nwg = nz > 1 ? ((nz + 7) / 8) * 8 * tiles : (long)8 * ((tm + 7) / 8) * tn;
-  const double gbytes = (double)M * K * sizeof(cplx<TA>) + (double)K * N * sizeof(cplx<TB>) +
-                        (double)M * N * 16.0 * (use_beta ? 2 : 1);
-  ProfScope ps(c, transa ? PW_PROF_GEMM_CN : PW_PROF_GEMM_NN, gbytes);
+  GemmSplit g;
+  int rc = gemm_split(c, M, N, K, (long)tm * tn, target_wg, 128, alpha, beta, C, ldc, g);
+  if (rc) return rc;
   bool split_bf16 = false;
   // the three-part operands of a 128 x 128 tile do not fit in LDS: that shape keeps FP32 MFMA
-  // default (-1): by size -- the split form pays off on large products (Si216's projector and
-  // Gram products: 4e10 complex multiply-adds, 3.49 -> 3.00 ms), not beside the FFT passes
-  // at Si64 (1.2e9)
   if constexpr (sizeof(TC) == 4 && WM * WN < 16)
-    split_bf16 = c->gemm_split_bf16 > 0 || (c->gemm_split_bf16 < 0 && (double)M * N * K >= 8589934592.0);
-  if constexpr (sizeof(TC) == 4 && WM * WN < 16) {
-    if (split_bf16) {
-      if (transa)
-        hipLaunchKernelGGL((k_zgemm_b3<TA, TB, 1, WM, WN>), dim3(nwg), dim3(64 * WM * WN), 0, c->stream, M, N, K, A,
-                           lda, B, ldb, kchunk, C, ldc, alpha, beta, direct, use_beta, part, tm, tn, nz);
-      else
-        hipLaunchKernelGGL((k_zgemm_b3<TA, TB, 0, WM, WN>), dim3(nwg), dim3(64 * WM * WN), 0, c->stream, M, N, K, A,
-                           lda, B, ldb, kchunk, C, ldc, alpha, beta, direct, use_beta, part, tm, tn, nz);
+    split_bf16 = c->gemm_split_bf16 > 0 || (c->gemm_split_bf16 < 0 && (double)M * N * K >= GEMM_SPLIT_MIN);
+  {
+    ProfScope ps(c, transa ? PW_PROF_GEMM_CN : PW_PROF_GEMM_NN,
+                 (double)M * K * sizeof(cplx<TA>) + (double)K * N * sizeof(cplx<TB>) +
+                     (double)M * N * 16.0 * (g.o.use_beta ? 2 : 1));
+    const dim3 grid((unsigned)g.nwg), blk(64 * WM * WN);
+    if constexpr (sizeof(TC) == 4 && WM * WN < 16) {
+      if (split_bf16) {
+        if (transa)
+          hipLaunchKernelGGL((k_zgemm_b3<TA, TB, 1, WM, WN>), grid, blk, 0, c->stream, M, N, K, A, lda, B, ldb,
+                             g.kchunk, g.o, tm, tn, g.nz);
+        else
+          hipLaunchKernelGGL((k_zgemm_b3<TA, TB, 0, WM, WN>), grid, blk, 0, c->stream, M, N, K, A, lda, B, ldb,
+                             g.kchunk, g.o, tm, tn, g.nz);
+      }
     }
+    if (!split_bf16) {
+      if (transa)
+        hipLaunchKernelGGL((k_zgemm<TC, TA, TB, 1, WM, WN>), grid, blk, 0, c->stream, M, N, K, A, lda, B, ldb, g.kchunk,
+                           g.o, tm, tn, g.nz);
+      else
+        hipLaunchKernelGGL((k_zgemm<TC, TA, TB, 0, WM, WN>), grid, blk, 0, c->stream, M, N, K, A, lda, B, ldb, g.kchunk,
+                           g.o, tm, tn, g.nz);
+    }
+    rc = gemm_finish(c, M, N, g);
   }
-  if (split_bf16) {
-    // launched above
-  } else if (transa)
-    hipLaunchKernelGGL((k_zgemm<TC, TA, TB, 1, WM, WN>), dim3(nwg), dim3(64 * WM * WN), 0, c->stream, M, N, K, A,
-                       lda, B, ldb, kchunk, C, ldc, alpha, beta, direct, use_beta, part, tm, tn, nz);
-  else
-    hipLaunchKernelGGL((k_zgemm<TC, TA, TB, 0, WM, WN>), dim3(nwg), dim3(64 * WM * WN), 0, c->stream, M, N, K, A,
-                       lda, B, ldb, kchunk, C, ldc, alpha, beta, direct, use_beta, part, tm, tn, nz);
-  if (nz > 1) {
-    const long tot = (long)M * N;
-    const int blocks = (int)std::min<long>((tot + 255) / 256, 2048);
-    hipLaunchKernelGGL(k_zgemm_reduce, dim3(blocks), dim3(256), 0, c->stream, M, N, nz, part, C, ldc,
-                       alpha, beta, use_beta);
-  }
-  return hip_check(c, hipGetLastError(), "zgemm");
+  return rc;
 }
 
-// Tile choice: big workgroup tiles cut the re-reads of A and B from HBM (each element is
-// read once per tile along the other dimension); small problems keep 64 x 64 tiles so the
-// grid still fills the chip.
+// The kernels whose WK wavefronts share one (16 T) x (16 T) tile.
+template <typename TC, typename TA, typename TB, int T, int WK>
+static int zgemm_wk_launch(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alpha, const cplx<TA>* A,
+                           long lda, const cplx<TB>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc,
+                           int target_wg) {
+  const int tm = (M + 16 * T - 1) / (16 * T), tn = (N + 16 * T - 1) / (16 * T);
+  GemmSplit g;
+  int rc = gemm_split(c, M, N, K, (long)tm * tn, target_wg, 16 * 4 * WK, alpha, beta, C, ldc, g);
+  if (rc) return rc;
+  ProfScope ps(c, transa ? PW_PROF_GEMM_CN : PW_PROF_GEMM_NN,
+               (double)M * K * sizeof(cplx<TA>) + (double)K * N * sizeof(cplx<TB>) +
+                   (double)M * N * 16.0 * (g.o.use_beta ? 2 : 1));
+  const dim3 grid((unsigned)g.nwg), blk(64 * WK);
+  if (transa)
+    hipLaunchKernelGGL((k_zgemm_wk<TC, TA, TB, 1, T, WK>), grid, blk, 0, c->stream, M, N, K, A, lda, B, ldb, g.kchunk,
+                       g.o, tm, tn, g.nz);
+  else
+    hipLaunchKernelGGL((k_zgemm_wk<TC, TA, TB, 0, T, WK>), grid, blk, 0, c->stream, M, N, K, A, lda, B, ldb, g.kchunk,
+                       g.o, tm, tn, g.nz);
+  return gemm_finish(c, M, N, g);
+}
+
 template <typename TC, typename TA, typename TB>
 static int zgemm_t(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alpha, const cplx<TA>* A,
                    long lda, const cplx<TB>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc) {
   if (M <= 0 || N <= 0) return PW_OK;
   // tuning knobs (pw_tune_set): tile shape and the split-K target workgroup count
   const int slot = transa ? 0 : 1;
-  int shape = c->tune_gemm_shape[slot];
-  if (shape < 0) {
-    // 32-column tiles when they cover N with less padding than 64-column ones (N = 160
-    // bands: 160 columns instead of 192, a fifth of the MFMA work saved).  Measured on the
-    // Si64 projector products of op_H, which run beside the FFT passes: 64 x 32 for A^H B
-    // (split-K fills the chip); for A B 128 x 32 in FP64, while in FP32 the 64 x 64 tile
-    // (less LDS per workgroup) shares the CUs with the FFT kernels better
-    // With many columns (N >= 256: Si216's 480 bands) the 128 x 64 tile halves the re-reads
-    // of the other operand and wins for both products (FP64 A^H B 8.2 -> 6.4 ms, A B 7.5 ->
-    // 5.8 ms at Ngw = 80 797, Nbeta = 1080).
-    const int pad64 = (N + 63) / 64 * 64, pad32 = (N + 31) / 32 * 32;
-    if (N >= 256) shape = 1;
-    else if (pad32 < pad64) shape = transa ? 5 : (sizeof(TC) == 8 ? 4 : 0);
-    else shape = 0;
+  int shape = c->tune_gemm_shape[slot], target = c->tune_gemm_wg[slot];
+  const double work = (double)M * N * K;
+  const long t32 = (long)((M + 31) / 32) * ((N + 31) / 32);
+  // Measured (us; K chunks so that two wavefronts per SIMD run):
+  //  - below 2^26 complex multiply-adds 32 x 32 tiles leave most of the chip idle: 16 x 16
+  //    tiles, eight wavefronts along K (A^H B 40 x 20 x 4573: 14 against 19 with 32 x 32 tiles
+  //    and 39 with LDS-staged 64 x 32 ones; 480 x 160 x 480: 17 against 32);
+  //  - A^H B of few tiles (the Gram and projector products of one k-point): four wavefronts
+  //    share a 32 x 32 tile's K, which quarters the partial sums (FP64 160 x 160 x 23871: 88
+  //    against 114 with a tile per wavefront; FP32 320 x 160 x 23871: 136 against 145); from 64
+  //    tiles on a tile per wavefront, whose neighbours share its loads in L1 (FP32 320 x 243 x
+  //    67500: 585 against 620; FP64 1080 x 480 x 80797: 5470 with 8 wavefronts against 8290);
+  //  - A B that fills the chip: a tile per wavefront in FP64 (23871 x 160 x 160: 91 against
+  //    105), four per tile in FP32, whose shorter MFMAs leave less time per load (23871 x 160 x
+  //    320: 108 against 130).
+  if constexpr (sizeof(TC) == 4) {
+    if (shape < 0 && (c->gemm_split_bf16 > 0 || (c->gemm_split_bf16 < 0 && work >= GEMM_SPLIT_MIN))) {
+      // the split-BF16 kernel's tiles
+      const int pad64 = (N + 63) / 64 * 64, pad32 = (N + 31) / 32 * 32;
+      shape = N >= 256 ? 1 : pad32 < pad64 && transa ? 5 : 0;
+      if (!target) target = transa ? (N >= 256 ? 2048 : 1024) : 512;
+    }
   }
-  // A B with a short K splits only when the tiles leave most of the chip idle; A^H B with
-  // many columns splits K over more workgroups
-  const int target = c->tune_gemm_wg[slot] > 0 ? c->tune_gemm_wg[slot] : (transa ? (N >= 256 ? 2048 : 1024) : 512);
+  if (shape < 0) {
+    if (work < 67108864.0) shape = 6;
+    else if (transa) shape = t32 < 64 ? 7 : t32 < 256 ? 0 : 1;
+    else shape = t32 < 1024 || sizeof(TC) == 4 ? 7 : 4;
+  }
+  if (!target) target = shape == 2 || shape == 3 ? 256 : shape == 5 ? 1024 : 512;
   switch (shape) {
     case 1: return zgemm_launch<TC, TA, TB, 4, 2>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
     case 4: return zgemm_launch<TC, TA, TB, 4, 1>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
     case 5: return zgemm_launch<TC, TA, TB, 2, 1>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
     case 2: return zgemm_launch<TC, TA, TB, 2, 4>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
     case 3: return zgemm_launch<TC, TA, TB, 4, 4>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
+    case 6: return zgemm_wk_launch<TC, TA, TB, 1, 8>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
+    case 7: return zgemm_wk_launch<TC, TA, TB, 2, 4>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
     default: return zgemm_launch<TC, TA, TB, 2, 2>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
   }
 }

@@ -195,10 +195,10 @@ struct pw_ctx {
   // FP32-path complex GEMMs on BF16 MFMA with 3-part operands: 1 always, 0 never, -1 by size
   int gemm_split_bf16 = -1;
   // tuning (pw_tune_set): [0] = A^H B products, [1] = A B products
-  // -1: by N (pw_gemm.hip: zgemm_t); 0: 2x2 wavefronts (64x64 tile), 1: 4x2, 2: 2x4, 3: 4x4,
-  // 4: 4x1 (128 x 32), 5: 2x1 (64 x 32)
+  // -1: by size (pw_gemm.hip: zgemm_t); 0: 2x2 wavefronts (64x64 tile), 1: 4x2, 2: 2x4, 3: 4x4,
+  // 4: 4x1 (128 x 32), 5: 2x1 (64 x 32); 6, 7: 8 / 4 wavefronts along K of a 16x16 / 32x32 tile
   int tune_gemm_shape[2] = {-1, -1};
-  int tune_gemm_wg[2] = {0, 0};     // split-K target workgroups (0 = 1024)
+  int tune_gemm_wg[2] = {0, 0};     // split-K target workgroups (0 = by shape)
   std::string err;
   // per-kernel timing (pw_profile_*): event pairs recorded around launches on `stream`
   bool profile = false;

@@ -115,11 +115,12 @@ def test_rho_batch(ns, nk, nb, mixed):
     w = np.ascontiguousarray(rng.random((nk, nb)))
     ld = np.array([p.shape[0] for p in psi], dtype=np.int64)
     pp = np.array([d.p.value for d in dev], dtype=np.uint64)
+    iks = np.arange(nk, dtype=np.int32)
     N = int(np.prod(ns))
     got = np.empty(N)
     print(f"case rho batch {ns} nk={nk} nb={nb} mixed={mixed}", flush=True)
     c.call("pw_rhoe_zero")
-    c.call("pw_rhoe_accum_batch_dev", nk, ptr(np.arange(nk, dtype=np.int32)), nb, ptr(pp), ptr(ld), ptr(w),
+    c.call("pw_rhoe_accum_batch_dev", nk, ptr(iks), nb, ptr(pp), ptr(ld), ptr(w),
            PW_MIXED if mixed else 0)
     c.call("pw_rhoe_get", ptr(got))
     ref = np.zeros(N)
