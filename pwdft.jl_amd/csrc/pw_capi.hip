@@ -103,6 +103,7 @@ void free_k(KData& k) {
   hipFree(k.d_col_cy);
   hipFree(k.d_xact);
   hipFree(k.d_ctab);
+  hipFree(k.d_ztab);
   hipFree(k.d_gk2);
   hipFree(k.d_gk);
   hipFree(k.d_gpos);
@@ -166,37 +167,34 @@ int op_H_device(pw_ctx* c, int ik, int ispin, int nb, const cplx<double>* psi, l
   if (nb == 0) return PW_OK;
   const unsigned terms = flags & PW_TERM_ALL;
   bool have = (flags & PW_ACCUMULATE) != 0;
-  // (small problems -- a few bands of a small sphere -- keep one stream: the fork and join
-  // would cost more than the overlap saves)
-  if ((terms & PW_TERM_VLOC) && (terms & PW_TERM_NLOC) && k.nbeta > 0 && c->overlap && c->stream2 &&
-      (long)k.ngw * nb >= (1L << 18)) {
-    // The nonlocal products (MFMA) run on stream2 beside the column / plane FFT passes
-    // (VALU / LDS): stream2 writes Hpsi = [Hpsi +] (beta D) (beta^H psi) first, and the gather
-    // pass, which waits for it, adds the kinetic and local terms.
-    if (ispin < 0 || ispin >= c->nspin || !c->d_v64[ispin])
-      return set_error(c, PW_ERR_STATE, "op_V_loc: potential of spin " + std::to_string(ispin) + " not set");
+  const bool vloc = (terms & PW_TERM_VLOC) != 0, nloc = (terms & PW_TERM_NLOC) && k.nbeta > 0;
+  if (vloc && (ispin < 0 || ispin >= c->nspin || !c->d_v64[ispin]))
+    return set_error(c, PW_ERR_STATE, "op_V_loc: potential of spin " + std::to_string(ispin) + " not set");
+  cplx<double>* bnl = nullptr;
+  if (nloc) {
     rc = ensure(c, &c->d_bnl, &c->bnl_bytes, (size_t)k.nbeta * nb * sizeof(cplx<double>));
     if (rc) return rc;
+    bnl = reinterpret_cast<cplx<double>*>(c->d_bnl);
+  }
+  const cplx<double> one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
+  auto project = [&]() {   // B = beta^H psi
+    if (flags & PW_MIXED)
+      return zgemm_f32in(c, 1, k.nbeta, nb, k.ngw, one, reinterpret_cast<const cplx<float>*>(k.d_beta32), k.ngw, psi,
+                         ldpsi, zero, bnl, k.nbeta, 1);
+    return zgemm(c, 1, k.nbeta, nb, k.ngw, one, reinterpret_cast<const cplx<double>*>(k.d_beta64), k.ngw, psi, ldpsi,
+                 zero, bnl, k.nbeta, 0);
+  };
+  // B = beta^H psi (MFMA) runs on stream2 beside the FFT passes (VALU, LDS).  Small problems --
+  // a few bands of a small sphere -- keep one stream: the fork and join would cost more than
+  // the overlap saves.
+  const bool fork = vloc && nloc && c->overlap && c->stream2 && (long)k.ngw * nb >= (1L << 18);
+  if (fork) {
     hipError_t e = hipEventRecord(c->ev_fork, c->stream);
     if (e == hipSuccess) e = hipStreamWaitEvent(c->stream2, c->ev_fork, 0);
     if (e != hipSuccess) return hip_check(c, e, "stream fork");
-    cplx<double>* bnl = reinterpret_cast<cplx<double>*>(c->d_bnl);
-    const cplx<double> one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
     hipStream_t main = c->stream;
     c->stream = c->stream2;  // the GEMM drivers launch on c->stream
-    if (flags & PW_MIXED) {
-      rc = zgemm_f32in(c, 1, k.nbeta, nb, k.ngw, one, reinterpret_cast<const cplx<float>*>(k.d_beta32), k.ngw,
-                       psi, ldpsi, zero, bnl, k.nbeta, 1);
-      if (!rc)
-        rc = zgemm_f32in(c, 0, k.ngw, nb, k.nbeta, one, reinterpret_cast<const cplx<float>*>(k.d_betaD32), k.ngw,
-                         bnl, k.nbeta, have ? one : zero, hpsi, ldh, 1);
-    } else {
-      rc = zgemm(c, 1, k.nbeta, nb, k.ngw, one, reinterpret_cast<const cplx<double>*>(k.d_beta64), k.ngw, psi,
-                 ldpsi, zero, bnl, k.nbeta, 0);
-      if (!rc)
-        rc = zgemm(c, 0, k.ngw, nb, k.nbeta, one, reinterpret_cast<const cplx<double>*>(k.d_betaD64), k.ngw, bnl,
-                   k.nbeta, have ? one : zero, hpsi, ldh, 0);
-    }
+    rc = project();
     e = hipEventRecord(c->ev_join, c->stream2);
     c->stream = main;
     if (!rc && e != hipSuccess) rc = hip_check(c, e, "stream join record");
@@ -204,38 +202,44 @@ int op_H_device(pw_ctx* c, int ik, int ispin, int nb, const cplx<double>* psi, l
       hipStreamWaitEvent(c->stream, c->ev_join, 0);  // keep the streams ordered on failure
       return rc;
     }
-    return vloc_apply(c, ik, ispin, nb, psi, ldpsi, hpsi, ldh, flags | PW_ACCUMULATE, c->ev_join);
   }
-  if (terms & PW_TERM_VLOC) {
-    if (ispin < 0 || ispin >= c->nspin || !c->d_v64[ispin])
-      return set_error(c, PW_ERR_STATE, "op_V_loc: potential of spin " + std::to_string(ispin) + " not set");
-    rc = vloc_apply(c, ik, ispin, nb, psi, ldpsi, hpsi, ldh, flags);
-    if (rc) return rc;
+  // With a nonlocal term the kinetic one goes into its product, which reads psi and Hpsi in row
+  // order; the scatter of the FFT result then only writes.  Its own reads of psi and Hpsi in
+  // column order cost more than their bytes (Si64 30 Ha, 243 bands FP32: 246 us without them,
+  // 702 with; FP64 Si64, 160 bands: 44 and 119).
+  if (vloc) {
+    rc = vloc_apply(c, ik, ispin, nb, psi, ldpsi, hpsi, ldh, nloc ? flags & ~(unsigned)PW_TERM_K : flags);
+    if (rc) {
+      if (fork) hipStreamWaitEvent(c->stream, c->ev_join, 0);
+      return rc;
+    }
     have = true;
-  } else if (terms & PW_TERM_K) {
+  } else if ((terms & PW_TERM_K) && !nloc) {
     rc = kinetic_apply(c, ik, nb, psi, ldpsi, hpsi, ldh, flags);
     if (rc) return rc;
     have = true;
   }
-  const bool nloc = (terms & PW_TERM_NLOC) && k.nbeta > 0;
   if (nloc) {
-    rc = ensure(c, &c->d_bnl, &c->bnl_bytes, (size_t)k.nbeta * nb * sizeof(cplx<double>));
-    if (rc) return rc;
-    cplx<double>* bnl = reinterpret_cast<cplx<double>*>(c->d_bnl);
-    const cplx<double> one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
-    if (flags & PW_MIXED) {
-      rc = zgemm_f32in(c, 1, k.nbeta, nb, k.ngw, one, reinterpret_cast<const cplx<float>*>(k.d_beta32), k.ngw,
-                       psi, ldpsi, zero, bnl, k.nbeta, 1);
-      if (rc) return rc;
-      rc = zgemm_f32in(c, 0, k.ngw, nb, k.nbeta, one, reinterpret_cast<const cplx<float>*>(k.d_betaD32),
-                       k.ngw, bnl, k.nbeta, have ? one : zero, hpsi, ldh, 1);
+    if (fork) {
+      const hipError_t e = hipStreamWaitEvent(c->stream, c->ev_join, 0);
+      if (e != hipSuccess) return hip_check(c, e, "stream join");
     } else {
-      rc = zgemm(c, 1, k.nbeta, nb, k.ngw, one, reinterpret_cast<const cplx<double>*>(k.d_beta64), k.ngw, psi,
-                 ldpsi, zero, bnl, k.nbeta, 0);
+      rc = project();
       if (rc) return rc;
-      rc = zgemm(c, 0, k.ngw, nb, k.nbeta, one, reinterpret_cast<const cplx<double>*>(k.d_betaD64), k.ngw,
-                 bnl, k.nbeta, have ? one : zero, hpsi, ldh, 0);
     }
+    GemmKin kin;
+    if (terms & PW_TERM_K) {
+      kin.gk2 = k.d_gk2;
+      kin.psi = psi;
+      kin.ldpsi = ldpsi;
+    }
+    const cplx<double> add = have ? one : zero;
+    if (flags & PW_MIXED)
+      rc = zgemm_f32in(c, 0, k.ngw, nb, k.nbeta, one, reinterpret_cast<const cplx<float>*>(k.d_betaD32), k.ngw, bnl,
+                       k.nbeta, add, hpsi, ldh, 1, kin);
+    else
+      rc = zgemm(c, 0, k.ngw, nb, k.nbeta, one, reinterpret_cast<const cplx<double>*>(k.d_betaD64), k.ngw, bnl,
+                 k.nbeta, add, hpsi, ldh, 0, kin);
     if (rc) return rc;
     have = true;
   }
@@ -554,11 +558,14 @@ int build_kdata(pw_ctx* c, KData& k, int ngw, const int64_t* idx, int base, cons
   std::sort(ent.begin(), ent.end(), [](const Ent& a, const Ent& b) {
     return a.col != b.col ? a.col < b.col : a.z < b.z;
   });
-  std::vector<int> e_igw(ngw), e_pos(ngw), col_ptr(ncol + 1, 0);
+  std::vector<int> e_igw(ngw), e_pos(ngw), col_ptr(ncol + 1, 0), ztab((size_t)ncol * n3, -1);
+  bool zhalf = true;
   const int cs = odd_stride(n3), ps = odd_stride(n1);
   for (int e = 0; e < ngw; ++e) {
     e_igw[e] = ent[e].igw;
     e_pos[e] = ent[e].col * cs + ent[e].z;
+    ztab[(size_t)ent[e].col * n3 + ent[e].z] = ent[e].igw;
+    zhalf = zhalf && line_window_holds(n3, ent[e].z);
     col_ptr[ent[e].col + 1]++;
   }
   for (int cc = 0; cc < ncol; ++cc) col_ij[cc] = (col_ij[cc] / n2) + ps * (col_ij[cc] % n2);
@@ -596,6 +603,7 @@ int build_kdata(pw_ctx* c, KData& k, int ngw, const int64_t* idx, int base, cons
   k.nxact = (int)xs.size();
   k.h_xact = xs;
   k.half = half;
+  k.zhalf = zhalf;
   int rc;
   if ((rc = upload(c, &k.d_ent_igw, e_igw.data(), ngw))) return rc;
   if ((rc = upload(c, &k.d_ent_pos, e_pos.data(), ngw))) return rc;
@@ -607,6 +615,7 @@ int build_kdata(pw_ctx* c, KData& k, int ngw, const int64_t* idx, int base, cons
   ctab.insert(ctab.end(), apos.begin(), apos.end());
   if ((rc = upload(c, &k.d_ctab, ctab.data(), ctab.size()))) return rc;
   k.d_apos = k.d_ctab + ntab;
+  if ((rc = upload(c, &k.d_ztab, ztab.data(), ztab.size()))) return rc;
   if ((rc = upload(c, &k.d_gk2, gk2.data(), ngw))) return rc;
   if ((rc = upload(c, &k.d_gk, gk, 3 * (size_t)ngw))) return rc;
   if ((rc = upload(c, &k.d_gpos, gpos.data(), ngw))) return rc;

@@ -23,6 +23,7 @@
 #include "pw_internal.h"
 #include "pw_fft_core.h"
 #include "pw_plane.h"
+#include "pw_col.h"
 
 namespace pw {
 
@@ -750,7 +751,7 @@ static bool plane_gp(const pw_ctx* c, size_t esz, int nxact, int nthreads, Plane
 
 template <typename T>
 static int vloc_run(pw_ctx* c, KData& k, const T* V, int nb, const cplx<double>* psi, long ldpsi,
-                    cplx<double>* hpsi, long ldh, int kin, int acc, hipEvent_t join = nullptr) {
+                    cplx<double>* hpsi, long ldh, int kin, int acc) {
   const size_t esz = sizeof(cplx<T>);
   const int C = cols_per_block(c, esz);
   // the gather kernel's own chunk: in FP32 at most 32 columns, so fewer bands' chunks share
@@ -760,6 +761,7 @@ static int vloc_run(pw_ctx* c, KData& k, const T* V, int nb, const cplx<double>*
   size_t plane_bytes = 0;
   int rl = 0;
   const bool compressed = !plane_applies<T>(c, k.nxact, k.half);
+  const bool cols = col_chunk<T>(c, k.zhalf) > 0;
   PlaneGP gp;
   bool global_plane = false;
   if (compressed) {
@@ -796,8 +798,11 @@ static int vloc_run(pw_ctx* c, KData& k, const T* V, int nb, const cplx<double>*
     const double psib = (double)nbb * k.ngw * 16.0;
     {
       ProfScope ps(c, PW_PROF_COL_IFFT, psib + wb + k.ngw * 8.0);
-      hipLaunchKernelGGL(k_col_ifft<T>, g1, dim3(COL_NT), col_lds(c, C, esz), c->stream, psi, ldpsi, b0,
-                         W, k.d_ent_igw, k.d_ent_pos, k.d_col_ptr, k.ncol, C, nbb, c->dim[2], tw[2]);
+      if (cols)
+        col_inv<T>(c, k, psi, ldpsi, b0, nbb, W);
+      else
+        hipLaunchKernelGGL(k_col_ifft<T>, g1, dim3(COL_NT), col_lds(c, C, esz), c->stream, psi, ldpsi, b0,
+                           W, k.d_ent_igw, k.d_ent_pos, k.d_col_ptr, k.ncol, C, nbb, c->dim[2], tw[2]);
     }
     {
       dim3 g2(c->n3, nbb);
@@ -816,27 +821,26 @@ static int vloc_run(pw_ctx* c, KData& k, const T* V, int nb, const cplx<double>*
       else
         plane_vloc<T>(c, k, W, V, nbb);
     }
-    if (join && b0 == 0) {
-      hipError_t e = hipStreamWaitEvent(c->stream, join, 0);
-      if (e != hipSuccess) return hip_check(c, e, "stream join");
-    }
     {
       ProfScope ps(c, PW_PROF_COL_FFT, wb + psib * ((kin ? 1 : 0) + (acc ? 1 : 0) + 1) + k.ngw * 16.0);
-      hipLaunchKernelGGL(k_col_fft<T>, dim3(col_grid(k.ncol, Cf, nbb)), dim3(COL_NT), col_lds(c, Cf, esz), c->stream,
-                         W, psi, ldpsi, hpsi, ldh, b0, k.d_ent_igw, k.d_ent_pos, k.d_col_ptr, k.ncol, Cf, nbb,
-                         c->dim[2], tw[2], k.d_gk2, kin, acc);
+      if (cols)
+        col_fwd<T>(c, k, psi, ldpsi, hpsi, ldh, b0, nbb, W, kin, acc);
+      else
+        hipLaunchKernelGGL(k_col_fft<T>, dim3(col_grid(k.ncol, Cf, nbb)), dim3(COL_NT), col_lds(c, Cf, esz), c->stream,
+                           W, psi, ldpsi, hpsi, ldh, b0, k.d_ent_igw, k.d_ent_pos, k.d_col_ptr, k.ncol, Cf, nbb,
+                           c->dim[2], tw[2], k.d_gk2, kin, acc);
     }
   }
   return hip_check(c, hipGetLastError(), "vloc kernels");
 }
 
 int vloc_apply(pw_ctx* c, int ik, int ispin, int nb, const cplx<double>* psi, long ldpsi,
-               cplx<double>* hpsi, long ldh, unsigned flags, hipEvent_t join) {
+               cplx<double>* hpsi, long ldh, unsigned flags) {
   const int kin = (flags & PW_TERM_K) ? 1 : 0;
   const int acc = (flags & PW_ACCUMULATE) ? 1 : 0;
   if (flags & PW_MIXED)
-    return vloc_run<float>(c, c->kd[ik], c->d_v32[ispin], nb, psi, ldpsi, hpsi, ldh, kin, acc, join);
-  return vloc_run<double>(c, c->kd[ik], c->d_v64[ispin], nb, psi, ldpsi, hpsi, ldh, kin, acc, join);
+    return vloc_run<float>(c, c->kd[ik], c->d_v32[ispin], nb, psi, ldpsi, hpsi, ldh, kin, acc);
+  return vloc_run<double>(c, c->kd[ik], c->d_v64[ispin], nb, psi, ldpsi, hpsi, ldh, kin, acc);
 }
 
 int vloc_apply_k(pw_ctx* c, KData& k, const double* V64, int nb, const cplx<double>* psi, long ldpsi,
@@ -858,6 +862,10 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
     for (int kk = 0; kk < nk; ++kk) maxcol = std::max(maxcol, c->kd[iks[kk]].ncol);
     C = std::min(C, maxcol);
   }
+  bool zhalf = true;
+  for (int kk = 0; kk < nk; ++kk) zhalf = zhalf && c->kd[iks[kk]].zhalf;
+  const int cchunk = col_chunk<T>(c, zhalf);
+  if (cchunk) C = cchunk;
   const int cnt = col_threads(c, C);
   const int nb8 = (nb + 7) / 8 * 8;
   std::vector<KBatch> kb(nk);
@@ -873,6 +881,7 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
     d.col_ptr = k.d_col_ptr;
     d.ctab = k.d_ctab;
     d.apos = k.d_apos;
+    d.ztab = k.d_ztab;
     d.gk2 = k.d_gk2;
     d.psi = psi[kk];
     d.hpsi = hpsi[kk];
@@ -906,8 +915,11 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
   const cplx<T>* tw[3];
   for (int d = 0; d < 3; ++d)
     tw[d] = reinterpret_cast<const cplx<T>*>(sizeof(T) == 8 ? c->d_tw64[d] : c->d_tw32[d]);
-  hipLaunchKernelGGL(k_col_ifft_batch<T>, dim3((unsigned)blk), dim3(cnt), col_lds(c, C, esz), c->stream, dkb,
-                     nk, nb, W, C, c->dim[2], tw[2]);
+  if (cchunk)
+    col_inv_batch<T>(c, dkb, nk, nb, blk, zhalf, W);
+  else
+    hipLaunchKernelGGL(k_col_ifft_batch<T>, dim3((unsigned)blk), dim3(cnt), col_lds(c, C, esz), c->stream, dkb,
+                       nk, nb, W, C, c->dim[2], tw[2]);
   if (planes)
     plane_vloc_batch<T>(c, dkb, nk, nb, maxx, half, W, V);
   else
@@ -917,8 +929,11 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
                          W + kb[kk].woff, V, k.d_col_cy, k.ncol, k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0], tw[1],
                          c->n3, rl);
     }
-  hipLaunchKernelGGL(k_col_fft_batch<T>, dim3((unsigned)blk), dim3(cnt), col_lds(c, C, esz), c->stream, dkb, nk,
-                     nb, W, C, c->dim[2], tw[2], kin, acc);
+  if (cchunk)
+    col_fwd_batch<T>(c, dkb, nk, nb, blk, zhalf, W, kin, acc);
+  else
+    hipLaunchKernelGGL(k_col_fft_batch<T>, dim3((unsigned)blk), dim3(cnt), col_lds(c, C, esz), c->stream, dkb, nk,
+                       nb, W, C, c->dim[2], tw[2], kin, acc);
   return hip_check(c, hipGetLastError(), "batched vloc kernels");
 }
 
@@ -1477,9 +1492,12 @@ static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldp
     const int ng = std::max(1, std::min(nbb, ngroup));
     const int bpg = (nbb + ng - 1) / ng;
     const int ngu = (nbb + bpg - 1) / bpg;
-    hipLaunchKernelGGL(k_col_ifft<T>, dim3(col_grid(k.ncol, C, nbb)), dim3(COL_NT), col_lds(c, C, esz),
-                       c->stream, psi, ldpsi, b0, W, k.d_ent_igw, k.d_ent_pos, k.d_col_ptr, k.ncol, C, nbb,
-                       c->dim[2], tw[2]);
+    if (col_chunk<T>(c, k.zhalf))
+      col_inv<T>(c, k, psi, ldpsi, b0, nbb, W);
+    else
+      hipLaunchKernelGGL(k_col_ifft<T>, dim3(col_grid(k.ncol, C, nbb)), dim3(COL_NT), col_lds(c, C, esz),
+                         c->stream, psi, ldpsi, b0, W, k.d_ent_igw, k.d_ent_pos, k.d_col_ptr, k.ncol, C, nbb,
+                         c->dim[2], tw[2]);
     ProfScope ps(c, PW_PROF_PLANE_RHOE, (double)nbb * c->n3 * k.ncol * esz + (double)ngu * c->N * 8.0);
     if (compressed)
       hipLaunchKernelGGL(k_plane_rhoe_c<T>, dim3(c->n3, ngu), dim3(PlaneNT<T>::value), plane_bytes, c->stream, W,
@@ -1502,12 +1520,13 @@ static int rhoe_batch_run(pw_ctx* c, int nk, const int* iks, int nb, const cplx<
                           const int64_t* ldpsi, const double* d_w) {
   const size_t esz = sizeof(cplx<T>);
   int maxcol = 1, maxx = 1;
-  bool half = true;
+  bool half = true, zhalf = true;
   for (int kk = 0; kk < nk; ++kk) {
     const KData& k = c->kd[iks[kk]];
     maxcol = std::max(maxcol, k.ncol);
     maxx = std::max(maxx, k.nxact);
     half = half && k.half;
+    zhalf = zhalf && k.zhalf;
   }
   const size_t kbytes = (size_t)nb * c->n3 * maxcol * esz;
   const int kc = (int)std::min<size_t>(nk, (256u << 20) / kbytes);
@@ -1518,7 +1537,9 @@ static int rhoe_batch_run(pw_ctx* c, int nk, const int* iks, int nb, const cplx<
     }
     return PW_OK;
   }
-  const int C = std::min(cols_per_block(c, esz), maxcol), cnt = col_threads(c, C), nb8 = (nb + 7) / 8 * 8;
+  const int cchunk = col_chunk<T>(c, zhalf);
+  const int C = cchunk ? cchunk : std::min(cols_per_block(c, esz), maxcol);
+  const int cnt = col_threads(c, C), nb8 = (nb + 7) / 8 * 8;
   const int ngroup = rho_groups(c, plane_rho_resident<T>(c, maxx), kc * nb);
   int rc = ensure(c, &c->d_work, &c->work_bytes, kc * kbytes);
   if (rc) return rc;
@@ -1539,6 +1560,7 @@ static int rhoe_batch_run(pw_ctx* c, int nk, const int* iks, int nb, const cplx<
       d.col_ptr = k.d_col_ptr;
       d.ctab = k.d_ctab;
       d.apos = k.d_apos;
+      d.ztab = k.d_ztab;
       d.psi = psi[k0 + i];
       d.ldpsi = ldpsi[k0 + i];
       d.woff = woff;
@@ -1554,8 +1576,11 @@ static int rhoe_batch_run(pw_ctx* c, int nk, const int* iks, int nb, const cplx<
     rc = desc_get(c, kb.data(), kb.size() * sizeof(KBatch), &dptr);
     if (rc) return rc;
     const KBatch* dkb = reinterpret_cast<const KBatch*>(dptr);
-    hipLaunchKernelGGL(k_col_ifft_batch<T>, dim3((unsigned)blk), dim3(cnt), col_lds(c, C, esz), c->stream, dkb, kn, nb,
-                       W, C, c->dim[2], twz);
+    if (cchunk)
+      col_inv_batch<T>(c, dkb, kn, nb, blk, zhalf, W);
+    else
+      hipLaunchKernelGGL(k_col_ifft_batch<T>, dim3((unsigned)blk), dim3(cnt), col_lds(c, C, esz), c->stream, dkb, kn,
+                         nb, W, C, c->dim[2], twz);
     const int tot = kn * nb, bpg = (tot + std::min(ngroup, tot) - 1) / std::min(ngroup, tot);
     const int ngu = (tot + bpg - 1) / bpg;
     plane_rho_batch<T>(c, dkb, nb, tot, maxx, W, bpg, ngu, d_w + (size_t)k0 * nb, rpart);
@@ -1603,7 +1628,10 @@ int g2r_apply(pw_ctx* c, KData& k, int nf, const cplx<double>* fG, long ldf, dou
   for (int d = 0; d < 3; ++d) tw[d] = reinterpret_cast<const cplx<double>*>(c->d_tw64[d]);
   for (int b0 = 0; b0 < nf; b0 += bb) {
     const int nbb = std::min(bb, nf - b0);
-    hipLaunchKernelGGL(k_col_ifft<double>, dim3(col_grid(k.ncol, C, nbb)), dim3(COL_NT), col_lds(c, C, esz),
+    if (col_chunk<double>(c, k.zhalf))
+      col_inv<double>(c, k, fG, ldf, b0, nbb, W);
+    else
+      hipLaunchKernelGGL(k_col_ifft<double>, dim3(col_grid(k.ncol, C, nbb)), dim3(COL_NT), col_lds(c, C, esz),
                        c->stream, fG, ldf, b0, W, k.d_ent_igw, k.d_ent_pos, k.d_col_ptr, k.ncol, C, nbb,
                        c->dim[2], tw[2]);
     double* o = out + (long)b0 * c->N;

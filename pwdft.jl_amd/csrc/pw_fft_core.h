@@ -262,4 +262,27 @@ inline bool line_window_holds(int n, int x) {
   return 2 * nz >= p.r0 || x < nz * p.r1 || x >= n - nz * p.r1;
 }
 
+// The inputs a first pass takes (and the outputs a last pass leaves): element j + R1 r for the
+// r with live(r).  Spheres of half the grid's radius (wave functions) occupy |x| < N / 4 or so
+// on each side of zero, so with HALF only the NZ lowest and the NZ highest r can be non-zero;
+// the others are constants the butterflies fold away.
+template <int N, bool HALF>
+struct Window {
+  using P = LinePlan<N>;
+  static constexpr int NZ = line_window(N, P::R1);
+  static constexpr bool all = !HALF || 2 * NZ >= P::R0;
+  static constexpr int NI = all ? P::R0 : 2 * NZ;
+  __host__ __device__ static constexpr int r(int i) { return all || i < NZ ? i : P::R0 - 2 * NZ + i; }
+};
+
+template <typename T, int S, int N, bool HALF>
+__device__ inline void dft_window(const cplx<T>* in, cplx<T>* v) {
+  using W = Window<N, HALF>;
+#pragma unroll
+  for (int r = 0; r < LinePlan<N>::R0; ++r) v[r] = mk((T)0, (T)0);
+#pragma unroll
+  for (int i = 0; i < W::NI; ++i) v[W::r(i)] = in[i];
+  DFT<T, S, LinePlan<N>::R0>::run(v);
+}
+
 }  // namespace pw

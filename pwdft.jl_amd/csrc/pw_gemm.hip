@@ -171,13 +171,18 @@ struct GemmOut {
   cplx<double> alpha, beta;
   int direct, use_beta;
   cplx<double>* part;   // !direct: partial sums [z][n][m]
+  GemmKin kin;          // kin.gk2 set: C += 1/2 gk2[m] psi[n][m]
 };
+__device__ inline void gemm_finish_one(const GemmOut& o, int m, int n, cplx<double> v) {
+  cplx<double> r = cmul(o.alpha, v);
+  if (o.use_beta) r = r + cmul(o.beta, o.C[(long)n * o.ldc + m]);
+  if (o.kin.gk2) r = r + scal(0.5 * o.kin.gk2[m], o.kin.psi[(long)n * o.kin.ldpsi + m]);
+  o.C[(long)n * o.ldc + m] = r;
+}
 __device__ inline void gemm_store(const GemmOut& o, int M, int N, int z, int m, int n, cplx<double> v) {
   if (m >= M || n >= N) return;
   if (o.direct) {
-    cplx<double> r = cmul(o.alpha, v);
-    if (o.use_beta) r = r + cmul(o.beta, o.C[(long)n * o.ldc + m]);
-    o.C[(long)n * o.ldc + m] = r;
+    gemm_finish_one(o, m, n, v);
   } else {
     o.part[((long)z * N + n) * M + m] = v;
   }
@@ -408,17 +413,13 @@ k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
       }
 }
 
-__global__ void k_zgemm_reduce(int M, int N, int nz, const cplx<double>* __restrict__ part,
-                               cplx<double>* __restrict__ C, long ldc, cplx<double> alpha,
-                               cplx<double> beta, int use_beta) {
+__global__ void k_zgemm_reduce(int M, int N, int nz, GemmOut o) {
   const long tot = (long)M * N;
   for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
     const int m = (int)(t % M), n = (int)(t / M);
     cplx<double> s = mk(0.0, 0.0);
-    for (int z = 0; z < nz; ++z) s = s + part[((long)z * N + n) * M + m];
-    cplx<double> r = cmul(alpha, s);
-    if (use_beta) r = r + cmul(beta, C[(long)n * ldc + m]);
-    C[(long)n * ldc + m] = r;
+    for (int z = 0; z < nz; ++z) s = s + o.part[((long)z * N + n) * M + m];
+    gemm_finish_one(o, m, n, s);
   }
 }
 
@@ -427,6 +428,11 @@ __global__ void k_zgemm_reduce(int M, int N, int nz, const cplx<double>* __restr
 // Si64 (1.2e9).
 constexpr double GEMM_SPLIT_MIN = 8589934592.0;
 
+// k-steps that one FP32 accumulator of the shared-tile kernels takes before its sum goes to FP64:
+// as long as the chains of the kernel these replaced (Si64 30 Ha projector products, error of
+// op_H against FP64: 1.3e-8 with 128, 2.2e-8 with 704, 1.7e-8 before).
+constexpr int GEMM_F32_CHAIN = 128;
+
 // Split of K over `nz` chunks for about `slots` workgroups on `tiles` tiles (no chunk shorter
 // than `kmin`), the partial-sum workspace and the epilogue.
 struct GemmSplit {
@@ -434,10 +440,11 @@ struct GemmSplit {
   long nwg = 0;
   GemmOut o{};
 };
-static int gemm_split(pw_ctx* c, int M, int N, int K, long tiles, long slots, int kmin, cplx<double> alpha,
-                      cplx<double> beta, cplx<double>* C, long ldc, GemmSplit& g) {
+static int gemm_split(pw_ctx* c, int M, int N, int K, long tiles, long slots, int kmin, int kmax, cplx<double> alpha,
+                      cplx<double> beta, cplx<double>* C, long ldc, const GemmKin& kin, GemmSplit& g) {
   const int ksteps = (K + GBK - 1) / GBK;
   long nz = std::min<long>(slots / std::max<long>(tiles, 1), K / std::max(kmin, GBK));
+  nz = std::max<long>(nz, kmax > 0 ? (K + kmax - 1) / kmax : 1);
   nz = std::max<long>(nz, 1);
   // a no-allocation call splits K only as far as its fixed partial-sum array holds
   if (c->no_alloc && nz > 1) nz = std::max<long>(1, std::min<long>(nz, (long)(c->gpart_bytes / ((size_t)M * N * 16))));
@@ -453,6 +460,7 @@ static int gemm_split(pw_ctx* c, int M, int N, int K, long tiles, long slots, in
   g.o.beta = beta;
   g.o.use_beta = (beta.x != 0.0 || beta.y != 0.0) ? 1 : 0;
   g.o.direct = nz == 1 ? 1 : 0;
+  g.o.kin = kin;
   if (nz > 1) {
     int rc = ensure(c, &c->d_gpart, &c->gpart_bytes, (size_t)nz * M * N * sizeof(cplx<double>));
     if (rc) return rc;
@@ -464,8 +472,7 @@ static int gemm_finish(pw_ctx* c, int M, int N, const GemmSplit& g) {
   if (g.nz > 1) {
     const long tot = (long)M * N;
     const int blocks = (int)std::min<long>((tot + 255) / 256, 2048);
-    hipLaunchKernelGGL(k_zgemm_reduce, dim3(blocks), dim3(256), 0, c->stream, M, N, g.nz, g.o.part, g.o.C, g.o.ldc,
-                       g.o.alpha, g.o.beta, g.o.use_beta);
+    hipLaunchKernelGGL(k_zgemm_reduce, dim3(blocks), dim3(256), 0, c->stream, M, N, g.nz, g.o);
   }
   return hip_check(c, hipGetLastError(), "zgemm");
 }
@@ -474,11 +481,11 @@ static int gemm_finish(pw_ctx* c, int M, int N, const GemmSplit& g) {
 template <typename TC, typename TA, typename TB, int WM, int WN>
 static int zgemm_launch(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alpha, const cplx<TA>* A,
                         long lda, const cplx<TB>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc,
-                        int target_wg) {
+                        const GemmKin& kin, int target_wg) {
   constexpr int BMC = 32 * WM, BNC = 32 * WN;
   const int tm = (M + BMC - 1) / BMC, tn = (N + BNC - 1) / BNC;
   GemmSplit g;
-  int rc = gemm_split(c, M, N, K, (long)tm * tn, target_wg, 128, alpha, beta, C, ldc, g);
+  int rc = gemm_split(c, M, N, K, (long)tm * tn, target_wg, 128, 0, alpha, beta, C, ldc, kin, g);
   if (rc) return rc;
   bool split_bf16 = false;
   // the three-part operands of a 128 x 128 tile do not fit in LDS: that shape keeps FP32 MFMA
@@ -516,10 +523,10 @@ static int zgemm_launch(pw_ctx* c, int transa, int M, int N, int K, cplx<double>
 template <typename TC, typename TA, typename TB, int T, int WK>
 static int zgemm_wk_launch(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alpha, const cplx<TA>* A,
                            long lda, const cplx<TB>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc,
-                           int target_wg) {
+                           const GemmKin& kin, int target_wg) {
   const int tm = (M + 16 * T - 1) / (16 * T), tn = (N + 16 * T - 1) / (16 * T);
   GemmSplit g;
-  int rc = gemm_split(c, M, N, K, (long)tm * tn, target_wg, 16 * 4 * WK, alpha, beta, C, ldc, g);
+  int rc = gemm_split(c, M, N, K, (long)tm * tn, target_wg, 16 * 4 * WK, sizeof(TC) == 4 ? GEMM_F32_CHAIN * 4 * WK : 0, alpha, beta, C, ldc, kin, g);
   if (rc) return rc;
   ProfScope ps(c, transa ? PW_PROF_GEMM_CN : PW_PROF_GEMM_NN,
                (double)M * K * sizeof(cplx<TA>) + (double)K * N * sizeof(cplx<TB>) +
@@ -536,7 +543,8 @@ static int zgemm_wk_launch(pw_ctx* c, int transa, int M, int N, int K, cplx<doub
 
 template <typename TC, typename TA, typename TB>
 static int zgemm_t(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alpha, const cplx<TA>* A,
-                   long lda, const cplx<TB>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc) {
+                   long lda, const cplx<TB>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc,
+                   const GemmKin& kin) {
   if (M <= 0 || N <= 0) return PW_OK;
   // tuning knobs (pw_tune_set): tile shape and the split-K target workgroup count
   const int slot = transa ? 0 : 1;
@@ -550,8 +558,10 @@ static int zgemm_t(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alph
   //  - A^H B of few tiles (the Gram and projector products of one k-point): four wavefronts
   //    share a 32 x 32 tile's K, which quarters the partial sums (FP64 160 x 160 x 23871: 88
   //    against 114 with a tile per wavefront; FP32 320 x 160 x 23871: 136 against 145); from 64
-  //    tiles on a tile per wavefront, whose neighbours share its loads in L1 (FP32 320 x 243 x
-  //    67500: 585 against 620; FP64 1080 x 480 x 80797: 5470 with 8 wavefronts against 8290);
+  //    tiles on, in FP64, a tile per wavefront, whose neighbours share its loads in L1 (1080 x
+  //    480 x 80797: 5470 with 8 wavefronts against 8290).  FP32 keeps the shared tile, whose
+  //    chains of FP32 sums are a quarter as long (320 x 243 x 67500: 620 against 585, with half
+  //    the rounding error);
   //  - A B that fills the chip: a tile per wavefront in FP64 (23871 x 160 x 160: 91 against
   //    105), four per tile in FP32, whose shorter MFMAs leave less time per load (23871 x 160 x
   //    320: 108 against 130).
@@ -565,33 +575,34 @@ static int zgemm_t(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alph
   }
   if (shape < 0) {
     if (work < 67108864.0) shape = 6;
-    else if (transa) shape = t32 < 64 ? 7 : t32 < 256 ? 0 : 1;
+    else if (transa) shape = t32 < 64 || sizeof(TC) == 4 ? 7 : t32 < 256 ? 0 : 1;
     else shape = t32 < 1024 || sizeof(TC) == 4 ? 7 : 4;
   }
   if (!target) target = shape == 2 || shape == 3 ? 256 : shape == 5 ? 1024 : 512;
   switch (shape) {
-    case 1: return zgemm_launch<TC, TA, TB, 4, 2>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
-    case 4: return zgemm_launch<TC, TA, TB, 4, 1>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
-    case 5: return zgemm_launch<TC, TA, TB, 2, 1>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
-    case 2: return zgemm_launch<TC, TA, TB, 2, 4>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
-    case 3: return zgemm_launch<TC, TA, TB, 4, 4>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
-    case 6: return zgemm_wk_launch<TC, TA, TB, 1, 8>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
-    case 7: return zgemm_wk_launch<TC, TA, TB, 2, 4>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
-    default: return zgemm_launch<TC, TA, TB, 2, 2>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, target);
+    case 1: return zgemm_launch<TC, TA, TB, 4, 2>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin, target);
+    case 4: return zgemm_launch<TC, TA, TB, 4, 1>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin, target);
+    case 5: return zgemm_launch<TC, TA, TB, 2, 1>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin, target);
+    case 2: return zgemm_launch<TC, TA, TB, 2, 4>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin, target);
+    case 3: return zgemm_launch<TC, TA, TB, 4, 4>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin, target);
+    case 6: return zgemm_wk_launch<TC, TA, TB, 1, 8>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin, target);
+    case 7: return zgemm_wk_launch<TC, TA, TB, 2, 4>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin, target);
+    default: return zgemm_launch<TC, TA, TB, 2, 2>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin, target);
   }
 }
 
 int zgemm(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alpha, const cplx<double>* A, long lda,
-          const cplx<double>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc, int prec) {
-  if (prec) return zgemm_t<float, double, double>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
-  return zgemm_t<double, double, double>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+          const cplx<double>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc, int prec,
+          const GemmKin& kin) {
+  if (prec) return zgemm_t<float, double, double>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin);
+  return zgemm_t<double, double, double>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin);
 }
 
 int zgemm_f32in(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alpha, const cplx<float>* A,
                 long lda, const cplx<double>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc,
-                int prec) {
+                int prec, const GemmKin& kin) {
   (void)prec;
-  return zgemm_t<float, float, double>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+  return zgemm_t<float, float, double>(c, transa, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, kin);
 }
 
 }  // namespace pw

@@ -94,7 +94,9 @@ struct KData {
   int* d_xact = nullptr;      // [nxact] distinct x of the columns
   int* d_ctab = nullptr;      // [nxact * n2] column of (a, y), x = xact[a], or -1
   int* d_apos = nullptr;      // [n1]    a of x, or -1 (in d_ctab's allocation)
-  bool half = false;          // every x and y lies in the half-sphere window of its line plan (pw_plane.h)
+  int* d_ztab = nullptr;      // [ncol * n3] psi row at (column, z), or -1
+  bool half = false;          // every x and y lies in the half-sphere window of its line plan (pw_fft_core.h)
+  bool zhalf = false;         // and every z
   double* d_gk2 = nullptr;    // [ngw]   |G+k|^2
   double* d_gk = nullptr;     // [3*ngw] G+k (x,y,z per entry, column-major 3 x ngw)
   int* d_gpos = nullptr;      // [ngw]   psi row -> x + ps (y + n2 z), ps = odd_stride(n1): slot in a whole padded grid
@@ -113,6 +115,7 @@ struct KBatch {
   const int* col_ptr;
   const int* ctab;
   const int* apos;
+  const int* ztab;
   const double* gk2;
   const cplx<double>* psi;
   cplx<double>* hpsi;
@@ -310,10 +313,8 @@ int op_H_device(pw_ctx* c, int ik, int ispin, int nb, const cplx<double>* psi, l
                 long ldh, unsigned flags);
 
 // FFT drivers (pw_fft.hip)
-// join: when set, the stream waits for this event before the first gather pass (the event
-// marks work on another stream that writes hpsi first).
 int vloc_apply(pw_ctx* c, int ik, int ispin, int nb, const cplx<double>* psi, long ldpsi,
-               cplx<double>* hpsi, long ldh, unsigned flags, hipEvent_t join = nullptr);
+               cplx<double>* hpsi, long ldh, unsigned flags);
 int kinetic_apply(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldpsi, cplx<double>* hpsi,
                   long ldh, unsigned flags);
 int rhoe_accum(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldpsi, const double* d_w,
@@ -390,14 +391,20 @@ int heev_small_batch(pw_ctx* c, int n, int nbatch, cplx<double>* A, long lda, lo
 int chol_inv_small_batch(pw_ctx* c, int n, int nbatch, cplx<double>* A, long lda, long stride, int* d_info);
 int small_dense_max_n();
 
+// The kinetic term a product may add to its result (gk2 set): C += 1/2 gk2[m] psi[n ldpsi + m].
+struct GemmKin {
+  const double* gk2 = nullptr;
+  const cplx<double>* psi = nullptr;
+  long ldpsi = 0;
+};
 // GEMM drivers (pw_gemm.hip)
 // C (M x N) = alpha * op(A) * B + beta * C ; op(A) = A (transa = 0, A is M x K) or
 // A^H (transa = 1, A is K x M).  All pointers are device pointers.
 int zgemm(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alpha, const cplx<double>* A,
           long lda, const cplx<double>* B, long ldb, cplx<double> beta, cplx<double>* C, long ldc,
-          int prec);
+          int prec, const GemmKin& kin = GemmKin());
 int zgemm_f32in(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alpha, const cplx<float>* A,
                 long lda, const cplx<double>* B, long ldb, cplx<double> beta, cplx<double>* C,
-                long ldc, int prec);
+                long ldc, int prec, const GemmKin& kin = GemmKin());
 
 }  // namespace pw

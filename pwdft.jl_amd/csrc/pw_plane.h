@@ -46,29 +46,6 @@ struct PlaneArgs {
 
 enum { MODE_VLOC = 0, MODE_RHO = 1, MODE_REAL = 2, MODE_RHOREG = 3 };
 
-// The inputs a first pass takes (and the outputs a last pass leaves): element j + R1 r for the
-// r with live(r).  Spheres of half the grid's radius (wave functions) occupy |x| < N / 4 or so
-// on each side of zero, so with HALF only the NZ lowest and the NZ highest r can be non-zero;
-// the others are constants the butterflies fold away.
-template <int N, bool HALF>
-struct Window {
-  using P = LinePlan<N>;
-  static constexpr int NZ = line_window(N, P::R1);
-  static constexpr bool all = !HALF || 2 * NZ >= P::R0;
-  static constexpr int NI = all ? P::R0 : 2 * NZ;
-  __host__ __device__ static constexpr int r(int i) { return all || i < NZ ? i : P::R0 - 2 * NZ + i; }
-};
-
-template <typename T, int S, int N, bool HALF>
-__device__ inline void dft_window(const cplx<T>* in, cplx<T>* v) {
-  using W = Window<N, HALF>;
-#pragma unroll
-  for (int r = 0; r < LinePlan<N>::R0; ++r) v[r] = mk((T)0, (T)0);
-#pragma unroll
-  for (int i = 0; i < W::NI; ++i) v[W::r(i)] = in[i];
-  DFT<T, S, LinePlan<N>::R0>::run(v);
-}
-
 // Inverse y-FFT of the active x lines, from the plane w (ncol entries) into Yc.
 template <typename T, int N, bool HALF>
 __device__ inline void plane_y_inv(LDS_AS cplx<T>* Yc, int nl, const cplx<T>* w, const int* ctab,

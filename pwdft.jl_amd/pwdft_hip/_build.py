@@ -12,12 +12,13 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "csrc")
 SOURCES = ["pw_capi.hip", "pw_fft.hip", "pw_plane.hip", "pw_plane_v64.hip", "pw_plane_v64f.hip", "pw_plane_v32.hip",
-           "pw_plane_r64.hip", "pw_plane_r32.hip", "pw_plane_g64.hip", "pw_gemm.hip", "pw_forces.hip", "pw_batch.hip", "pw_dense.hip", "pw_scf.hip", "pw_proj.hip", "pw_eig.hip", "pw_lobpcg.hip", "pw_small.hip", "pw_noalloc.hip"]
+           "pw_plane_r64.hip", "pw_plane_r32.hip", "pw_plane_g64.hip", "pw_col.hip", "pw_col_c64.hip",
+           "pw_col_c64f.hip", "pw_col_c32.hip", "pw_gemm.hip", "pw_forces.hip", "pw_batch.hip", "pw_dense.hip", "pw_scf.hip", "pw_proj.hip", "pw_eig.hip", "pw_lobpcg.hip", "pw_small.hip", "pw_noalloc.hip"]
 OUT = os.path.join(HERE, "libpwdft_hip.so")
 
-# Flags of single sources: the plane kernels' pruned butterflies fold their zero inputs away
+# Flags of single sources: the plane and column kernels' pruned butterflies fold their zero inputs away
 # only where x + 0 may become x, which differs from IEEE for a negative zero
-EXTRA_FLAGS = {s: ["-fno-signed-zeros"] for s in SOURCES if s.startswith("pw_plane_")}
+EXTRA_FLAGS = {s: ["-fno-signed-zeros"] for s in SOURCES if s.startswith(("pw_plane_", "pw_col_"))}
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -46,7 +47,7 @@ def build_library(verbose=False):
         jobs = [[hipcc] + [f for f in HIPCC_FLAGS if f != "-shared"] + EXTRA_FLAGS.get(s, []) + ["-c", "-o", o, os.path.join(CSRC, s)]
                 for s, o in zip(SOURCES, objs)]
         with ThreadPoolExecutor(max_workers=max(1, min(8, os.cpu_count() or 1))) as pool:
-            list(pool.map(run, sorted(jobs, key=lambda j: "pw_plane_" not in j[-1])))
+            list(pool.map(run, sorted(jobs, key=lambda j: "pw_plane_" not in j[-1] and "pw_col_" not in j[-1])))
         run([hipcc] + HIPCC_FLAGS + ["-o", tmp] + objs + LIBS)
     n = check_no_packed_fp32(tmp)
     os.replace(tmp, OUT)

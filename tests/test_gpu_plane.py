@@ -1,4 +1,4 @@
-"""The plane kernels (csrc/pw_plane.h) through the C ABI against numpy's FFT: every line
+"""The plane and column kernels (csrc/pw_plane.h, pw_col.h) through the C ABI against numpy's FFT: every line
 length with a two-pass plan, lengths without one, unequal lengths, index sets inside and
 outside the half-sphere window, and density groups of several bands.  Tolerances are those
 of the operator tests: 1e-12 (FP64) and 2e-5 (mixed) of the largest value."""
@@ -53,6 +53,8 @@ VLOC += [((n, n, 12), "full", False) for n in (12, 20, 27, 45, 72, 75, 96)]
 VLOC += [((n, n, 12), "full", True) for n in (27, 72)]
 VLOC += [((40, 75, 12), "half", m) for m in (False, True)] + [((75, 40, 12), "half", m) for m in (False, True)]
 VLOC += [((108, 64, 16), "half", False), ((27, 160, 12), "half", True), ((45, 36, 12), "full", False)]
+VLOC += [((16, 15, n), "half", m) for n in PLANS for m in (False, True)]
+VLOC += [((16, 15, n), "full", False) for n in PLANS] + [((16, 15, n), "full", True) for n in (27, 72, 125)]
 VLOC += [((125, 8, 12), "half", False), ((10, 125, 12), "half", True), ((5, 6, 4), "full", False)]
 
 
