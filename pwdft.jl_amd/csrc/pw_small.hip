@@ -23,6 +23,7 @@
 #include <cmath>
 
 #include "pw_internal.h"
+#include "pw_fft_core.h"
 
 namespace pw {
 
@@ -221,6 +222,200 @@ __global__ void __launch_bounds__(SM_NT) k_heev_jacobi(cplx<double>* __restrict_
   if (lane == 0 && info) info[blockIdx.x] = converged ? 0 : 1;
 }
 
+// The same solver for n <= 32, built for the length of a round, which the rotation parameters'
+// serial chain, the barriers and the instructions around them set (mean per solve over an SCF of
+// Si2, n = 24: 184 us, 16: 76, 8: 17; 110 over the three orders with the kernel above, 78 now):
+//  - A is updated from one buffer into another, so a round has one barrier: every wavefront
+//    computes all rotation parameters for itself from the buffer nobody writes;
+//  - a thread keeps one block of A or one pair of V for the whole solve (no index division per
+//    round), A's blocks and V's pairs on different wavefronts side by side;
+//  - tan(theta) only has to annihilate A_pq to about 1e-14 of itself, so it comes from FP32 root
+//    and reciprocal and one Newton step; c = (1 + t^2)^(-1/2) and s = t c, which make the
+//    rotation orthogonal, stay FP64.
+__device__ inline void jac_pair(int r, int k, int m, int n, int& p, int& q) {
+  if (k == 0) {
+    p = m - 1;
+    q = r;
+  } else {
+    p = r + k;
+    if (p >= m - 1) p -= m - 1;
+    q = r - k + (m - 1);
+    if (q >= m - 1) q -= m - 1;
+  }
+  if (p > q) { const int t = p; p = q; q = t; }
+  if (q >= n) q = -1;   // p meets the dummy: not rotated this round
+}
+
+constexpr int JLD = 33;   // column stride: odd, and a constant
+
+template <int NT>
+__global__ void __launch_bounds__(NT) k_heev_jacobi32(cplx<double>* __restrict__ A, long lda, long stride, int n,
+                                                      double* __restrict__ w, int nvec, int* __restrict__ info) {
+  constexpr int NW = NT / 64;
+  extern __shared__ char smem_raw[];
+  LDS_AS cplx<double>* cur = (LDS_AS cplx<double>*)smem_raw;   // n columns of JLD
+  LDS_AS cplx<double>* nxt = cur + n * JLD;
+  LDS_AS cplx<double>* v = nxt + n * JLD;
+  __shared__ cplx<double> rcs[NW][16], rph[NW][16];   // (c, s) and e^{-i phi} of each pair
+  __shared__ int pq[31 * 16];   // slot p | q << 8 of every pair of every round; q = 255: the dummy
+  __shared__ double dsort[32];
+  __shared__ int rank[32];
+  __shared__ double red[NW];
+  __shared__ int flag;
+  cplx<double>* M = A + (long)blockIdx.x * stride;
+  const int tid = threadIdx.x, wl = tid & 63, wave = tid >> 6;
+  const int nn = n * n;
+  double fro = 0.0;
+  for (int t = tid; t < nn; t += NT) {
+    const int i = t % n, j = t / n;
+    cplx<double> x;
+    if (i < j) x = M[(long)j * lda + i];
+    else if (i == j) x = mk(M[(long)j * lda + i].x, 0.0);
+    else { const cplx<double> u = M[(long)i * lda + j]; x = mk(u.x, -u.y); }
+    cur[i + JLD * j] = x;
+    v[i + JLD * j] = mk(i == j ? 1.0 : 0.0, 0.0);
+    fro += x.x * x.x + x.y * x.y;
+  }
+  const int m = (n + 1) / 2 * 2, npair = m / 2;
+  for (int t = tid; t < (m - 1) * 16; t += NT) {
+    int p = 0, q = 255;
+    if ((t & 15) < npair) jac_pair(t >> 4, t & 15, m, n, p, q);
+    pq[t] = p | (q < 0 ? 255 : q) << 8;
+  }
+  for (int o = 32; o > 0; o >>= 1) fro += __shfl_xor(fro, o, 64);
+  if (wl == 0) red[wave] = fro;
+  __syncthreads();
+  fro = 0.0;
+  for (int q = 0; q < NW; ++q) fro += red[q];
+  // the floor of the general kernel: below it an entry is the rotations' own rounding noise
+  const double gfloor2 = 4.0 * 2.220446049250313e-16 * 2.220446049250313e-16 * fro;
+  // this thread's work: A blocks (rows of pair k, columns of pair j), then V pairs (row j of V,
+  // columns of pair k), the V items starting on a wavefront of their own
+  const int na = npair * npair, v0 = (na + 63) / 64 * 64;
+  const int kind = tid < na ? 1 : tid >= v0 && tid < v0 + npair * n ? 2 : 0;
+  const int u0 = kind == 2 ? tid - v0 : tid, d0 = kind == 2 ? n : npair;
+  const int j = kind == 2 ? u0 % d0 : u0 / d0, k = kind == 2 ? u0 / d0 : u0 % d0;
+  bool converged = false;
+  for (int sweep = 0; sweep < SM_SWEEPS; ++sweep) {
+    if (tid == 0) flag = 0;
+    // this round's pairs, read a round ahead: the wavefront's wl-th, and the item's two
+    int ew = pq[wl & 15], ek = pq[k], ej = kind == 1 ? pq[j] : 0;
+    for (int r = 0; r < m - 1; ++r) {
+      const int cw = ew, ck = ek, cj = ej;
+      const int rn = r + 1 < m - 1 ? (r + 1) * 16 : 0;
+      ew = pq[rn + (wl & 15)];
+      ek = pq[rn + k];
+      if (kind == 1) ej = pq[rn + j];
+      if (wl < npair) {
+        const int p = cw & 255, q = cw >> 8;
+        double c = 1.0, s = 0.0;
+        cplx<double> ph = mk(1.0, 0.0);
+        if (q != 255) {
+          const cplx<double> g = cur[p + JLD * q];
+          const double ag2 = g.x * g.x + g.y * g.y;
+          const double app = cur[p + JLD * p].x, aqq = cur[q + JLD * q].x;
+          if (ag2 > 1e-30 * fabs(app * aqq) && ag2 > gfloor2) {
+            const double rag = rsqrt(ag2);   // 1 / |A_pq|
+            const double tau = (aqq - app) * (0.5 * rag);   // |tau| < 1e16 by the floor
+            const float tf = fabsf((float)tau);
+            double t = (double)__builtin_amdgcn_rcpf(tf + __builtin_amdgcn_sqrtf(1.0f + tf * tf));
+            const double at = fabs(tau);
+            // t^2 + 2 |tau| t - 1 = 0
+            t -= fma(t, t + 2.0 * at, -1.0) * (double)__builtin_amdgcn_rcpf(2.0f * ((float)t + tf));
+            if (tau < 0.0) t = -t;
+            c = rsqrt(1.0 + t * t);
+            s = t * c;
+            ph = mk(g.x * rag, -g.y * rag);   // e^{-i phi}
+          }
+        }
+        rcs[wave][wl] = mk(c, s);
+        rph[wave][wl] = ph;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      if (kind == 1) {
+        const int p = ck & 255, q = ck >> 8, p2 = cj & 255, q2 = cj >> 8;
+        const bool qv = q != 255, q2v = q2 != 255;
+        const cplx<double> z = mk(0.0, 0.0);
+        cplx<double> b00 = cur[p + JLD * p2];
+        cplx<double> b01 = q2v ? cur[p + JLD * q2] : z;
+        cplx<double> b10 = qv ? cur[q + JLD * p2] : z;
+        cplx<double> b11 = (qv && q2v) ? cur[q + JLD * q2] : z;
+        const cplx<double> cs = rcs[wave][k], cs2 = rcs[wave][j];
+        if (cs2.y != 0.0) {   // columns p2, q2
+          const cplx<double> ph2 = rph[wave][j];
+          jac_rot(b00, b01, cs2.x, cs2.y, ph2);
+          jac_rot(b10, b11, cs2.x, cs2.y, ph2);
+        }
+        if (cs.y != 0.0) {    // rows p, q: e^{i phi}
+          const cplx<double> phc = mk(rph[wave][k].x, -rph[wave][k].y);
+          jac_rot(b00, b10, cs.x, cs.y, phc);
+          jac_rot(b01, b11, cs.x, cs.y, phc);
+        }
+        nxt[p + JLD * p2] = b00;
+        if (q2v) nxt[p + JLD * q2] = b01;
+        if (qv) nxt[q + JLD * p2] = b10;
+        if (qv && q2v) nxt[q + JLD * q2] = b11;
+      } else if (kind == 2) {
+        const cplx<double> cs = rcs[wave][k];
+        if (cs.y != 0.0) {
+          const int p = ck & 255, q = ck >> 8;
+          cplx<double> x0 = v[j + JLD * p], x1 = v[j + JLD * q];
+          jac_rot(x0, x1, cs.x, cs.y, rph[wave][k]);
+          v[j + JLD * p] = x0;
+          v[j + JLD * q] = x1;
+        }
+      }
+      __syncthreads();
+      LDS_AS cplx<double>* t = cur;
+      cur = nxt;
+      nxt = t;
+    }
+    // would the next sweep rotate any pair?  (the rotations' own test on every pair)
+    int any = 0;
+    if (kind == 1) {
+      // the blocks of round 0's pairs hold every entry once
+      const int row[2] = {pq[k] & 255, pq[k] >> 8}, col[2] = {pq[j] & 255, pq[j] >> 8};
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const int i = row[a], l = col[b];
+          if (l != 255 && l > i) {
+            const cplx<double> g = cur[i + JLD * l];
+            const double ag2 = g.x * g.x + g.y * g.y;
+            if (ag2 > 1e-30 * fabs(cur[i + JLD * i].x * cur[l + JLD * l].x) && ag2 > gfloor2) any = 1;
+          }
+        }
+    }
+    if (any) flag = 1;
+    __syncthreads();
+    const int again = flag;
+    __syncthreads();
+    if (!again) {
+      converged = true;
+      break;
+    }
+  }
+  // eigenvalues: the diagonal; sort ascending (ties by index) with the vectors
+  if (tid < n) dsort[tid] = cur[tid + JLD * tid].x;
+  __syncthreads();
+  if (tid < n) {
+    const double d = dsort[tid];
+    int r = 0;
+    for (int j = 0; j < n; ++j) r += (dsort[j] < d || (dsort[j] == d && j < tid)) ? 1 : 0;
+    rank[tid] = r;
+    w[(long)blockIdx.x * n + r] = d;
+  }
+  __syncthreads();
+  for (int t = tid; t < nn; t += NT) {
+    const int i = t % n, j = t / n;
+    const int r = rank[j];
+    if (r < nvec) M[(long)r * lda + i] = v[i + JLD * j];
+  }
+  if (tid == 0 && info) info[blockIdx.x] = converged ? 0 : 1;
+}
+
 // Matrix b of the stack: inv(chol(Hermitian(A)).U) in place, strict lower triangle zeroed;
 // info[b] (potrf) and info[nbatch + b] (trtri) as rocSOLVER would set them.
 // Thread (ti, tj) of a G x G grid (G = 16 or 32) holds the entries (ti + G a, tj + G b), a, b < 64 / G, in
@@ -386,6 +581,16 @@ __global__ void __launch_bounds__(G * G) k_chol_inv_small(cplx<double>* __restri
 int heev_small_batch(pw_ctx* c, int n, int nbatch, cplx<double>* A, long lda, long stride, double* d_w, int nvec,
                      int* d_info) {
   if (n < 1 || n > SM_NMAX || nbatch < 1) return set_error(c, PW_ERR_ARG, "heev_small_batch: order out of range");
+  if (n <= 32) {
+    // one thread per block of A and per pair of V
+    const int npair = (n + 1) / 2, items = (npair * npair + 63) / 64 * 64 + npair * n;
+    const size_t lds3 = 3 * (size_t)n * JLD * sizeof(cplx<double>);
+    auto kern = items <= 128 ? k_heev_jacobi32<128> : items <= 192 ? k_heev_jacobi32<192>
+              : items <= 512 ? k_heev_jacobi32<512> : k_heev_jacobi32<768>;
+    const int nt = items <= 128 ? 128 : items <= 192 ? 192 : items <= 512 ? 512 : 768;
+    hipLaunchKernelGGL(kern, dim3(nbatch), dim3(nt), lds3, c->stream, A, lda, stride, n, d_w, nvec, d_info);
+    return hip_check(c, hipGetLastError(), "k_heev_jacobi32");
+  }
   const size_t lds = 2 * (size_t)n * n * sizeof(cplx<double>);
   hipLaunchKernelGGL(k_heev_jacobi, dim3(nbatch), dim3(SM_NT), lds, c->stream, A, lda, stride, n, d_w, nvec, d_info);
   return hip_check(c, hipGetLastError(), "k_heev_jacobi");
