@@ -104,11 +104,12 @@ enum {
                                    1024 threads (whole-box kernel), 256 (register-line kernel,
                                    which takes 256 or 512) */
   PW_TUNE_EIG_SYNC = 14,        /* the device tridiagonal reduction's cross-workgroup exchanges:
-                                   3 (default) by order: 2 up to n = 640, else 1;
+                                   3 (default) the same as 2;
                                    2 one exchange per column (the owner of the next
                                    column publishes it with its p segments and every
-                                   workgroup forms the next reflector itself), device-coherent
-                                   atomic accesses; 1 two exchanges per column (the owner
+                                   workgroup forms the next reflector itself), each value
+                                   its own arrival flag (n = 480: 2.2 ms,
+                                   n = 960: 6.3 ms); 1 two exchanges per column (the owner
                                    publishes the next reflector), device-coherent atomic
                                    accesses, each producer waiting for its stores before the
                                    flag (n = 480: 10.8 ms, n = 960: 21.4 ms); 0 two exchanges

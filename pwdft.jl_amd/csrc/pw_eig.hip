@@ -25,10 +25,9 @@
 //
 // Only the upper triangle of A is read, as Julia's Hermitian(A) does.  Cross-workgroup
 // waits are bounded: a wait that exceeds its spin limit sets a status word, every other
-// wait then ends at once, and the host reports the failure.  A step costs ~7.4 us at
-// n = 480 with 64 workgroups and one exchange (17 us with 26 workgroups and two): the round
-// trips to device-coherent memory on its critical path bound this one-dimensional
-// distribution.
+// wait then ends at once, and the host reports the failure.  A step costs ~4.7 us at
+// n = 480 with 64 workgroups and one exchange: the round trip to device-coherent memory and
+// the chain of sums on its critical path bound this one-dimensional distribution.
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
@@ -44,9 +43,24 @@ constexpr int HT_NT = 256;                 // threads per workgroup (4 wavefront
 constexpr long HT_SPIN = 1L << 22;         // spin limit of one cross-workgroup wait
 constexpr size_t HT_LDS = 160 * 1024 - 256;  // LDS bytes per workgroup, less room for the static shared state
 
+// Sum over the wavefront (all lanes active; every lane gets it): row shifts and row broadcasts
+// of the data-parallel primitives, ~20 cycles a level where a shuffle through LDS takes ~130,
+// six levels deep on every critical path below.
+template <int CTRL, int ROWS>
+__device__ inline double dpp_add(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+  return v + __hiloint2double(hi, lo);
+}
 __device__ inline double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v = dpp_add<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8: lane 15 of each row of 16 holds the row's sum
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);   // row_bcast 15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);   // row_bcast 31 into rows 2 and 3: lane 63 holds the sum
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
 }
 
 // Thread 0: wait until *ctr >= target; false once the status word is set or the spin limit
@@ -349,26 +363,78 @@ __device__ void hetrd_reflector_ip(cplx<double>* col, int i, int n, double* red,
 // step i's update; after the gather every workgroup applies step i's rank-2 update to that
 // one column and forms v_{i+1} itself -- the same data and the same arithmetic in every
 // workgroup, so the same bits -- instead of waiting for the owner to publish the reflector.
-// v_0 comes from column 0 of A, which every workgroup reads.  Workgroup 0 writes V, tau, d
-// and e for the eigenvector back-transform and ZSTEDC.
-// pg: 2 x n published p, sp: 2 x P x 2 partial sums, cg: 2 x n published next column (all by
-// step parity); sync[1]: arrivals.
-template <bool LIGHT>
+// v_0 comes from column 0 of A, which every workgroup reads.  The owner of the last column
+// writes V, tau, d and e for the eigenvector back-transform and the tridiagonal solvers.
+//
+// What bounds it is the latency of one step: the exchange, then a chain of two short sums
+// and a square root.  The exchange has no counter: a slot holds HX_EMPTY until its value
+// arrives and the reader polls the value itself, which leaves one store and one load to
+// device-coherent memory on the path, where waiting for the stores, counting the arrivals on
+// one address, polling the counter and only then loading the values took four round trips
+// (7.4 us a column at n = 480 on 64 workgroups, now 4.7; 3.8 at n = 160, 6.6 at n = 960).
+// The rank-2 update of step i - 1 goes in the pass
+// that forms p for step i, one reading of the owned columns instead of two.
+//
+// Four buffers by step: after the gather of step i every workgroup that gathered step i - 1
+// has published step i, so nobody reads that step's slots any more and their next owners
+// (the writers of step i + 3) empty them; the stores are waited for before step i + 2 is
+// published, and nobody reads step i + 3 before having gathered step i + 2 from the same
+// workgroups.  A workgroup leaves after its last column's p segment.
+// pg, cg: HX_BUF x n published p and next column, filled with HX_EMPTY before the launch.
+constexpr int HX_BUF = 4;
+constexpr long long HX_EMPTY = -1;   // bits of a NaN that arithmetic does not make
+
+__device__ inline void hx_store(cplx<double>* p, cplx<double> v) {
+  // a NaN of the caller's with the bits of an empty slot goes out as another NaN
+  long long x = __double_as_longlong(v.x), y = __double_as_longlong(v.y);
+  if (x == HX_EMPTY) x = 0x7ff8000000000000LL;
+  if (y == HX_EMPTY) y = 0x7ff8000000000000LL;
+  long long* q = reinterpret_cast<long long*>(p);
+  __hip_atomic_store(q, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void hx_clear(cplx<double>* p) {
+  long long* q = reinterpret_cast<long long*>(p);
+  __hip_atomic_store(q, HX_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(q + 1, HX_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// True when both parts have arrived.
+__device__ inline bool hx_load(const cplx<double>* p, cplx<double>* v) {
+  const long long* q = reinterpret_cast<const long long*>(p);
+  const long long x = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const long long y = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  *v = mk(__longlong_as_double(x), __longlong_as_double(y));
+  return x != HX_EMPTY && y != HX_EMPTY;
+}
+
+// Empties the exchange slots (count 32-bit words) and clears the status words.
+__global__ void k_hetrd_init(unsigned* slots, long count, unsigned* sync, int nsync) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < count) slots[t] = 0xffffffffu;
+  if (t < nsync) sync[t] = 0u;
+}
+
+// KR: rows of a gathered vector per thread, n <= KR * HT_NT.
+template <int KR>
 __global__ void __launch_bounds__(HT_NT) k_hetrd_dist1(const cplx<double>* __restrict__ A, long lda, int n,
                                                        int ncl_max, cplx<double>* __restrict__ V, long ldv,
                                                        cplx<double>* __restrict__ tau, double* __restrict__ dd,
-                                                       double* __restrict__ ee, cplx<double>* pg, double* sp,
-                                                       cplx<double>* cg, unsigned* sync, int* status) {
+                                                       double* __restrict__ ee, cplx<double>* pg,
+                                                       cplx<double>* cg, int* status) {
+  constexpr int NW = HT_NT / 64;
   extern __shared__ char smem_raw[];
   const int P = gridDim.x, w = blockIdx.x, tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   cplx<double>* Acol = reinterpret_cast<cplx<double>*>(smem_raw);
   cplx<double>* vb = Acol + (size_t)ncl_max * n;   // v_i
-  cplx<double>* wb = vb + n;                        // w_i
-  cplx<double>* vn = wb + n;                        // column i + 1, then v_{i+1}
-  double* red = reinterpret_cast<double*>(vn + n);
+  cplx<double>* vo = vb + n;                        // v_{i-1}, then v_{i+1}
+  cplx<double>* wb = vo + n;                        // w_{i-1}, then w_i
+  double* red = reinterpret_cast<double*>(wb + n);  // 2 NW
   __shared__ HetrdShared sh;
+  __shared__ double rn[NW];
+  __shared__ cplx<double> head[3];                  // p[i+1], p[i+2], column i + 1 at row i + 2
   const int ncl = w < n ? (n - 1 - w) / P + 1 : 0;
+  const bool writer = (n - 1) % P == w;
 
   for (long t = tid; t < (long)ncl * n; t += HT_NT) {
     const int lc = (int)(t / n), r = (int)(t % n);
@@ -384,117 +450,181 @@ __global__ void __launch_bounds__(HT_NT) k_hetrd_dist1(const cplx<double>* __res
     }
     Acol[(long)lc * n + r] = a;
   }
-  // column 0 of Hermitian(A) below the diagonal (conjugated row 0 of the upper triangle)
+  // column 0 of Hermitian(A) below the diagonal (conjugated row 0 of the upper triangle);
+  // no update is due before step 0
   for (int r = 1 + tid; r < n; r += HT_NT) {
     const cplx<double> u = A[(long)r * lda];
-    vn[r] = mk(u.x, -u.y);
+    vb[r] = mk(u.x, -u.y);
+    vo[r] = mk(0.0, 0.0);
+    wb[r] = mk(0.0, 0.0);
   }
+  if (tid == 0) sh.ok = 1;
   __syncthreads();
-  hetrd_reflector_ip(vn, 0, n, red, &sh);
-  if (w == 0) {
-    for (int r = 1 + tid; r < n; r += HT_NT) V[r] = vn[r];
+  hetrd_reflector_ip(vb, 0, n, red, &sh);
+  cplx<double> taui = mk(sh.tr, sh.ti);
+  if (writer) {
+    for (int r = 1 + tid; r < n; r += HT_NT) V[r] = vb[r];
     if (tid == 0) {
-      tau[0] = mk(sh.tr, sh.ti);
+      tau[0] = taui;
       ee[0] = sh.beta;
       dd[0] = A[0].x;
     }
   }
-  {
-    cplx<double>* t = vb;
-    vb = vn;
-    vn = t;
-  }
 
   for (int i = 0; i <= n - 2; ++i) {
-    const int par = i & 1;
-    const cplx<double> taui = mk(sh.tr, sh.ti);
-    // p_j = tau A22[:, j]^H v for the owned columns j > i; the owner of column i + 1
-    // publishes it as well
+    cplx<double>* pgi = pg + (long)(i % HX_BUF) * n;
+    cplx<double>* cgi = cg + (long)(i % HX_BUF) * n;
+    // the owned columns j > i, two at a time per wavefront: step i - 1's update, then
+    // p_j = tau A22[:, j]^H v; the owner of column i + 1 publishes it as well
     const int lc0 = (i + 1 <= w) ? 0 : (i + 1 - w + P - 1) / P;
-    double spr = 0.0, spi = 0.0;
-    for (int lc = lc0 + wave; lc < ncl; lc += HT_NT / 64) {
-      const int j = w + lc * P;
-      const cplx<double>* col = Acol + (long)lc * n;
-      double ar = 0.0, ai = 0.0;
+    for (int lc = lc0 + wave; lc < ncl; lc += 2 * NW) {
+      const int l2 = lc + NW < ncl ? lc + NW : lc;
+      const int ja = w + lc * P, jb = w + l2 * P;
+      cplx<double>* ca = Acol + (long)lc * n;
+      cplx<double>* cb = Acol + (long)l2 * n;
+      const cplx<double> wa = wb[ja], va = vo[ja], wc = wb[jb], vc = vo[jb];
+      const bool pub = ja == i + 1;
+      double ar = 0.0, ai = 0.0, br = 0.0, bi = 0.0;
       for (int r = i + 1 + lane; r < n; r += 64) {
-        const cplx<double> a = col[r], v = vb[r];
+        const cplx<double> v0 = vo[r], w0 = wb[r], v = vb[r];
+        const cplx<double> a = ca[r] - (cmulc(v0, wa) + cmulc(w0, va));
+        const cplx<double> b = cb[r] - (cmulc(v0, wc) + cmulc(w0, vc));
+        if (pub) hx_store(cgi + r, a);
+        ca[r] = a;
+        cb[r] = b;   // (the same column again where the second one is missing)
         ar += a.x * v.x + a.y * v.y;
         ai += a.x * v.y - a.y * v.x;
+        br += b.x * v.x + b.y * v.y;
+        bi += b.x * v.y - b.y * v.x;
       }
       ar = wave_sum(ar);
       ai = wave_sum(ai);
-      const cplx<double> p = cmul(taui, mk(ar, ai));
+      br = wave_sum(br);
+      bi = wave_sum(bi);
       if (lane == 0) {
-        xstore<LIGHT>(pg + (long)par * n + j, p);
-        const cplx<double> v = vb[j];
-        spr += p.x * v.x + p.y * v.y;
-        spi += p.x * v.y - p.y * v.x;
+        hx_store(pgi + ja, cmul(taui, mk(ar, ai)));
+        if (l2 != lc) hx_store(pgi + jb, cmul(taui, mk(br, bi)));
       }
     }
-    if (i + 1 <= n - 2 && (i + 1) % P == w) {
-      const cplx<double>* col = Acol + (long)((i + 1) / P) * n;
-      for (int r = i + 1 + tid; r < n; r += HT_NT) xstore<LIGHT>(cg + (long)par * n + r, col[r]);
-    }
-    {
-      double* red2 = red + HT_NT / 64;
-      __syncthreads();
-      if (lane == 0) {
-        red[wave] = spr;
-        red2[wave] = spi;
+    if (!writer && w + (ncl - 1) * P < i + 2) return;   // no column left
+
+    // gather: rows r = i + 1 + tid + k HT_NT of p and of column i + 1
+    cplx<double> p[KR], c[KR];
+    long spins = 0;
+    while (true) {
+      bool all = true;
+#pragma unroll
+      for (int k = 0; k < KR; ++k) {
+        if (i + 1 + k * HT_NT >= n) break;
+        const int r = min(i + 1 + tid + k * HT_NT, n - 1);
+        all &= hx_load(cgi + r, &c[k]);
+        all &= hx_load(pgi + r, &p[k]);
       }
-      __syncthreads();
-      if (tid == 0) {
-        double a = 0.0, b = 0.0;
-        for (int q = 0; q < HT_NT / 64; ++q) {
-          a += red[q];
-          b += red2[q];
-        }
-        xstore<LIGHT>(sp + ((long)par * P + w) * 2 + 0, a);
-        xstore<LIGHT>(sp + ((long)par * P + w) * 2 + 1, b);
+      if (all) break;
+      if ((++spins & 255) == 0 &&
+          (spins > HT_SPIN || __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+        __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sh.ok = 0;
+        break;
       }
     }
-    xpublish<LIGHT>();
-    __syncthreads();
-    if (tid == 0) __hip_atomic_fetch_add(&sync[1], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (tid == 0) sh.ok = wait_geq(&sync[1], (unsigned)P * (unsigned)(i + 1), status) ? 1 : 0;
+    // s = sum conj(p_r) v_r
+    double sr = 0.0, si = 0.0;
+#pragma unroll
+    for (int k = 0; k < KR; ++k) {
+      const int r = i + 1 + tid + k * HT_NT;
+      if (r >= n) break;
+      const cplx<double> v = vb[r];
+      sr += p[k].x * v.x + p[k].y * v.y;
+      si += p[k].x * v.y - p[k].y * v.x;
+    }
+    sr = wave_sum(sr);
+    si = wave_sum(si);
+    if (lane == 0) {
+      red[2 * wave] = sr;
+      red[2 * wave + 1] = si;
+    }
+    if (tid == 0) head[0] = p[0];
+    if (tid == 1) {
+      head[1] = p[0];
+      head[2] = c[0];
+    }
+    __builtin_amdgcn_s_waitcnt(0);   // the slots emptied in the step before
     __syncthreads();
     if (!sh.ok) return;
-    xacquire<LIGHT>();
-    double sr = 0.0, si = 0.0;
-    for (int q = tid; q < P; q += HT_NT) {
-      sr += xload<LIGHT>(sp + ((long)par * P + q) * 2 + 0);
-      si += xload<LIGHT>(sp + ((long)par * P + q) * 2 + 1);
+    // empty the slots of step i - 1 for their next use
+    {
+      cplx<double>* pgn = pg + (long)((i + HX_BUF - 1) % HX_BUF) * n;
+      cplx<double>* cgn = cg + (long)((i + HX_BUF - 1) % HX_BUF) * n;
+      const int in = i + HX_BUF - 1;
+      for (int lc = tid; lc < ncl; lc += HT_NT)
+        if (w + lc * P > in) hx_clear(pgn + w + lc * P);
+      if ((in + 1) % P == w)
+        for (int r = in + 1 + tid; r < n; r += HT_NT) hx_clear(cgn + r);
     }
-    sr = block_sum(sr, red);
-    si = block_sum(si, red);
+    sr = si = 0.0;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+      sr += red[2 * q];
+      si += red[2 * q + 1];
+    }
     const cplx<double> alpha2 = cmul(mk(-0.5 * taui.x, -0.5 * taui.y), mk(sr, si));
-    for (int r = i + 1 + tid; r < n; r += HT_NT) wb[r] = xload<LIGHT>(pg + (long)par * n + r) + cmul(alpha2, vb[r]);
-    const bool more = i + 1 <= n - 2;
-    if (more)
-      for (int r = i + 1 + tid; r < n; r += HT_NT) vn[r] = xload<LIGHT>(cg + (long)par * n + r);
+    // w_i, and step i's update of column i + 1 (v_i[i + 1] = 1)
+    const cplx<double> w1 = head[0] + alpha2;
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < KR; ++k) {
+      const int r = i + 1 + tid + k * HT_NT;
+      if (r >= n) break;
+      const cplx<double> v = vb[r];
+      const cplx<double> wr = p[k] + cmul(alpha2, v);
+      wb[r] = wr;
+      c[k] = c[k] - (cmulc(v, w1) + wr);
+      if (r >= i + 3) s += c[k].x * c[k].x + c[k].y * c[k].y;
+    }
+    if (writer && tid == 0) dd[i + 1] = c[0].x;
+    if (i == n - 2) return;
+    // v_{i+1}: ZLARFG on (alpha = row i + 2, the rows below it)
+    s = wave_sum(s);
+    if (lane == 0) rn[wave] = s;
+    const cplx<double> v2 = vb[i + 2];
+    const cplx<double> alpha = head[2] - (cmulc(v2, w1) + (head[1] + cmul(alpha2, v2)));
     __syncthreads();
-    // step i's update of the owned columns j > i, and of the next column in every workgroup
-    for (int lc = lc0; lc < ncl; ++lc) hetrd_update_col(Acol + (long)lc * n, w + lc * P, i, n, vb, wb);
-    if (more) {
-      hetrd_update_col(vn, i + 1, i, n, vb, wb);
-      __syncthreads();
-      const double d1 = vn[i + 1].x;
-      hetrd_reflector_ip(vn, i + 1, n, red, &sh);
-      if (w == 0) {
-        for (int r = i + 2 + tid; r < n; r += HT_NT) V[(long)(i + 1) * ldv + r] = vn[r];
-        if (tid == 0) {
-          tau[i + 1] = mk(sh.tr, sh.ti);
-          ee[i + 1] = sh.beta;
-          dd[i + 1] = d1;
-        }
-      }
-      cplx<double>* t = vb;
-      vb = vn;
-      vn = t;
+    s = 0.0;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) s += rn[q];
+    double beta;
+    cplx<double> scale;
+    if (s == 0.0 && alpha.y == 0.0) {
+      beta = alpha.x;
+      taui = mk(0.0, 0.0);
+      scale = mk(0.0, 0.0);
+    } else {
+      const double nrm = sqrt(alpha.x * alpha.x + alpha.y * alpha.y + s);
+      beta = alpha.x >= 0.0 ? -nrm : nrm;
+      taui = mk((beta - alpha.x) / beta, -alpha.y / beta);
+      const double ar = alpha.x - beta, ai = alpha.y;
+      const double den = ar * ar + ai * ai;
+      scale = mk(ar / den, -ai / den);
+    }
+#pragma unroll
+    for (int k = 0; k < KR; ++k) {
+      const int r = i + 1 + tid + k * HT_NT;
+      if (r >= n) break;
+      if (r < i + 2) continue;
+      const cplx<double> v = r == i + 2 ? mk(1.0, 0.0) : cmul(c[k], scale);
+      vo[r] = v;
+      if (writer) V[(long)(i + 1) * ldv + r] = v;
+    }
+    if (writer && tid == 0) {
+      tau[i + 1] = taui;
+      ee[i + 1] = beta;
     }
     __syncthreads();
+    cplx<double>* t = vb;
+    vb = vo;
+    vo = t;
   }
-  if ((n - 1) % P == w && tid == 0) dd[n - 1] = Acol[(long)((n - 1) / P) * n + (n - 1)].x;
 }
 
 // Back-transform by blocks of WY_NB reflectors (compact WY form, LAPACK ZLARFT / ZLARFB,
@@ -1194,7 +1324,7 @@ int heevd_dist(pw_ctx* c, void* rb, int n, cplx<double>* A, long lda, double* d_
   size_t lds = 0;
   const int P = hetrd_workgroups(n, &ncl, &lds, c->eig_min_wg);
   if (P <= 0) return set_error(c, PW_ERR_ARG, "heevd_dist: order " + std::to_string(n) + " out of range");
-  // workspace: V (n x n), T blocks, tau (n), pg (2n), cg (2n) complex; e (n), sp (4P)
+  // workspace: V (n x n), T blocks, tau (n), pg and cg (HX_BUF n each) complex; e (n), sp (4P)
   // doubles; sync (2) + status
   const size_t vbytes = (size_t)n * n * sizeof(cplx<double>);
   const int nblk = (n - 1 + WY_NB - 1) / WY_NB;
@@ -1202,7 +1332,7 @@ int heevd_dist(pw_ctx* c, void* rb, int n, cplx<double>* A, long lda, double* d_
   // (+ 2n doubles: the tridiagonal's diagonal and the computed eigenvalues of the device path;
   // + n nvec + nvec^2 complex: its copy of the vectors and their Gram matrix)
   const size_t lw = lowest && nvec > 0 ? ((size_t)n * nvec + (size_t)nvec * nvec) * sizeof(cplx<double>) : 0;
-  const size_t off_lw = (vbytes + tbytes + 5 * (size_t)n * sizeof(cplx<double>) +
+  const size_t off_lw = (vbytes + tbytes + (1 + 2 * HX_BUF) * (size_t)n * sizeof(cplx<double>) +
                          ((size_t)3 * n + 4 * P) * sizeof(double) + 64 + 255) & ~(size_t)255;
   const size_t need = off_lw + lw;
   int rc = ensure(c, &c->d_eig, &c->eig_bytes, need);
@@ -1212,8 +1342,8 @@ int heevd_dist(pw_ctx* c, void* rb, int n, cplx<double>* A, long lda, double* d_
   cplx<double>* Tb = V + (size_t)n * n;
   cplx<double>* tau = Tb + (size_t)nblk * WY_NB * WY_NB;
   cplx<double>* pg = tau + n;
-  cplx<double>* cg = pg + 2 * (size_t)n;
-  double* E = reinterpret_cast<double*>(cg + 2 * (size_t)n);
+  cplx<double>* cg = pg + HX_BUF * (size_t)n;
+  double* E = reinterpret_cast<double*>(cg + HX_BUF * (size_t)n);
   double* sp = E + n;
   double* Dt = sp + 4 * (size_t)P;
   double* Wt = Dt + n;
@@ -1221,9 +1351,11 @@ int heevd_dist(pw_ctx* c, void* rb, int n, cplx<double>* A, long lda, double* d_
   int* status = reinterpret_cast<int*>(sync + 2);
   cplx<double>* Zc = reinterpret_cast<cplx<double>*>(base + off_lw);
   cplx<double>* Gz = Zc + (size_t)n * (nvec > 0 ? nvec : 0);
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, c->stream, sync, 3, 0u);
+  const long slots = 2 * HX_BUF * (long)n * (long)(sizeof(cplx<double>) / sizeof(unsigned));
+  hipLaunchKernelGGL(k_hetrd_init, dim3((unsigned)((slots + 255) / 256)), dim3(256), 0, c->stream,
+                     reinterpret_cast<unsigned*>(pg), slots, sync, 3);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return hip_check(c, e, "k_fill_u32");
+  if (e != hipSuccess) return hip_check(c, e, "k_hetrd_init");
   const cplx<double>* Ac = A;
   long ldal = lda, ldv = n;
   int nn = n, nclm = ncl;
@@ -1231,13 +1363,14 @@ int heevd_dist(pw_ctx* c, void* rb, int n, cplx<double>* A, long lda, double* d_
   void* args[] = {(void*)&Ac, (void*)&ldal, (void*)&nn, (void*)&nclm, (void*)&V, (void*)&ldv, (void*)&tau,
                   (void*)&dd, (void*)&E, (void*)&pg, (void*)&sp, (void*)&sync, (void*)&status};
   void* args1[] = {(void*)&Ac, (void*)&ldal, (void*)&nn, (void*)&nclm, (void*)&V, (void*)&ldv, (void*)&tau,
-                   (void*)&dd, (void*)&E, (void*)&pg, (void*)&sp, (void*)&cg, (void*)&sync, (void*)&status};
-  // by order: the single-exchange form is faster up to n ~ 480 (n = 160: 2.33 -> 2.19 ms),
-  // slower at n = 960 (15.8 -> 16.6 ms), where each step's local work outweighs an exchange
-  const int mode = c->eig_light == 3 ? (n <= 640 ? 2 : 1) : c->eig_light;
-  if (mode == 2)
-    e = hipLaunchCooperativeKernel((const void*)k_hetrd_dist1<true>, dim3(P), dim3(HT_NT), args1, (unsigned)lds,
-                                   c->stream);
+                   (void*)&dd, (void*)&E, (void*)&pg, (void*)&cg, (void*)&status};
+  // one exchange per column at every order (eigenvalues of n = 160: 1.6 ms against 2.0 with
+  // two exchanges, n = 480: 4.6 against 5.6, n = 960: 10.4 against 12.6), on 64 workgroups:
+  // 96 to 256 are up to 5 % slower, the work they share being off the critical path
+  const int mode = c->eig_light == 3 ? 2 : c->eig_light;
+  if (mode == 2 && n <= 5 * HT_NT)
+    e = hipLaunchCooperativeKernel(n <= 3 * HT_NT ? (const void*)k_hetrd_dist1<3> : (const void*)k_hetrd_dist1<5>,
+                                   dim3(P), dim3(HT_NT), args1, (unsigned)lds, c->stream);
   else
     e = hipLaunchCooperativeKernel(mode ? (const void*)k_hetrd_dist<true> : (const void*)k_hetrd_dist<false>,
                                    dim3(P), dim3(HT_NT), args, (unsigned)lds, c->stream);

@@ -218,3 +218,36 @@ def test_heev_lowest_zstedc_mode(ctx):
     _check_pairs(A, w1, X1, ref, 320)
     ov = np.abs(np.einsum("ij,ij->j", X0.conj(), X1))
     assert np.abs(ov - 1).max() < 1e-9
+
+
+@pytest.mark.parametrize("n", [127, 255, 256, 257, 513, 768, 769, 1270])
+def test_heevd_gathered_rows(ctx, n):
+    """The reduction with one exchange per column where a gathered vector fills its 256
+    threads' rows exactly, by one short or one over, at both row counts per thread and near
+    the largest order: against numpy, with the bounds of the orders above."""
+    rng = np.random.default_rng(n)
+    A = _herm(rng, n, "random")
+    print(f"case heevd gathered rows n={n}", flush=True)
+    w, X = _eig(ctx, A)
+    ref = np.linalg.eigvalsh(A)
+    scale = max(1.0, np.abs(ref).max())
+    assert np.abs(w - ref).max() < 1e-12 * scale * max(1.0, np.sqrt(n) / 4)
+    assert np.abs(X.conj().T @ X - np.eye(n)).max() < 1e-12 * max(1.0, np.sqrt(n) / 4)
+    assert np.abs(A @ X - X * w).max() < 1e-12 * scale * max(1.0, np.sqrt(n) / 4)
+
+
+@pytest.mark.parametrize("n", [1, 4, 7, 9, 12, 15, 16, 17, 23, 24, 25, 31, 32, 33])
+@pytest.mark.parametrize("kind", ["random", "degenerate", "graded", "diagonal"])
+def test_heevd_small_orders(ctx, n, kind):
+    """The one-workgroup Jacobi eigensolver at odd and even orders, at both sides of its
+    workgroup widths and of order 32, where the form for larger orders takes over: against
+    numpy, with the bounds of the orders above."""
+    rng = np.random.default_rng(n * 37 + len(kind))
+    A = _herm(rng, n, kind)
+    print(f"case heevd small n={n} kind={kind}", flush=True)
+    w, X = _eig(ctx, A)
+    ref = np.linalg.eigvalsh(A)
+    scale = max(1.0, np.abs(ref).max())
+    assert np.abs(w - ref).max() < 1e-12 * scale
+    assert np.abs(X.conj().T @ X - np.eye(n)).max() < 1e-12
+    assert np.abs(A @ X - X * w).max() < 1e-12 * scale
