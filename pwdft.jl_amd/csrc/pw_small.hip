@@ -13,10 +13,9 @@
 //    confirm it); eigenvalues sorted ascending with their vectors.  Complex 2x2 step: the pair (p, q) with A_pq = |g| e^{i phi} is made
 //    real by diag(1, e^{-i phi}) and diagonalised by the classical rotation
 //    t = sign(tau) / (|tau| + sqrt(1 + tau^2)), tau = (A_qq - A_pp) / (2 |g|).
-//  - k_chol_inv_small: U = chol(Hermitian(A)).U by right-looking elimination, then U^-1 by
-//    back substitution over rows, the matrix held in registers (a 4 x 4 tile per thread) and
-//    one barrier per step; the strict lower triangle zeroed.  Status: 0, or the index
-//    (1-based) of the first non-positive pivot.
+//  - k_chol_inv_small: inv(chol(Hermitian(A)).U) by right-looking elimination of [A | I], the
+//    matrix held in registers and one barrier per step; the strict lower triangle zeroed.
+//    Status: 0, or the index (1-based) of the first non-positive pivot.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -418,37 +417,44 @@ __global__ void __launch_bounds__(NT) k_heev_jacobi32(cplx<double>* __restrict__
 
 // Matrix b of the stack: inv(chol(Hermitian(A)).U) in place, strict lower triangle zeroed;
 // info[b] (potrf) and info[nbatch + b] (trtri) as rocSOLVER would set them.
-// Thread (ti, tj) of a G x G grid (G = 16 or 32) holds the entries (ti + G a, tj + G b), a, b < 64 / G, in
-// registers from the load to the store.  Factorization (right-looking): at step k the holders
-// of row k publish it to an LDS row (two rows alternate), one barrier, then every thread
-// scales what it needs of row k by 1 / sqrt(A_kk) and updates its own trailing entries.
-// Inverse (X = U^-1, rows from the last): the holders of row i finish X_ij = (delta_ij -
-// S_ij) / U_ii and publish it, one barrier, then every thread adds U_ri X_ij to its sums S_rj
-// of the rows r < i (U's column i read from LDS, where U was stored after the factorization).
-// One barrier per step in both phases.
-template <int G>
-__global__ void __launch_bounds__(G * G) k_chol_inv_small(cplx<double>* __restrict__ A, long lda, long stride, int n,
-                                                           int* __restrict__ info, int nbatch) {
-  constexpr int E = SM_NMAX / G;   // entries per thread along each axis
-  extern __shared__ char smem_raw[];
-  cplx<double>* u = reinterpret_cast<cplx<double>*>(smem_raw);   // n x n: U after the factorization
+//
+// Right-looking elimination on [A | I]: the row operations that bring A to upper triangular
+// form turn I into L^-1, A = L D L^H, and inv(U) = L^-H D^-1/2.  A's part of row i is its
+// columns j >= i and L^-1's the columns j < i (its diagonal is 1), so both share one n x n
+// square, and one pass of n steps gives the inverse without U ever being stored.  Thread
+// (ti, tj) of a 16 x 16 grid holds the entries (ti + 16 a, tj + 16 b) in registers from the
+// load to the store; at step k the holders of row k publish it to an LDS row (two rows
+// alternate), one barrier, then every thread updates its entries of the rows i > k in the
+// columns j >= i and j <= k.  Both factors of a product are scaled by 1 / sqrt(A_kk), so
+// nothing overflows that U and its inverse can hold.
+//
+// What bounds it is the chain of a step (LDS row, reciprocal root, update).  Separate passes
+// for U and its inverse were 2 n steps; on 1024 threads, which one matrix above order 32
+// took, a step also cost ~1 us in instructions issued for entries that are finished
+// (a call with its
+// synchronisation, n = 40: 83 us, now 48; n = 24: 58 us, now 33; the kernel alone 4.6 us to
+// n = 16, 12.5 at n = 24).
+template <int E>   // entries per thread along each axis, n <= 16 E
+__global__ void __launch_bounds__(256) k_chol_inv_small(cplx<double>* __restrict__ A, long lda, long stride, int n,
+                                                       int* __restrict__ info, int nbatch) {
+  constexpr int G = 16;
   __shared__ cplx<double> rowbuf[2][SM_NMAX];
   __shared__ double rdiag[SM_NMAX];
-  static_assert((G == 16 || G == 32) && SM_NMAX == 64, "G x G grid, E x E entries per thread");
+  static_assert(G * E <= SM_NMAX, "row buffers");
   cplx<double>* M = A + (long)blockIdx.x * stride;
-  const int tid = threadIdx.x, ti = tid % G, tj = tid / G;
-  cplx<double> r[E][E];   // r[b][a]: entry (ti + G a, tj + G b)
+  const int tid = threadIdx.x, tj = tid % G, ti = tid / G;
+  cplx<double> r[E][E];   // r[a][b]: entry (ti + G a, tj + G b)
 #pragma unroll
-  for (int b = 0; b < E; ++b)
+  for (int a = 0; a < E; ++a)
 #pragma unroll
-    for (int a = 0; a < E; ++a) {
+    for (int b = 0; b < E; ++b) {
       const int i = ti + G * a, j = tj + G * b;
       cplx<double> v = mk(0.0, 0.0);
       if (j < n && i <= j) {
         v = M[(long)j * lda + i];
         if (i == j) v.y = 0.0;
       }
-      r[b][a] = v;
+      r[a][b] = v;
     }
   int bad = 0;
   for (int k = 0; k < n; ++k) {
@@ -458,124 +464,61 @@ __global__ void __launch_bounds__(G * G) k_chol_inv_small(cplx<double>* __restri
       for (int a = 0; a < E; ++a)
         if (a == ak) {
 #pragma unroll
-          for (int b = 0; b < E; ++b) {
-            const int j = tj + G * b;
-            if (j >= k && j < n) rowbuf[buf][j] = r[b][a];
-          }
+          for (int b = 0; b < E; ++b) rowbuf[buf][tj + G * b] = r[a][b];
         }
     }
     __syncthreads();
+    // the row reads are unconditional (every index is a valid LDS slot) so they issue together
     const double dkk = rowbuf[buf][k].x;
+    cplx<double> m[E], x[E];
+#pragma unroll
+    for (int a = 0; a < E; ++a) m[a] = rowbuf[buf][ti + G * a];
+#pragma unroll
+    for (int b = 0; b < E; ++b) x[b] = rowbuf[buf][tj + G * b];
     if (!(dkk > 0.0)) {   // the same value on every thread: a uniform exit
       bad = k + 1;
       break;
     }
-    // 1 / sqrt and sqrt from one reciprocal square root; the row reads are unconditional
-    // (every index < SM_NMAX is a valid LDS slot) so they issue together and wait once
-    const double rd = rsqrt(dkk), d = dkk * rd;
-    cplx<double> uki[E], ukj[E];
+    const double rd = rsqrt(dkk);
+    if (tid == 0) rdiag[k] = rd;
+#pragma unroll
+    for (int a = 0; a < E; ++a) m[a] = scal(rd, m[a]);
+#pragma unroll
+    for (int b = 0; b < E; ++b) x[b] = tj + G * b == k ? mk(rd, 0.0) : scal(rd, x[b]);
 #pragma unroll
     for (int a = 0; a < E; ++a) {
+      // tile rows wholly up to k are finished, tiles between k and the diagonal are zero:
+      // skipped on every thread alike
+      if (G * a + G - 1 <= k || G * a >= n) continue;
       const int i = ti + G * a;
-      const cplx<double> v = rowbuf[buf][i];
-      uki[a] = (i > k && i < n) ? scal(rd, v) : mk(0.0, 0.0);
-    }
 #pragma unroll
-    for (int b = 0; b < E; ++b) {
-      const int j = tj + G * b;
-      const cplx<double> v = rowbuf[buf][j];
-      ukj[b] = (j > k && j < n) ? scal(rd, v) : mk(0.0, 0.0);
-    }
-    // tile rows a and columns b wholly before k are finished: skipped on every thread alike
-#pragma unroll
-    for (int b = 0; b < E; ++b) {
-      if (G * b + G - 1 < k || G * b >= n) continue;
-#pragma unroll
-      for (int a = 0; a < E; ++a) {
-        if (G * a + G - 1 < k || G * a > G * b + G - 1) continue;
-        const int i = ti + G * a, j = tj + G * b;
-        if (j < n && i <= j) {
-          if (i == k) r[b][a] = j == k ? mk(d, 0.0) : scal(rd, r[b][a]);            // row k of U
-          else if (i > k) r[b][a] = r[b][a] - cmulc(ukj[b], uki[a]);               // A_ij -= conj(U_ki) U_kj
+      for (int b = 0; b < E; ++b) {
+        if (b < a && G * b > k) continue;
+        const int j = tj + G * b;
+        if (i > k && (j >= i || j <= k)) {   // -= conj(m_i) x_j
+          r[a][b].x = fma(-x[b].x, m[a].x, fma(-x[b].y, m[a].y, r[a][b].x));
+          r[a][b].y = fma(-x[b].y, m[a].x, fma(x[b].x, m[a].y, r[a][b].y));
         }
       }
     }
   }
   const int bb = blockIdx.x;
-  if (bad) {
-    if (tid == 0) {
-      info[bb] = bad;
-      info[nbatch + bb] = 0;
-    }
-    return;
-  }
-  // U into LDS (its columns feed the inverse), 1 / U_ii
-#pragma unroll
-  for (int b = 0; b < E; ++b)
-#pragma unroll
-    for (int a = 0; a < E; ++a) {
-      const int i = ti + G * a, j = tj + G * b;
-      if (j < n && i <= j) {
-        u[i + n * j] = r[b][a];
-        if (i == j) rdiag[i] = 1.0 / r[b][a].x;
-      }
-      r[b][a] = mk(0.0, 0.0);   // from here: the sums S, then X
-    }
-  __syncthreads();
-  for (int i = n - 1; i >= 0; --i) {
-    const int buf = i & 1, ai = i / G;
-    if (ti == i % G) {
-#pragma unroll
-      for (int a = 0; a < E; ++a)
-        if (a == ai) {
-#pragma unroll
-          for (int b = 0; b < E; ++b) {
-            const int j = tj + G * b;
-            if (j >= i && j < n) {
-              const cplx<double> x = scal(rdiag[i], mk((j == i ? 1.0 : 0.0) - r[b][a].x, -r[b][a].y));
-              r[b][a] = x;
-              rowbuf[buf][j] = x;
-            }
-          }
-        }
-    }
-    __syncthreads();
-    cplx<double> uri[E], xij[E];
-#pragma unroll
-    for (int a = 0; a < E; ++a) {
-      const int rr = ti + G * a;
-      const cplx<double> v = u[min(rr, n - 1) + n * i];   // unconditional (clamped) read
-      uri[a] = rr < i ? v : mk(0.0, 0.0);
-    }
-#pragma unroll
-    for (int b = 0; b < E; ++b) {
-      const int j = tj + G * b;
-      const cplx<double> v = rowbuf[buf][j];
-      xij[b] = (j >= i && j < n) ? v : mk(0.0, 0.0);
-    }
-#pragma unroll
-    for (int b = 0; b < E; ++b) {
-      if (G * b + G - 1 < i || G * b >= n) continue;
-#pragma unroll
-      for (int a = 0; a < E; ++a) {
-        if (G * a >= i) continue;
-        const int rr = ti + G * a, j = tj + G * b;
-        if (rr < i && j >= i && j < n) r[b][a] = r[b][a] + cmul(uri[a], xij[b]);
-      }
-    }
-  }
-  // X (upper triangle) and zeros below the diagonal
-#pragma unroll
-  for (int b = 0; b < E; ++b)
-#pragma unroll
-    for (int a = 0; a < E; ++a) {
-      const int i = ti + G * a, j = tj + G * b;
-      if (i < n && j < n) M[(long)j * lda + i] = i <= j ? cplx<double>(r[b][a]) : mk(0.0, 0.0);
-    }
   if (tid == 0) {
-    info[bb] = 0;
+    info[bb] = bad;
     info[nbatch + bb] = 0;
   }
+  if (bad) return;
+  __syncthreads();   // rdiag
+  // inv(U)_ji = conj(L^-1_ij) / sqrt(D_i), zeros below the diagonal
+#pragma unroll
+  for (int a = 0; a < E; ++a)
+#pragma unroll
+    for (int b = 0; b < E; ++b) {
+      const int i = ti + G * a, j = tj + G * b;
+      if (i >= n || j >= n) continue;
+      const double rd = rdiag[i];
+      M[(long)i * lda + j] = j < i ? mk(rd * r[a][b].x, -rd * r[a][b].y) : mk(j == i ? rd : 0.0, 0.0);
+    }
 }
 
 int heev_small_batch(pw_ctx* c, int n, int nbatch, cplx<double>* A, long lda, long stride, double* d_w, int nvec,
@@ -598,13 +541,9 @@ int heev_small_batch(pw_ctx* c, int n, int nbatch, cplx<double>* A, long lda, lo
 
 int chol_inv_small_batch(pw_ctx* c, int n, int nbatch, cplx<double>* A, long lda, long stride, int* d_info) {
   if (n < 1 || n > SM_NMAX || nbatch < 1) return set_error(c, PW_ERR_ARG, "chol_inv_small_batch: order out of range");
-  const size_t lds = (size_t)n * n * sizeof(cplx<double>);
-  // one matrix above order 32 (the recursive inverse's blocks): a 32 x 32 grid of 2 x 2 tiles,
-  // a quarter of the arithmetic per thread and step; stacks of small matrices keep 16 x 16
-  if (nbatch == 1 && n > 32)
-    hipLaunchKernelGGL(k_chol_inv_small<32>, dim3(1), dim3(1024), lds, c->stream, A, lda, stride, n, d_info, nbatch);
-  else
-    hipLaunchKernelGGL(k_chol_inv_small<16>, dim3(nbatch), dim3(256), lds, c->stream, A, lda, stride, n, d_info, nbatch);
+  auto kern = n <= 16 ? k_chol_inv_small<1> : n <= 32 ? k_chol_inv_small<2>
+            : n <= 48 ? k_chol_inv_small<3> : k_chol_inv_small<4>;
+  hipLaunchKernelGGL(kern, dim3(nbatch), dim3(256), 0, c->stream, A, lda, stride, n, d_info, nbatch);
   return hip_check(c, hipGetLastError(), "k_chol_inv_small");
 }
 
