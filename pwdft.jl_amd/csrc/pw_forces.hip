@@ -41,18 +41,22 @@ __global__ void k_delta(cplx<double>* __restrict__ d, int n, int g0) {
 
 // dE_Ps_loc/dtau_a = sum_G Re(-i G V_sp(G) exp(-i G.tau_a) conj(rho(G)))
 //                  = -sum_G G V_sp(G) (cos(G.tau) Im rho + sin(G.tau) Re rho).
-// One block per atom; the G = 0 term vanishes with G.
+// Block a nz + z: atom a's sum over the z-th of nz equal chunks of G, into part[a][z];
+// the G = 0 term vanishes with G.  One block per atom left all but natoms of the 256 compute
+// units idle through ng / FNT serial steps of a double-precision sincos (8 atoms, 20 Ha:
+// 108 us; split over the chip 6.7, and 3 for the sum of the parts).
 __global__ void __launch_bounds__(FNT) k_loc_tau(const cplx<double>* __restrict__ rhoG,
-                                                 const double* __restrict__ G, int ng,
+                                                 const double* __restrict__ G, int ng, int chunk,
                                                  const double* __restrict__ vg,
                                                  const double* __restrict__ tau,
-                                                 const int* __restrict__ species, double* __restrict__ dtau) {
+                                                 const int* __restrict__ species, int nz, double* __restrict__ part) {
   __shared__ double sh[FNT / 64];
-  const int a = blockIdx.x;
+  const int a = blockIdx.x / nz, z = blockIdx.x % nz;
   const double tx = tau[3 * a], ty = tau[3 * a + 1], tz = tau[3 * a + 2];
   const double* v = vg + (size_t)species[a] * ng;
+  const int g0 = z * chunk, g1 = min(ng, g0 + chunk);
   double fx = 0.0, fy = 0.0, fz = 0.0;
-  for (int g = threadIdx.x; g < ng; g += FNT) {
+  for (int g = g0 + threadIdx.x; g < g1; g += FNT) {
     const double gx = G[3 * g], gy = G[3 * g + 1], gz = G[3 * g + 2];
     double s, cs;
     sincos(gx * tx + gy * ty + gz * tz, &s, &cs);
@@ -66,10 +70,24 @@ __global__ void __launch_bounds__(FNT) k_loc_tau(const cplx<double>* __restrict_
   fy = block_sum(fy, sh);
   fz = block_sum(fz, sh);
   if (threadIdx.x == 0) {
-    dtau[3 * a] = fx;
-    dtau[3 * a + 1] = fy;
-    dtau[3 * a + 2] = fz;
+    double* o = part + 3 * (size_t)blockIdx.x;
+    o[0] = fx;
+    o[1] = fy;
+    o[2] = fz;
   }
+}
+
+// dtau[a][x] = the sum of atom a's nz partial sums in a fixed order; one wavefront per atom.
+__global__ void __launch_bounds__(64) k_loc_tau_sum(const double* __restrict__ part, int nz,
+                                                    double* __restrict__ dtau) {
+  const int a = blockIdx.x, lane = threadIdx.x;
+  const double* p = part + 3 * (size_t)a * nz;
+  double f[3] = {0.0, 0.0, 0.0};
+  for (int z = lane; z < nz; z += 64)
+    for (int x = 0; x < 3; ++x) f[x] += p[3 * z + x];
+  for (int o = 32; o > 0; o >>= 1)
+    for (int x = 0; x < 3; ++x) f[x] += __shfl_xor(f[x], o, 64);
+  if (lane < 3) dtau[3 * a + lane] = lane == 0 ? f[0] : lane == 1 ? f[1] : f[2];
 }
 
 // dE_Ps_loc/dV_sp(G) = Re(S_sp(G) conj(rho(G))), S_sp(G) = sum_{a in sp} exp(-i G.tau_a);
@@ -104,25 +122,27 @@ __global__ void __launch_bounds__(FNT) k_loc_vg(const cplx<double>* __restrict__
   if (threadIdx.x == 0) part[blockIdx.x] = e;
 }
 
-// out[:, alpha * nbeta + j] = (G+k)_alpha * beta[:, j]  (the i is applied in k_nloc_reduce)
-__global__ void k_gbeta3(const cplx<double>* __restrict__ beta, const double* __restrict__ gk, int ngw,
+// out[:, q * nbeta + j] = beta[:, j] for q = 0, (G+k)_{q-1} * beta[:, j] for q = 1..3 (the i is
+// applied in k_nloc_reduce): one operand, so that the projections and their three derivatives
+// are one product in place of two (Si8, 20 Ha, per k-point: products, their reductions and
+// this kernel 39 us, now 25).
+__global__ void k_gbeta4(const cplx<double>* __restrict__ beta, const double* __restrict__ gk, int ngw,
                          int nbeta, cplx<double>* __restrict__ out) {
   const long per = (long)ngw * nbeta;
-  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < 3 * per; t += (long)gridDim.x * blockDim.x) {
-    const int alpha = (int)(t / per);
-    const long r = t - alpha * per;
+  for (long r = blockIdx.x * (long)blockDim.x + threadIdx.x; r < per; r += (long)gridDim.x * blockDim.x) {
     const int g = (int)(r % ngw);
-    out[t] = scal(gk[3 * g + alpha], beta[r]);
+    const cplx<double> v = beta[r];
+    out[r] = v;
+    for (int x = 0; x < 3; ++x) out[r + (x + 1) * per] = scal(gk[3 * g + x], v);
   }
 }
 
 // One block per projector j: DB_j = sum_i D[i, j] B[i, st] over the non-zeros of column j,
 //   part[4j]       = sum_st w_st Re(conj(DB_j) B[j, st])               (E_Ps_nloc)
-//   part[4j+1+al]  = sum_st w_st Im(conj(DB_j) X[al*nbeta + j, st])   (half the force)
-// with B = beta^H psi (nbeta x nb) and X = ((G+k)_al beta)^H psi (3 nbeta x nb), so that
-// Im(conj(DB) X) = Re(conj(DB) <i (G+k) beta|psi>).
-__global__ void __launch_bounds__(FNT) k_nloc_reduce(const cplx<double>* __restrict__ B,
-                                                     const cplx<double>* __restrict__ X, int nbeta, int nb,
+//   part[4j+1+al]  = sum_st w_st Im(conj(DB_j) B[(1+al)*nbeta + j, st])   (half the force)
+// with B = [beta, (G+k)_al beta]^H psi (4 nbeta x nb), so that
+// Im(conj(DB_j) B[(1+al)*nbeta + j]) = Re(conj(DB_j) <i (G+k)_al beta_j|psi>).
+__global__ void __launch_bounds__(FNT) k_nloc_reduce(const cplx<double>* __restrict__ B, int nbeta, int nb,
                                                      const int* __restrict__ cptr, const int* __restrict__ rows,
                                                      const double* __restrict__ vals,
                                                      const double* __restrict__ w, double* __restrict__ part) {
@@ -131,14 +151,13 @@ __global__ void __launch_bounds__(FNT) k_nloc_reduce(const cplx<double>* __restr
   const int q0 = cptr[j], q1 = cptr[j + 1];
   double e = 0.0, f0 = 0.0, f1 = 0.0, f2 = 0.0;
   for (int st = threadIdx.x; st < nb; st += FNT) {
-    const cplx<double>* Bs = B + (size_t)nbeta * st;
+    const cplx<double>* Bs = B + (size_t)4 * nbeta * st;
     cplx<double> db = mk(0.0, 0.0);
     for (int q = q0; q < q1; ++q) db = db + scal(vals[q], Bs[rows[q]]);
     const double ws = w[st];
     const cplx<double> b = Bs[j];
     e += ws * (db.x * b.x + db.y * b.y);
-    const cplx<double>* Xs = X + (size_t)3 * nbeta * st + j;
-    const cplx<double> x0 = Xs[0], x1 = Xs[nbeta], x2 = Xs[2 * nbeta];
+    const cplx<double> x0 = Bs[j + nbeta], x1 = Bs[j + 2 * nbeta], x2 = Bs[j + 3 * nbeta];
     f0 += ws * (db.x * x0.y - db.y * x0.x);
     f1 += ws * (db.x * x1.y - db.y * x1.x);
     f2 += ws * (db.x * x2.y - db.y * x2.x);
@@ -254,13 +273,19 @@ static int loc_grad(pw_ctx* c, const double* rho, double* E, double* dE_dvg, dou
   cplx<double>* delta = reinterpret_cast<cplx<double>*>(reinterpret_cast<char*>(c->d_fgrid) + gbytes);
   cplx<double>* rhoG = delta + ng;
   const int nblk = (ng + FNT - 1) / FNT;
-  // partial sums: dE/dvg (ng * nsp), E partials (nblk), dE/dtau (3 natoms)
+  // dE/dtau: four blocks per compute unit between the atoms, at least one step of FNT each
+  const int nz0 = std::max(1, std::min(nblk, (4 * 256 + c->natoms - 1) / c->natoms));
+  const int chunk = ((ng + nz0 - 1) / nz0 + FNT - 1) / FNT * FNT;
+  const int nz = (ng + chunk - 1) / chunk;
+  // partial sums: dE/dvg (ng * nsp), E partials (nblk), dE/dtau (3 natoms) and its nz parts
   const size_t nv = (size_t)ng * c->nsp_loc;
-  rc = ensure(c, &c->d_fpart, &c->fpart_bytes, (nv + nblk + 3 * (size_t)c->natoms) * sizeof(double));
+  rc = ensure(c, &c->d_fpart, &c->fpart_bytes,
+              (nv + nblk + 3 * (size_t)c->natoms * (1 + (size_t)nz)) * sizeof(double));
   if (rc) return rc;
   double* dvg = reinterpret_cast<double*>(c->d_fpart);
   double* epart = dvg + nv;
   double* dtau = epart + nblk;
+  double* tpart = dtau + 3 * (size_t)c->natoms;
   const double s = 1.0 / (double)c->N;
   const int gb = (int)std::min<long>((c->N + 255) / 256, 4096);
   hipError_t e = hipSuccess;
@@ -277,9 +302,12 @@ static int loc_grad(pw_ctx* c, const double* rho, double* E, double* dE_dvg, dou
   rc = vloc_apply_k(c, k, rhoN, 1, delta, ng, rhoG, ng);
   if (rc) return rc;
   if (dE_dtau) {
-    hipLaunchKernelGGL(k_loc_tau, dim3(c->natoms), dim3(FNT), 0, c->stream, rhoG, k.d_gk, ng, c->d_vg, c->d_tau,
-                       c->d_species, dtau);
+    hipLaunchKernelGGL(k_loc_tau, dim3((unsigned)nz * c->natoms), dim3(FNT), 0, c->stream, rhoG, k.d_gk, ng, chunk,
+                       c->d_vg, c->d_tau, c->d_species, nz, tpart);
     rc = hip_check(c, hipGetLastError(), "k_loc_tau");
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_loc_tau_sum, dim3(c->natoms), dim3(64), 0, c->stream, tpart, nz, dtau);
+    rc = hip_check(c, hipGetLastError(), "k_loc_tau_sum");
     if (rc) return rc;
     e = hipMemcpyAsync(dE_dtau, dtau, 3 * (size_t)c->natoms * sizeof(double), hipMemcpyDeviceToHost, c->stream);
     if (e != hipSuccess) return hip_check(c, e, "dE/dtau download");
@@ -320,33 +348,30 @@ static int nloc_forces(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long 
   const int nbeta = k.nbeta;
   int rc = ensure_dcsr(c);
   if (rc) return rc;
-  rc = ensure(c, &c->d_fbeta, &c->fbeta_bytes, 3 * (size_t)k.ngw * nbeta * sizeof(cplx<double>));
+  rc = ensure(c, &c->d_fbeta, &c->fbeta_bytes, 4 * (size_t)k.ngw * nbeta * sizeof(cplx<double>));
   if (rc) return rc;
-  const size_t mB = (size_t)nbeta * nb, mX = 3 * mB;
-  rc = ensure(c, &c->d_fmat, &c->fmat_bytes, (mB + mX) * sizeof(cplx<double>) + (size_t)nb * sizeof(double));
+  const size_t mB = 4 * (size_t)nbeta * nb;
+  rc = ensure(c, &c->d_fmat, &c->fmat_bytes, mB * sizeof(cplx<double>) + (size_t)nb * sizeof(double));
   if (rc) return rc;
   rc = ensure(c, &c->d_fpart, &c->fpart_bytes, 4 * (size_t)nbeta * sizeof(double));
   if (rc) return rc;
   cplx<double>* gb = reinterpret_cast<cplx<double>*>(c->d_fbeta);
   cplx<double>* Bm = reinterpret_cast<cplx<double>*>(c->d_fmat);
-  cplx<double>* Xm = Bm + mB;
-  double* dw = reinterpret_cast<double*>(Xm + mX);
+  double* dw = reinterpret_cast<double*>(Bm + mB);
   double* part = reinterpret_cast<double*>(c->d_fpart);
   const cplx<double>* beta = reinterpret_cast<const cplx<double>*>(k.d_beta64);
   hipError_t e = hipMemcpyAsync(dw, w, nb * sizeof(double), hipMemcpyHostToDevice, c->stream);
   if (e != hipSuccess) return hip_check(c, e, "band weights upload");
-  const long tot = 3L * k.ngw * nbeta;
-  hipLaunchKernelGGL(k_gbeta3, dim3((int)std::min<long>((tot + 255) / 256, 8192)), dim3(256), 0, c->stream, beta,
+  const long tot = (long)k.ngw * nbeta;
+  hipLaunchKernelGGL(k_gbeta4, dim3((int)std::min<long>((tot + 255) / 256, 8192)), dim3(256), 0, c->stream, beta,
                      k.d_gk, k.ngw, nbeta, gb);
-  rc = hip_check(c, hipGetLastError(), "k_gbeta3");
+  rc = hip_check(c, hipGetLastError(), "k_gbeta4");
   if (rc) return rc;
   const cplx<double> one = mk(1.0, 0.0), zero = mk(0.0, 0.0);
-  rc = zgemm(c, 1, nbeta, nb, k.ngw, one, beta, k.ngw, psi, ldpsi, zero, Bm, nbeta, 0);
+  rc = zgemm(c, 1, 4 * nbeta, nb, k.ngw, one, gb, k.ngw, psi, ldpsi, zero, Bm, 4 * nbeta, 0);
   if (rc) return rc;
-  rc = zgemm(c, 1, 3 * nbeta, nb, k.ngw, one, gb, k.ngw, psi, ldpsi, zero, Xm, 3 * nbeta, 0);
-  if (rc) return rc;
-  hipLaunchKernelGGL(k_nloc_reduce, dim3(nbeta), dim3(FNT), 0, c->stream, Bm, Xm, nbeta, nb, c->d_dcol_ptr,
-                     c->d_drow, c->d_dval, dw, part);
+  hipLaunchKernelGGL(k_nloc_reduce, dim3(nbeta), dim3(FNT), 0, c->stream, Bm, nbeta, nb, c->d_dcol_ptr, c->d_drow,
+                     c->d_dval, dw, part);
   rc = hip_check(c, hipGetLastError(), "k_nloc_reduce");
   if (rc) return rc;
   std::vector<double> hp(4 * (size_t)nbeta);

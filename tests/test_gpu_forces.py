@@ -91,6 +91,25 @@ def test_E_Ps_loc_grad_vs_oracle(si8):
     assert abs(gsh[5, 0] - 2.0 * dvg[pw.idx_g2shells == 5, 0].sum()) < 1e-12
 
 
+@pytest.mark.parametrize("natoms,ecut", [(1, 3.0), (3, 9.0), (33, 9.0), (200, 12.0)])
+def test_forces_Ps_loc_split_vs_oracle(natoms, ecut):
+    """The local force's sum over G split over blocks: one block per atom's whole sphere, a
+    block per 256 vectors with a partial last one, and several steps per block."""
+    import pwdft_hip as ph
+    from oracle.forces import calc_forces_Ps_loc
+    L = ph.gen_lattice_sc(A_SI)
+    frac = np.random.default_rng(natoms).uniform(size=(natoms, 3))
+    atoms = ph.Atoms(["Si"] * natoms, frac, L)
+    H = ph.Hamiltonian(atoms, ["Si-q4.lda.gth"], ecut, meshk=(1, 1, 1), use_symmetry=False)
+    oH = oracle_ham(["Si"] * natoms, frac, L, "Si-q4.lda.gth", ecut, kpoints=(H.pw.k, H.pw.wk),
+                    Nstates=H.electrons.Nstates)
+    rho = np.random.default_rng(natoms + 1).uniform(0.1, 1.0, size=H.pw.Npoints)
+    print(f"case forces_Ps_loc natoms={natoms} ecut={ecut}", flush=True)
+    F = ph.calc_forces_Ps_loc(H, rho)
+    Fo = calc_forces_Ps_loc(oH, rho)
+    assert np.abs(F - Fo).max() < 1e-11 * max(1.0, np.abs(Fo).max()), np.abs(F - Fo).max()
+
+
 def test_forces_Ps_nloc_vs_oracle(si8):
     import pwdft_hip as ph
     from oracle.energy import calc_E_Ps_nloc

@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(16, 16, 4), (15, 17, 3), (17, 1, 5), (1, 33, 127), (10, 8, 411), (40, 20, 4573), (31, 33, 2049),
           (65, 63, 515), (257, 160, 1633), (300, 243, 1000), (160, 160, 2625), (4000, 17, 31), (33000, 33, 64),
-          (240, 240, 240), (409, 405, 411)]
+          (240, 240, 240), (409, 405, 411), (8, 8, 411), (9, 8, 2100), (8, 7, 3), (24, 24, 513), (1, 1, 1)]
 
 
 def padded(rng, rows, cols, ld):
