@@ -20,8 +20,8 @@
 //     and conquer (ZSTEDC).
 //  3. k_larft + k_apply_q_wy: eigenvectors of A = Q (eigenvectors of T), the reflectors
 //     applied by blocks of 32 in compact WY form (I - V T V^H) to the wanted columns only,
-//     four columns per workgroup staged in LDS (one beyond n ~ 1500), each block's
-//     reflectors staged by 64-row chunks.
+//     one or four columns per workgroup staged in LDS, each block's reflectors staged by
+//     64-row chunks.
 //
 // Only the upper triangle of A is read, as Julia's Hermitian(A) does.  Cross-workgroup
 // waits are bounded: a wait that exceeds its spin limit sets a status word, every other
@@ -680,9 +680,12 @@ __global__ void __launch_bounds__(WY_NT_T) k_larft(const cplx<double>* __restric
 // C[:, c] <- Q C[:, c] for the columns c < ncols, Q = B_0 B_1 ... (B_b = I - V_b T_b V_b^H):
 // the blocks are applied last to first to CW columns per workgroup staged in LDS.  Each
 // block's reflectors are read from HBM / L2 in chunks of WY_RC rows staged in LDS with
-// coalesced loads; from a chunk every thread accumulates its share of W = V_b^H C (thread:
-// reflector l, column q, half of the chunk's rows), and after W2 = T_b W the same chunks give
-// C -= V_b W2 (thread: row, column).  V_b's implicit entries: v_l[i0 + l + 1] = 1, zero above.
+// coalesced loads, the next chunk's on their way during the work on one (n = 480, 160 columns,
+// four per workgroup: 371 us, now 235): the chunks' load latency in series bounded it, and
+// now the LDS reads of their products do.  From a chunk every thread accumulates its share
+// of W = V_b^H C (thread: reflector l, column q, half of the chunk's rows), and after
+// W2 = T_b W the same chunks, from the last, which is still staged, give C -= V_b W2
+// (thread: row, column).  V_b's implicit entries: v_l[i0 + l + 1] = 1, zero above.
 constexpr int WY_RC = 64;      // rows of a staged reflector chunk
 template <int CW>
 __global__ void __launch_bounds__(HT_NT) k_apply_q_wy(const cplx<double>* __restrict__ V, long ldv,
@@ -709,24 +712,41 @@ __global__ void __launch_bounds__(HT_NT) k_apply_q_wy(const cplx<double>* __rest
   constexpr int NH = CW == 4 ? 2 : 8;                         // row groups of a chunk
   constexpr int RH = WY_RC / NH;                              // rows per group
   const int nblk = (n - 1 + WY_NB - 1) / WY_NB;
+  // a chunk goes from memory to registers while the one before it is worked on
+  constexpr int NF = WY_RC * WY_NB / HT_NT;
+  cplx<double> pv[NF];
+  auto fetch = [&](int i0, int rb) {
+    const int nr = min(WY_NB, n - 1 - i0);
+#pragma unroll
+    for (int u = 0; u < NF; ++u) {
+      const int e = tid + u * HT_NT, rr = e & (WY_RC - 1), l = e >> 6, r = rb + rr, r1 = i0 + l + 1;
+      cplx<double> v = mk(r == r1 ? 1.0 : 0.0, 0.0);
+      if (r < n && l < nr && r > r1) v = V[(long)(i0 + l) * ldv + r];
+      pv[u] = v;
+    }
+  };
+  auto stage = [&]() {
+#pragma unroll
+    for (int u = 0; u < NF; ++u) {
+      const int e = tid + u * HT_NT;
+      Vs[e & (WY_RC - 1)][e >> 6] = pv[u];
+    }
+  };
+  fetch((nblk - 1) * WY_NB, (nblk - 1) * WY_NB + 1);
   for (int b = nblk - 1; b >= 0; --b) {
     const int i0 = b * WY_NB;
     const int nr = min(WY_NB, n - 1 - i0);
     for (int t = tid; t < WY_NB * WY_NB; t += HT_NT) Ts[t % WY_NB][t / WY_NB] = Tb[(long)b * WY_NB * WY_NB + t];
     // W = V_b^H C over the rows i0 + 1 .. n - 1, chunk by chunk
     cplx<double> acc = mk(0.0, 0.0);
+    const int rlast = i0 + 1 + (n - 2 - i0) / WY_RC * WY_RC;   // the last chunk's first row
     for (int rb = i0 + 1; rb < n; rb += WY_RC) {
       __syncthreads();   // the previous chunk's readers are done
-      for (int e = tid; e < WY_RC * WY_NB; e += HT_NT) {
-        const int rr = e & (WY_RC - 1), l = e >> 6, r = rb + rr;
-        cplx<double> v = mk(0.0, 0.0);
-        if (r < n && l < nr) {
-          const int r1 = i0 + l + 1;
-          v = r == r1 ? mk(1.0, 0.0) : (r > r1 ? V[(long)(i0 + l) * ldv + r] : mk(0.0, 0.0));
-        }
-        Vs[rr][l] = v;
-      }
+      stage();
       __syncthreads();
+      if (rb < rlast) fetch(i0, rb + WY_RC);
+      else if (rb > i0 + 1) fetch(i0, rb - WY_RC);
+      else if (b > 0) fetch(i0 - WY_NB, i0 - WY_NB + 1);
       if (l1 < nr && q1 < nc) {
         for (int k = 0; k < RH; ++k) {
           const int rr = h1 * RH + k, r = rb + rr;
@@ -765,19 +785,16 @@ __global__ void __launch_bounds__(HT_NT) k_apply_q_wy(const cplx<double>* __rest
       for (int l = k; l < nr; ++l) s = s + cmul(Ts[k][l], W[l][q]);
       W2[k][q] = s;
     }
-    // C -= V_b W2, chunk by chunk (thread: row of the chunk, column)
-    for (int rb = i0 + 1; rb < n; rb += WY_RC) {
+    // C -= V_b W2, chunk by chunk from the last, which is still staged (thread: row of the
+    // chunk, column)
+    for (int rb = rlast; rb > i0; rb -= WY_RC) {
       __syncthreads();   // W2 written / the previous chunk's readers are done
-      for (int e = tid; e < WY_RC * WY_NB; e += HT_NT) {
-        const int rr = e & (WY_RC - 1), l = e >> 6, r = rb + rr;
-        cplx<double> v = mk(0.0, 0.0);
-        if (r < n && l < nr) {
-          const int r1 = i0 + l + 1;
-          v = r == r1 ? mk(1.0, 0.0) : (r > r1 ? V[(long)(i0 + l) * ldv + r] : mk(0.0, 0.0));
-        }
-        Vs[rr][l] = v;
+      if (rb < rlast) {
+        stage();
+        __syncthreads();
+        if (rb > i0 + 1) fetch(i0, rb - WY_RC);
+        else if (b > 0) fetch(i0 - WY_NB, i0 - WY_NB + 1);
       }
-      __syncthreads();
       for (int t = tid; t < WY_RC * CW; t += HT_NT) {
         const int rr = t & (WY_RC - 1), q = t >> 6, r = rb + rr;
         if (r < n && q < nc) {
@@ -1403,8 +1420,11 @@ int heevd_dist(pw_ctx* c, void* rb, int n, cplx<double>* A, long lda, double* d_
     hipLaunchKernelGGL(k_larft, dim3(nblk), dim3(WY_NT_T), 0, c->stream, V, ldv, tau, n, Tb);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_check(c, e, "k_larft");
-    // four columns per workgroup while they fit LDS beside the static staging (~60 KiB)
-    const bool cw4 = (size_t)WY_CW * n * sizeof(cplx<double>) <= 96 * 1024;
+    // One column per workgroup while all of them run at once (two per compute unit beside the
+    // ~50 KiB of static staging), four, which share the reflectors' loads, beyond that as long
+    // as they fit LDS: n = 480, 160 columns 185 us against 235; n = 480, 480 columns 322
+    // against 357; n = 960, 960 columns 2190 against 1275.
+    const bool cw4 = nvec > 512 && (size_t)WY_CW * n * sizeof(cplx<double>) <= 96 * 1024;
     const int cw = cw4 ? WY_CW : 1;
     const int blocks = (nvec + cw - 1) / cw;
     const size_t sh = (size_t)cw * n * sizeof(cplx<double>);

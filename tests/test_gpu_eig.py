@@ -251,3 +251,24 @@ def test_heevd_small_orders(ctx, n, kind):
     assert np.abs(w - ref).max() < 1e-12 * scale
     assert np.abs(X.conj().T @ X - np.eye(n)).max() < 1e-12
     assert np.abs(A @ X - X * w).max() < 1e-12 * scale
+
+
+@pytest.mark.parametrize("n,nvec", [(65, 1), (66, 31), (97, 97), (480, 160), (513, 512), (520, 513)])
+def test_heev_lowest_back_transform(ctx, n, nvec):
+    """The reflectors applied to the wanted columns at partial blocks and chunks of rows, and
+    on both sides of the rule between one and four columns per workgroup (512): residuals and
+    orthonormality with the bounds of the orders above."""
+    import ctypes
+    from pwdft_hip._lib import DeviceMatrix
+    rng = np.random.default_rng(n + nvec)
+    A = _herm(rng, n, "random")
+    dA = DeviceMatrix.from_host(ctx, A)
+    w = np.zeros(n)
+    print(f"case heev lowest n={n} nvec={nvec}", flush=True)
+    ctx.call("pw_heev_lowest_dev", n, nvec, dA.p, n, w.ctypes.data_as(ctypes.c_void_p))
+    X = dA.download()[:, :nvec]
+    ref = np.linalg.eigvalsh(A)
+    scale = max(1.0, np.abs(ref).max())
+    assert np.abs(w[:nvec] - ref[:nvec]).max() < 1e-12 * scale * max(1.0, np.sqrt(n) / 4)
+    assert np.abs(X.conj().T @ X - np.eye(nvec)).max() < 1e-12 * max(1.0, np.sqrt(n) / 4)
+    assert np.abs(A @ X - X * w[:nvec]).max() < 1e-12 * scale * max(1.0, np.sqrt(n) / 4)
