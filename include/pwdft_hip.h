@@ -76,8 +76,10 @@ enum {
                                    used anyway for line lengths without a two-pass plan); 2:
                                    always the global-plane pass (compressed planes in HBM, used
                                    anyway when even the compressed plane exceeds LDS) */
-  PW_TUNE_OVERLAP = 6,          /* 1 (default): op_H runs its nonlocal products on a second
-                                   stream beside the FFT passes; 0: one stream, in sequence */
+  PW_TUNE_OVERLAP = 6,          /* 1 (default): op_H runs beta^H psi on a second stream
+                                   beside the FFT passes where the sizes make that pay (2^18
+                                   sphere entries to 6e8 multiply-adds); 0: one stream, in
+                                   sequence */
   PW_TUNE_COL_CHUNK = 7,        /* z-columns per workgroup of the column FFT kernels (0: the
                                    default, as many as 48 KiB of LDS hold) */
   PW_TUNE_GEMM_SPLIT_BF16 = 8,  /* the mixed path's complex GEMMs on BF16 MFMA with each operand

@@ -186,8 +186,13 @@ int op_H_device(pw_ctx* c, int ik, int ispin, int nb, const cplx<double>* psi, l
   };
   // B = beta^H psi (MFMA) runs on stream2 beside the FFT passes (VALU, LDS).  Small problems --
   // a few bands of a small sphere -- keep one stream: the fork and join would cost more than
-  // the overlap saves.
-  const bool fork = vloc && nloc && c->overlap && c->stream2 && (long)k.ngw * nb >= (1L << 18);
+  // the overlap saves.  From about 6e8 multiply-adds on, a product fills the chip by itself and
+  // only takes the FFT passes' issue slots and caches (in sequence against beside: 72^3, 160
+  // bands, 320 projectors 797 against 810 us FP64, 519 against 535 mixed; 122 bands 599 against
+  // 617; 108^3, 243 bands 2565 against 2603); below it the overlap saves up to 9 % (64^3, 100
+  // bands 242 against 226 us; 100 x 54 x 100, 42 bands, 160 projectors 217 against 197).
+  const bool fork = vloc && nloc && c->overlap && c->stream2 && (long)k.ngw * nb >= (1L << 18) &&
+                    (double)k.ngw * nb * k.nbeta < 6e8;
   if (fork) {
     hipError_t e = hipEventRecord(c->ev_fork, c->stream);
     if (e == hipSuccess) e = hipStreamWaitEvent(c->stream2, c->ev_fork, 0);
