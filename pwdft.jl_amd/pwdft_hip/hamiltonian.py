@@ -442,18 +442,20 @@ def calc_rhoe_(Ham, psiks, Rhoe, Focc=None):
     Focc = Ham.electrons.Focc if Focc is None else Focc
     c.call("pw_rhoe_zero")
     nk = Ham.pw.Nkpt
-    nb = psiks[0].cols if isinstance(psiks[0], DeviceMatrix) else 0
-    if (nk > 1 and 0 < nb <= Focc.shape[0] and
-            all(isinstance(p, DeviceMatrix) and p.cols == nb and p.rows >= n for p, n in zip(psiks, Ham.pw.Ngw))):
+    blocks = [psiks[ik] for ik in range(nk)]
+    nb = blocks[0].cols if isinstance(blocks[0], DeviceMatrix) else 0
+    # (occupations of fewer bands or k-points than there are take the loop, which checks its index)
+    if (nk > 1 and 0 < nb <= Focc.shape[0] and Focc.ndim == 2 and Focc.shape[1] >= nk and
+            all(isinstance(p, DeviceMatrix) and p.cols == nb and p.rows >= n for p, n in zip(blocks, Ham.pw.Ngw))):
         # every k-point in the same launches
-        w = np.ascontiguousarray((Ham.pw.wk[:, None] * Focc[:nb, :nk].T), dtype=float)
+        w = np.ascontiguousarray((Ham.pw.wk[:nk, None] * Focc[:nb, :nk].T), dtype=float)
         ik_a = np.arange(nk, dtype=np.int32)
-        ldp = np.array([p.rows for p in psiks[:nk]], dtype=np.int64)
-        c.call("pw_rhoe_accum_batch_dev", nk, ptr(ik_a), nb, _ptr_array([p.p for p in psiks[:nk]]), ptr(ldp), ptr(w),
+        ldp = np.array([p.rows for p in blocks], dtype=np.int64)
+        c.call("pw_rhoe_accum_batch_dev", nk, ptr(ik_a), nb, _ptr_array([p.p for p in blocks]), ptr(ldp), ptr(w),
                Ham.flags_prec)
         nk = 0
     for ik in range(nk):
-        psi = psiks[ik]
+        psi = blocks[ik]
         w = np.ascontiguousarray(Ham.pw.wk[ik] * Focc[:, ik], dtype=float)
         if isinstance(psi, DeviceMatrix):
             c.call("pw_rhoe_accum_dev", ik, psi.cols, psi.p, psi.rows, ptr(w), Ham.flags_prec)

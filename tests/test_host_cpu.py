@@ -246,3 +246,67 @@ def test_autotune_cache_round_trip(tmp_path):
     at.apply_settings(ctx, {"band_batch": 32, "gemm_nn_shape": 4, "fft_order": 2, "unknown": 7})
     assert ctx.calls == [("pw_tune_set", (at.TUNE_FFT_ORDER, 2)), ("pw_tune_set", (at.TUNE_BAND_BATCH, 32)),
                          ("pw_tune_set", (at.TUNE_GEMM_NN_SHAPE, 4))]
+
+
+def _rhoe_stub(nk=4, nb=3, ngw=5):
+    """A Hamiltonian stand-in whose context records its calls, and nk device blocks for it."""
+    from types import SimpleNamespace
+    from pwdft_hip._lib import DeviceMatrix
+
+    class Ctx:
+        h = None
+
+        def __init__(self):
+            self.calls = []
+
+        def call(self, name, *args):
+            if name == "pw_rhoe_accum_batch_dev":   # the weights live as long as the call
+                w = np.ctypeslib.as_array(ctypes.cast(args[5], ctypes.POINTER(ctypes.c_double)), (args[0], args[2]))
+                args = args[:5] + (w.copy(),)
+            self.calls.append((name, args))
+
+    ctx = Ctx()
+
+    def block(cols=nb):
+        m = DeviceMatrix.__new__(DeviceMatrix)
+        m.ctx, m.rows, m.cols, m.p = ctx, ngw, cols, ctypes.c_void_p(4096)
+        return m
+
+    H = SimpleNamespace(ctx=ctx, flags_prec=0, rhoe_symmetrizer=None, pw=SimpleNamespace(
+        Nkpt=nk, Ngw=[ngw] * nk, wk=np.full(nk, 1.0 / nk)))
+    return H, ctx, [block() for _ in range(nk)], block
+
+
+@pytest.mark.parametrize("short", ["blocks", "one_column", "columns"])
+def test_calc_rhoe_short_arguments(short):
+    """Fewer blocks than k-points, or occupations of fewer k-points, are an IndexError as in the loop
+    over k-points; the batched entry point, which reads Nkpt entries of each array, is not called."""
+    from pwdft_hip.hamiltonian import calc_rhoe_
+    H, ctx, psi, _ = _rhoe_stub()
+    focc = np.full((3, 4), 2.0)
+    if short == "blocks":
+        psi = psi[:2]
+    else:
+        focc = focc[:, :1 if short == "one_column" else 3]
+    with pytest.raises(IndexError):
+        calc_rhoe_(H, psi, np.zeros(8), focc)
+    assert "pw_rhoe_accum_batch_dev" not in [n for n, _ in ctx.calls]
+
+
+def test_calc_rhoe_batch_arguments():
+    """Equal blocks go to the batched entry point with one entry per k-point, unequal ones to the loop;
+    any indexable holds the blocks."""
+    from pwdft_hip._lib import DeviceVector
+    from pwdft_hip.hamiltonian import calc_rhoe_
+    out = DeviceVector.__new__(DeviceVector)
+    out.p = ctypes.c_void_p(8192)
+    for holder in (list, tuple, lambda b: dict(enumerate(b)), lambda b: b + b):
+        H, ctx, psi, block = _rhoe_stub()
+        focc = np.arange(15.0).reshape(3, 5)
+        calc_rhoe_(H, holder(psi), out, focc)
+        (args,) = [a for n, a in ctx.calls if n == "pw_rhoe_accum_batch_dev"]
+        assert args[0] == 4 and args[2] == 3 and len(args[3]) == 4
+        assert np.array_equal(args[5], 0.25 * focc[:, :4].T)
+    H, ctx, psi, block = _rhoe_stub()
+    calc_rhoe_(H, psi[:3] + [block(2)], out, np.full((3, 4), 2.0))
+    assert [n for n, _ in ctx.calls].count("pw_rhoe_accum_dev") == 4
