@@ -335,9 +335,60 @@ k_col_ifft(const cplx<double>* __restrict__ psi, long ldpsi, int b0, cplx<T>* __
                    c0, dz, twz);
 }
 
-// 2c. The plane pass where the line lengths have no two-pass plan (125, 162, ...) or
-// PW_TUNE_PLANE_COMPRESSED asks for it; otherwise pw_plane.h runs.  Only the active x lines are
-// kept, compressed (Yc: nxact lines of n2, stride ys; column c sits at slot col_cy[c] =
+// 2. The padded plane in LDS, for what the plane kernels (pw_plane.h) do not take: line lengths
+// without a two-pass plan and, in FP32 and for the density, spheres wider than half the grid.
+// Per (z-plane, band) the inverse y-FFT on the active x lines, then per x-row one wavefront
+// does inverse x-FFT, * V/N (read from L2 inside the first forward pass) and forward
+// x-FFT, then forward y-FFT on the active x lines.  In place on the plane w (ncol entries).
+template <typename T>
+__device__ inline void plane_vloc_body(cplx<T>* __restrict__ w, const T* __restrict__ V, int z,
+                                       const int* __restrict__ col_ij, int ncol, const int* __restrict__ xact,
+                                       int nxact, FftDim dx, FftDim dy, const cplx<T>* __restrict__ twx,
+                                       const cplx<T>* __restrict__ twy) {
+  extern __shared__ char smem_raw[];
+  cplx<T>* lds = reinterpret_cast<cplx<T>*>(smem_raw);
+  const int n1 = dx.n, n2 = dy.n, np = n1 * n2, ps = odd_stride(n1);
+  cplx<T>* tx = lds + ps * n2;
+  cplx<T>* ty = tx + n1;
+  int* xl = reinterpret_cast<int*>(ty + n2);
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  for (int i = tid; i < ps * n2; i += nthr) lds[i] = mk((T)0, (T)0);
+  stage(tx, twx, n1);
+  stage(ty, twy, n2);
+  stage(xl, xact, nxact);
+  __syncthreads();
+  for (int c = tid; c < ncol; c += nthr) lds[col_ij[c]] = w[c];
+  __syncthreads();
+  wave_lines<T, +1, FFT_ME>(lds, nxact, xl, 0, ps, dy, ty);
+  __syncthreads();
+  {
+    const T* v = V + (long)z * np;
+    const int lane = tid & 63, wave = tid >> 6, nwave = nthr >> 6;
+    const int g = lane / dx.L, q = lane - g * dx.L;
+    for (int t0 = wave * dx.gpw; t0 < n2; t0 += nwave * dx.gpw) {
+      const int row = t0 + g;
+      const bool active = g < dx.gpw && row < n2;
+      const int base = active ? row * ps : 0;
+      wave_row_vloc<T>(lds, base, dx, tx, q, active, v + (long)(active ? row : 0) * n1);
+    }
+  }
+  __syncthreads();
+  wave_lines<T, -1, FFT_ME>(lds, nxact, xl, 0, ps, dy, ty);
+  __syncthreads();
+  for (int c = tid; c < ncol; c += nthr) w[c] = lds[col_ij[c]];
+}
+
+template <typename T>
+__global__ void __launch_bounds__(PlaneNT<T>::value)
+k_plane_vloc(cplx<T>* __restrict__ W, const T* __restrict__ V, const int* __restrict__ col_ij,
+             int ncol, const int* __restrict__ xact, int nxact, FftDim dx, FftDim dy,
+             const cplx<T>* __restrict__ twx, const cplx<T>* __restrict__ twy, int n3) {
+  const int z = blockIdx.x, bl = blockIdx.y;
+  plane_vloc_body<T>(W + ((long)bl * n3 + z) * ncol, V, z, col_ij, ncol, xact, nxact, dx, dy, twx, twy);
+}
+
+// 2c. The plane pass where neither the plane kernels nor LDS take the padded plane, or
+// PW_TUNE_PLANE_COMPRESSED asks for it.  Only the active x lines are kept, compressed (Yc: nxact lines of n2, stride ys; column c sits at slot col_cy[c] =
 // a*ys + y for x = xact[a]).  The x-transform of each row runs in a
 // per-wavefront row buffer of n1 entries: the row is expanded from Yc (zero at inactive x),
 // transformed (inverse, * V/N, forward) and its active entries gathered back.  rl rows are
@@ -466,6 +517,39 @@ k_plane_rhoe_c(const cplx<T>* __restrict__ W, const double* __restrict__ wts, in
 // G->R of real fields on a sphere (FP64), after k_col_ifft: per (z-plane, field) the inverse
 // y-FFT of the active x lines and the inverse x-FFT of every row, then
 // out[f N + r] = scale Re f(r) (added to out when acc is set).
+__global__ void __launch_bounds__(PlaneNT<double>::value)
+k_plane_g2r(const cplx<double>* __restrict__ W, double* __restrict__ out, long N, double scale, int acc,
+            const int* __restrict__ col_ij, int ncol, const int* __restrict__ xact, int nxact, FftDim dx, FftDim dy,
+            const cplx<double>* __restrict__ twx, const cplx<double>* __restrict__ twy, int n3) {
+  extern __shared__ char smem_raw[];
+  cplx<double>* lds = reinterpret_cast<cplx<double>*>(smem_raw);
+  const int n1 = dx.n, n2 = dy.n, np = n1 * n2, ps = odd_stride(n1);
+  cplx<double>* tx = lds + ps * n2;
+  cplx<double>* ty = tx + n1;
+  int* xl = reinterpret_cast<int*>(ty + n2);
+  const int z = blockIdx.x, f = blockIdx.y;
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  for (int i = tid; i < ps * n2; i += nthr) lds[i] = mk(0.0, 0.0);
+  stage(tx, twx, n1);
+  stage(ty, twy, n2);
+  stage(xl, xact, nxact);
+  __syncthreads();
+  const cplx<double>* w = W + ((long)f * n3 + z) * ncol;
+  for (int c = tid; c < ncol; c += nthr) lds[col_ij[c]] = w[c];
+  __syncthreads();
+  wave_lines<double, +1, FFT_ME>(lds, nxact, xl, 0, ps, dy, ty);
+  __syncthreads();
+  wave_lines<double, +1, FFT_ME>(lds, n2, nullptr, ps, 1, dx, tx);
+  __syncthreads();
+  double* o = out + (long)f * N + (long)z * np;
+  for (int i = tid; i < np; i += nthr) {
+    const int j = i / n1, x = i - j * n1;
+    const double v = scale * lds[x + ps * j].x;
+    o[i] = acc ? o[i] + v : v;
+  }
+}
+
+// The same for planes beyond LDS, in the compressed form of k_plane_vloc_c.
 __global__ void __launch_bounds__(PlaneNT<double>::value)
 k_plane_g2r_c(const cplx<double>* __restrict__ W, double* __restrict__ out, long N, double scale, int acc,
               const int* __restrict__ col_cy, int ncol, const int* __restrict__ xact, int nxact, FftDim dx,
@@ -647,6 +731,17 @@ k_col_ifft_batch(const KBatch* __restrict__ kb, int nk, int nb, cplx<T>* __restr
 }
 
 template <typename T>
+__global__ void __launch_bounds__(PlaneNT<T>::value)
+k_plane_vloc_batch(const KBatch* __restrict__ kb, int nb, cplx<T>* __restrict__ W, const T* __restrict__ V,
+                   FftDim dx, FftDim dy, const cplx<T>* __restrict__ twx, const cplx<T>* __restrict__ twy,
+                   int n3) {
+  const int z = blockIdx.x, kk = blockIdx.y / nb, bl = blockIdx.y - kk * nb;
+  const KBatch& d = kb[kk];
+  plane_vloc_body<T>(W + d.woff + ((long)bl * n3 + z) * d.ncol, V, z, d.col_ij, d.ncol, d.xact, d.nxact, dx, dy,
+                     twx, twy);
+}
+
+template <typename T>
 __global__ void __launch_bounds__(COL_NT)
 k_col_fft_batch(const KBatch* __restrict__ kb, int nk, int nb, const cplx<T>* __restrict__ W, int C, FftDim dz,
                 const cplx<T>* __restrict__ twz, int kin, int acc) {
@@ -656,6 +751,62 @@ k_col_fft_batch(const KBatch* __restrict__ kb, int nk, int nb, const cplx<T>* __
   if (!batch_col_block(d, C, nb, w - d.blk0, c0, bl)) return;
   col_fft_body<T>(W + d.woff + (long)bl * dz.n * d.ncol, d.psi + (long)bl * d.ldpsi, d.hpsi + (long)bl * d.ldh,
                   d.ent_igw, d.ent_pos, d.col_ptr, d.ncol, C, c0, dz, twz, d.gk2, kin, acc);
+}
+
+// rho planes: per (z-plane, band group): y/x inverse FFT of each band and
+// sum_b w_b |psi_b(r)|^2 accumulated in registers (plane point tid + r * blockDim.x in
+// register r, NR <= RHO_REGS per thread: the launch picks the smallest NR that covers the
+// plane, so no accumulator registers go unused); one partial plane per group.
+constexpr int RHO_REGS = 16;
+template <typename T, int NR>
+__global__ void __launch_bounds__(PlaneNT<T>::value)
+k_plane_rhoe(const cplx<T>* __restrict__ W, const double* __restrict__ wts, int nb, int bpg,
+             double* __restrict__ rpart, long N, const int* __restrict__ col_ij, int ncol,
+             const int* __restrict__ xact, int nxact, FftDim dx, FftDim dy,
+             const cplx<T>* __restrict__ twx, const cplx<T>* __restrict__ twy, int n3) {
+  extern __shared__ char smem_raw[];
+  cplx<T>* lds = reinterpret_cast<cplx<T>*>(smem_raw);
+  const int n1 = dx.n, n2 = dy.n, np = n1 * n2, ps = odd_stride(n1);
+  cplx<T>* tx = lds + ps * n2;
+  cplx<T>* ty = tx + n1;
+  int* xl = reinterpret_cast<int*>(ty + n2);
+  const int z = blockIdx.x, g = blockIdx.y;
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  stage(tx, twx, n1);
+  stage(ty, twy, n2);
+  stage(xl, xact, nxact);
+  double acc[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) acc[r] = 0.0;
+  const int bend = min(nb, (g + 1) * bpg);
+  for (int b = g * bpg; b < bend; ++b) {
+    for (int i = tid; i < ps * n2; i += nthr) lds[i] = mk((T)0, (T)0);
+    __syncthreads();
+    const cplx<T>* w = W + ((long)b * n3 + z) * ncol;
+    for (int c = tid; c < ncol; c += nthr) lds[col_ij[c]] = w[c];
+    __syncthreads();
+    wave_lines<T, +1, FFT_ME>(lds, nxact, xl, 0, ps, dy, ty);
+    __syncthreads();
+    wave_lines<T, +1, FFT_ME>(lds, n2, nullptr, ps, 1, dx, tx);
+    __syncthreads();
+    const double wb = wts[b];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const int i = tid + r * nthr;
+      if (i < np) {
+        const int j = i / n1, x = i - j * n1;
+        const double re = (double)lds[x + ps * j].x, im = (double)lds[x + ps * j].y;
+        acc[r] += wb * (re * re + im * im);
+      }
+    }
+    __syncthreads();
+  }
+  double* out = rpart + (long)g * N + (long)z * np;
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const int i = tid + r * nthr;
+    if (i < np) out[i] = acc[r];
+  }
 }
 
 __global__ void k_rho_reduce(double* __restrict__ rho, const double* __restrict__ rpart, int ng,
@@ -707,6 +858,27 @@ static bool lanes_ok(const FftDim& d) { return d.L >= 1 && d.L <= 64 && d.gpw >=
 static size_t plane_lds(const pw_ctx* c, size_t esz, int nxact) {
   return ((size_t)odd_stride(c->n1) * c->n2 + c->n1 + c->n2) * esz + (size_t)nxact * sizeof(int);
 }
+// Whether the padded kernels take planes with at most maxx active x that the plane kernels do
+// not.  Where LDS holds the padded plane they beat the compressed ones (compressed / padded, us per
+// op_V_loc and per density of half spheres in FP64: 10^3, 64 bands 52 / 26 and 52 / 34;
+// 240 x 24 x 24, 32 bands 134 / 104 and 103 / 83; 125 x 50 x 50, 40 bands 286 / 254 and 209 / 173;
+// a sphere of radius 20 on 72^3, 160 bands: density 534 / 409, op_V_loc in FP32 441 / 327), whose
+// row buffers moreover do not fit beside planes long in x (375 x 20).
+static bool padded_applies(const pw_ctx* c, size_t esz, int maxx) {
+  return c->plane_compressed == 0 && plane_lds(c, esz, maxx) <= 160 * 1024;
+}
+// Threads of a padded-plane workgroup (the kernels index by blockDim.x): wavefronts for one
+// pass over the plane's lines, max(nxact y lines, n2 x rows) / lines per wavefront, when that
+// is at most half of PlaneNT.  Small planes (20^2: one wavefront) then fit many workgroups
+// per CU instead of one or two mostly idle ones; large planes keep PlaneNT.
+template <typename T>
+static int plane_threads(const pw_ctx* c, int nxact) {
+  const FftDim& dx = c->dim[0];
+  const FftDim& dy = c->dim[1];
+  const int waves = std::max(1, std::max((nxact + dy.gpw - 1) / dy.gpw, (c->n2 + dx.gpw - 1) / dx.gpw));
+  return 2 * 64 * waves <= PlaneNT<T>::value ? 64 * waves : PlaneNT<T>::value;
+}
+
 // Threads of a column workgroup holding C columns: wavefronts for one pass over its C lines
 // when that is at most half of COL_NT, else COL_NT (the column kernels index by blockDim.x).
 static int col_threads(const pw_ctx* c, int C) {
@@ -758,9 +930,10 @@ static int vloc_run(pw_ctx* c, KData& k, const T* V, int nb, const cplx<double>*
   // an XCD at once and Hpsi's scattered rows merge in L2 (Si64: 151 -> 87 MB written per
   // launch); W's layout does not depend on the chunk
   const int Cf = (sizeof(T) == 4 && c->tune_col_chunk <= 0) ? std::min(C, 32) : C;
-  size_t plane_bytes = 0;
+  size_t plane_bytes = plane_lds(c, esz, k.nxact);
   int rl = 0;
-  const bool compressed = !plane_applies<T>(c, k.nxact, k.half);
+  const bool planes = plane_applies<T>(c, k.nxact, k.half);
+  const bool compressed = !planes && !padded_applies(c, esz, k.nxact);
   const bool cols = col_chunk<T>(c, k.zhalf) > 0;
   PlaneGP gp;
   bool global_plane = false;
@@ -818,8 +991,11 @@ static int vloc_run(pw_ctx* c, KData& k, const T* V, int nb, const cplx<double>*
       } else if (compressed)
         hipLaunchKernelGGL(k_plane_vloc_c<T>, g2, dim3(PlaneNT<T>::value), plane_bytes, c->stream, W, V,
                            k.d_col_cy, k.ncol, k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0], tw[1], c->n3, rl);
-      else
+      else if (planes)
         plane_vloc<T>(c, k, W, V, nbb);
+      else
+        hipLaunchKernelGGL(k_plane_vloc<T>, g2, dim3(plane_threads<T>(c, k.nxact)), plane_bytes, c->stream, W, V,
+                           k.d_col_ij, k.ncol, k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0], tw[1], c->n3);
     }
     {
       ProfScope ps(c, PW_PROF_COL_FFT, wb + psib * ((kin ? 1 : 0) + (acc ? 1 : 0) + 1) + k.ngw * 16.0);
@@ -879,6 +1055,8 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
     d.ent_igw = k.d_ent_igw;
     d.ent_pos = k.d_ent_pos;
     d.col_ptr = k.d_col_ptr;
+    d.col_ij = k.d_col_ij;
+    d.xact = k.d_xact;
     d.ctab = k.d_ctab;
     d.apos = k.d_apos;
     d.ztab = k.d_ztab;
@@ -900,11 +1078,14 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
   if (blk > 0x7fffffffL) return set_error(c, PW_ERR_ARG, "op_H batch too large for one launch");
   if (plane_lds(c, esz, maxx) > 160 * 1024)
     return set_error(c, PW_ERR_ARG, "z-plane does not fit in LDS for this precision");
-  // without a plane kernel for these lengths, the compressed planes k-point after k-point
+  // the compressed planes run k-point after k-point
   const bool planes = plane_applies<T>(c, maxx, half);
   size_t plane_bytes = 0;
   const int rl = planes ? 0 : plane_c_rows(c, esz, maxx, PlaneNT<T>::value, &plane_bytes);
-  if (!planes && rl < 1) return set_error(c, PW_ERR_ARG, "z-plane does not fit in LDS for this precision");
+  const bool padded = !planes && (padded_applies(c, esz, maxx) || (rl < 1 && plane_lds(c, esz, maxx) <= 160 * 1024));
+  if (padded) plane_bytes = plane_lds(c, esz, maxx);
+  if (!planes && !padded && rl < 1)
+    return set_error(c, PW_ERR_ARG, "z-plane does not fit in LDS for this precision");
   int rc = ensure(c, &c->d_work, &c->work_bytes, (size_t)woff * esz);
   if (rc) return rc;
   const void* dptr = nullptr;
@@ -922,6 +1103,9 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
                        nk, nb, W, C, c->dim[2], tw[2]);
   if (planes)
     plane_vloc_batch<T>(c, dkb, nk, nb, maxx, half, W, V);
+  else if (padded)
+    hipLaunchKernelGGL(k_plane_vloc_batch<T>, dim3(c->n3, nk * nb), dim3(plane_threads<T>(c, maxx)), plane_bytes,
+                       c->stream, dkb, nb, W, V, c->dim[0], c->dim[1], tw[0], tw[1], c->n3);
   else
     for (int kk = 0; kk < nk; ++kk) {
       const KData& k = c->kd[iks[kk]];
@@ -1466,9 +1650,13 @@ static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldp
   KData& k = c->kd[ik];
   const size_t esz = sizeof(cplx<T>);
   const int C = cols_per_block(c, esz);
-  size_t plane_bytes = 0;
+  const int np = c->n1 * c->n2;
+  size_t plane_bytes = plane_lds(c, esz, k.nxact);
   int rl = 0;
-  const bool compressed = !(k.half && plane_applies<T>(c, k.nxact, true));
+  const bool planes = k.half && plane_applies<T>(c, k.nxact, true);
+  // the padded kernel keeps each thread's share of the plane (<= RHO_REGS points) in registers;
+  // planes beyond that take the compressed kernel, which accumulates in HBM
+  const bool compressed = !planes && !(padded_applies(c, esz, k.nxact) && np <= RHO_REGS * PlaneNT<T>::value);
   if (compressed) {
     rl = plane_c_rows(c, esz, k.nxact, PlaneNT<T>::value, &plane_bytes);
     if (rl < 1) return set_error(c, PW_ERR_ARG, "z-plane too large for calc_rhoe kernel");
@@ -1480,7 +1668,7 @@ static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldp
   if (rc) return rc;
   // band groups: about one round of resident plane workgroups over the n3 planes; each group's
   // partial plane is reduced afterwards in a fixed order
-  const int ngroup = rho_groups(c, compressed ? 3 : plane_rho_resident<T>(c, k.nxact), bb);
+  const int ngroup = rho_groups(c, planes ? plane_rho_resident<T>(c, k.nxact) : 3, bb);
   rc = ensure(c, &c->d_rpart, &c->rpart_bytes, (size_t)ngroup * c->N * sizeof(double));
   if (rc) return rc;
   cplx<T>* W = reinterpret_cast<cplx<T>*>(c->d_work);
@@ -1503,8 +1691,19 @@ static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldp
       hipLaunchKernelGGL(k_plane_rhoe_c<T>, dim3(c->n3, ngu), dim3(PlaneNT<T>::value), plane_bytes, c->stream, W,
                          d_w + b0, nbb, bpg, reinterpret_cast<double*>(c->d_rpart), c->N, k.d_col_cy, k.ncol,
                          k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0], tw[1], c->n3, rl);
-    else
+    else if (planes)
       plane_rho<T>(c, k, W, nbb, bpg, ngu, d_w + b0, reinterpret_cast<double*>(c->d_rpart));
+    else {
+      // the plane's points over the threads, at most RHO_REGS each
+      int nt = plane_threads<T>(c, k.nxact);
+      while ((np + nt - 1) / nt > RHO_REGS) nt += 64;
+      const int nr = (np + nt - 1) / nt;
+      auto kern = nr <= 4 ? k_plane_rhoe<T, 4> : nr <= 6 ? k_plane_rhoe<T, 6> : nr <= 8 ? k_plane_rhoe<T, 8>
+                : nr <= 12 ? k_plane_rhoe<T, 12> : k_plane_rhoe<T, RHO_REGS>;
+      hipLaunchKernelGGL(kern, dim3(c->n3, ngu), dim3(nt), plane_bytes, c->stream, W, d_w + b0, nbb,
+                         bpg, reinterpret_cast<double*>(c->d_rpart), c->N, k.d_col_ij, k.ncol, k.d_xact, k.nxact,
+                         c->dim[0], c->dim[1], tw[0], tw[1], c->n3);
+    }
     hipLaunchKernelGGL(k_rho_reduce, dim3(1024), dim3(256), 0, c->stream, c->d_rho,
                        reinterpret_cast<const double*>(c->d_rpart), ngu, c->N, 1.0 / c->omega);
   }
@@ -1599,9 +1798,10 @@ int g2r_apply(pw_ctx* c, KData& k, int nf, const cplx<double>* fG, long ldf, dou
               int acc) {
   const size_t esz = sizeof(cplx<double>);
   const int C = cols_per_block(c, esz);
-  size_t plane_bytes = 0;
+  size_t plane_bytes = plane_lds(c, esz, k.nxact);
   int rl = 0;
-  const bool compressed = !plane_applies<double>(c, k.nxact, false);
+  const bool planes = plane_applies<double>(c, k.nxact, false);
+  const bool compressed = !planes && !padded_applies(c, esz, k.nxact);
   PlaneGP gp;
   bool global_plane = false;
   if (compressed) {
@@ -1651,8 +1851,12 @@ int g2r_apply(pw_ctx* c, KData& k, int nf, const cplx<double>* fG, long ldf, dou
       hipLaunchKernelGGL(k_plane_g2r_c, dim3(c->n3, nbb), dim3(PlaneNT<double>::value), plane_bytes, c->stream, W,
                          o, c->N, scale, acc, k.d_col_cy, k.ncol, k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0],
                          tw[1], c->n3, rl);
-    else
+    else if (planes)
       plane_real(c, k, W, nbb, o, scale, acc);
+    else
+      hipLaunchKernelGGL(k_plane_g2r, dim3(c->n3, nbb), dim3(plane_threads<double>(c, k.nxact)), plane_bytes, c->stream,
+                         W, o, c->N, scale, acc, k.d_col_ij, k.ncol, k.d_xact, k.nxact, c->dim[0], c->dim[1], tw[0],
+                         tw[1], c->n3);
   }
   return hip_check(c, hipGetLastError(), "G->R kernels");
 }

@@ -113,6 +113,8 @@ struct KBatch {
   const int* ent_igw;
   const int* ent_pos;
   const int* col_ptr;
+  const int* col_ij;
+  const int* xact;
   const int* ctab;
   const int* apos;
   const int* ztab;

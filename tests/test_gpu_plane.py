@@ -74,18 +74,14 @@ RHO = [((n, n, 120), m) for n in (15, 24, 27, 45, 72, 75) for m in (False, True)
 RHO += [((108, 108, 120), False), ((135, 135, 150), True), ((40, 75, 120), True), ((75, 27, 120), False)]
 
 
-@pytest.mark.parametrize("ns,mixed", RHO)
-def test_rho_groups(ns, mixed):
-    """More bands than groups, so a workgroup carries its plane state over several bands."""
+def check_rho(ns, idx, nb, mixed):
     from pwdft_hip._lib import PW_MIXED, ptr
-    idx = index_set(ns, [(n - 1) // 4 for n in ns])
     c = context(ns, idx)
     rng = np.random.default_rng(2)
-    nb = 16
     psi = rand(rng, idx.size, nb)
     w = rng.random(nb)
     N = int(np.prod(ns))
-    print(f"case rho {ns} mixed={mixed}", flush=True)
+    print(f"case rho {ns} ngw={idx.size} mixed={mixed}", flush=True)
     c.call("pw_rhoe_zero")
     c.call("pw_rhoe_accum", 0, nb, ptr(psi), idx.size, ptr(w), PW_MIXED if mixed else 0)
     got = np.empty(N)
@@ -97,6 +93,76 @@ def test_rho_groups(ns, mixed):
         ref += w[b] * np.abs(np.fft.ifftn(f.reshape(ns[2], ns[1], ns[0])).reshape(-1)) ** 2
     ref *= float(N) ** 2 / 3.7
     assert np.abs(got - ref).max() <= (2e-5 if mixed else 1e-12) * np.abs(ref).max()
+    c.close()
+
+
+@pytest.mark.parametrize("ns,mixed", RHO)
+def test_rho_groups(ns, mixed):
+    """More bands than groups, so a workgroup carries its plane state over several bands."""
+    check_rho(ns, index_set(ns, [(n - 1) // 4 for n in ns]), 16, mixed)
+
+
+# planes long in x (whose compressed form leaves no room for row buffers), lengths without a plan, and
+# spheres beyond the half-sphere window
+@pytest.mark.parametrize("ns,extent,mixed", [
+    ((375, 20, 12), "half", False), ((320, 30, 12), "half", False), ((125, 50, 12), "half", True),
+    ((10, 10, 12), "half", False), ((72, 72, 12), "wide", False), ((72, 72, 12), "wide", True),
+    ((96, 96, 12), "full", False), ((125, 80, 12), "full", False), ((16, 15, 12), "full", True)])
+def test_rho_general(ns, extent, mixed):
+    radius = {"half": [(n - 1) // 4 for n in ns], "wide": [0.28 * n for n in ns],
+              "full": [n // 2 - 0.6 for n in ns]}[extent]
+    check_rho(ns, index_set(ns, radius), 3, mixed)
+
+
+# the plane passes of the batched op_H: plane kernels, padded planes (one length without a plan, planes
+# long in x, an FP32 sphere beyond the window)
+@pytest.mark.parametrize("ns,extent,mixed", [
+    ((24, 36, 20), "half", False), ((24, 36, 20), "half", True), ((125, 12, 12), "half", False),
+    ((12, 125, 12), "half", True), ((375, 20, 12), "half", False),
+    ((45, 45, 12), "wide", True), ((45, 45, 12), "wide", False), ((96, 96, 12), "full", False)])
+@pytest.mark.parametrize("acc", [False, True])
+def test_op_H_batch(ns, extent, mixed, acc):
+    """Local potential and kinetic term over k-points of different spheres, against numpy."""
+    from pwdft_hip._lib import (PW_ACCUMULATE, PW_MIXED, PW_TERM_K, PW_TERM_VLOC, PW_TUNE_FUSED_BATCH, DeviceMatrix,
+                                ptr)
+    rng = np.random.default_rng(4)
+    nk, nb = 3, 2
+    # the first sphere is the widest, and one k-point alone goes beyond the window
+    scale = {"half": [(n - 1) // 4 for n in ns], "wide": [0.3 * n for n in ns],
+             "full": [n // 2 - 0.6 for n in ns]}[extent]
+    sets = [index_set(ns, [r - ik * (0.5 if extent == "half" else 0.1 * r) for r in scale], shift=0.2 * ik / nk)
+            for ik in range(nk)]
+    c = context(ns, sets[0])
+    c.call("pw_tune_set", PW_TUNE_FUSED_BATCH, 0)   # the three-stage launches also where a box fits LDS
+    gk = [rng.standard_normal((s.size, 3)) for s in sets]
+    for ik in range(nk):
+        c.call("pw_set_kpoint", ik, sets[ik].size, ptr(sets[ik]), 0, ptr(gk[ik]))
+    V = rng.standard_normal(int(np.prod(ns)))
+    c.call("pw_set_vloc", 0, ptr(V))
+    psi = [rand(rng, s.size, nb) for s in sets]
+    # what is there before is added to, or (NaN) never read
+    old = [rand(rng, s.size, nb) if acc else np.full((s.size, nb), np.nan + 0j) for s in sets]
+    dev = [DeviceMatrix.from_host(c, p) for p in psi]
+    out = [DeviceMatrix.from_host(c, o) for o in old]
+    iks = np.arange(nk, dtype=np.int32)
+    ld = np.array([s.size for s in sets], dtype=np.int64)
+    pp = np.array([d.p.value for d in dev], dtype=np.uint64)
+    hp = np.array([d.p.value for d in out], dtype=np.uint64)
+    print(f"case op_H batch {ns} {extent} mixed={mixed} acc={acc}", flush=True)
+    c.call("pw_op_H_batch_dev", nk, ptr(iks), 0, nb, ptr(pp), ptr(ld), ptr(hp), ptr(ld),
+           PW_TERM_VLOC | PW_TERM_K | (PW_MIXED if mixed else 0) | (PW_ACCUMULATE if acc else 0))
+    c.call("pw_synchronize")
+    for ik in range(nk):
+        f = np.zeros((nb, ns[2], ns[1], ns[0]), dtype=complex)
+        f.reshape(nb, -1)[:, sets[ik]] = psi[ik].T
+        f = np.fft.fftn(np.fft.ifftn(f, axes=(1, 2, 3)) * V.reshape(ns[2], ns[1], ns[0]), axes=(1, 2, 3))
+        ref = f.reshape(nb, -1)[:, sets[ik]].T + 0.5 * (gk[ik] ** 2).sum(1)[:, None] * psi[ik]
+        if acc:
+            ref = ref + old[ik]
+        got = out[ik].download()
+        assert np.abs(got - ref).max() <= (2e-5 if mixed else 1e-12) * np.abs(ref).max(), ik
+    for d in dev + out:
+        d.free()
     c.close()
 
 
