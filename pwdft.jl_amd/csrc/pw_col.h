@@ -249,9 +249,10 @@ ColKernel<T> col_kernel(int n, bool fwd, int* chunk, size_t* lds) {
 extern template ColKernel<double> col_kernel<double, true>(int, bool, int*, size_t*);
 extern template ColKernel<double> col_kernel<double, false>(int, bool, int*, size_t*);
 extern template ColKernel<float> col_kernel<float, true>(int, bool, int*, size_t*);
+extern template ColKernel<float> col_kernel<float, false>(int, bool, int*, size_t*);
 
 // Host side (pw_col.hip).  col_chunk: columns per workgroup of the kernels for this context, 0
-// where they do not apply (no plan for n3, FP32 beyond half spheres, PW_TUNE_COL_CHUNK or
+// where they do not apply (no plan for n3, PW_TUNE_COL_CHUNK or
 // PW_TUNE_FFT_ORDER asking for the general kernels).  Launches go to the context stream.
 template <typename T>
 int col_chunk(const pw_ctx* c, bool zhalf);

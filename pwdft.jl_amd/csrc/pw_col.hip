@@ -6,11 +6,7 @@ namespace pw {
 template <typename T>
 static ColKernel<T> kernel_of(const pw_ctx* c, bool zhalf, bool fwd, int* chunk, size_t* lds) {
   if (c->tune_col_chunk > 0 || c->fft_order != 0) return nullptr;
-  if (zhalf) return col_kernel<T, true>(c->n3, fwd, chunk, lds);
-  if constexpr (sizeof(T) == 8)
-    return col_kernel<T, false>(c->n3, fwd, chunk, lds);
-  else
-    return nullptr;
+  return zhalf ? col_kernel<T, true>(c->n3, fwd, chunk, lds) : col_kernel<T, false>(c->n3, fwd, chunk, lds);
 }
 
 template <typename T>

@@ -336,7 +336,7 @@ k_col_ifft(const cplx<double>* __restrict__ psi, long ldpsi, int b0, cplx<T>* __
 }
 
 // 2. The padded plane in LDS, for what the plane kernels (pw_plane.h) do not take: line lengths
-// without a two-pass plan and, in FP32 and for the density, spheres wider than half the grid.
+// without a two-pass plan.
 // Per (z-plane, band) the inverse y-FFT on the active x lines, then per x-row one wavefront
 // does inverse x-FFT, * V/N (read from L2 inside the first forward pass) and forward
 // x-FFT, then forward y-FFT on the active x lines.  In place on the plane w (ncol entries).
@@ -861,9 +861,8 @@ static size_t plane_lds(const pw_ctx* c, size_t esz, int nxact) {
 // Whether the padded kernels take planes with at most maxx active x that the plane kernels do
 // not.  Where LDS holds the padded plane they beat the compressed ones (compressed / padded, us per
 // op_V_loc and per density of half spheres in FP64: 10^3, 64 bands 52 / 26 and 52 / 34;
-// 240 x 24 x 24, 32 bands 134 / 104 and 103 / 83; 125 x 50 x 50, 40 bands 286 / 254 and 209 / 173;
-// a sphere of radius 20 on 72^3, 160 bands: density 534 / 409, op_V_loc in FP32 441 / 327), whose
-// row buffers moreover do not fit beside planes long in x (375 x 20).
+// 240 x 24 x 24, 32 bands 134 / 104 and 103 / 83; 125 x 50 x 50, 40 bands 286 / 254 and 209 / 173),
+// whose row buffers moreover do not fit beside planes long in x (375 x 20).
 static bool padded_applies(const pw_ctx* c, size_t esz, int maxx) {
   return c->plane_compressed == 0 && plane_lds(c, esz, maxx) <= 160 * 1024;
 }
@@ -932,7 +931,7 @@ static int vloc_run(pw_ctx* c, KData& k, const T* V, int nb, const cplx<double>*
   const int Cf = (sizeof(T) == 4 && c->tune_col_chunk <= 0) ? std::min(C, 32) : C;
   size_t plane_bytes = plane_lds(c, esz, k.nxact);
   int rl = 0;
-  const bool planes = plane_applies<T>(c, k.nxact, k.half);
+  const bool planes = plane_applies<T>(c, k.nxact);
   const bool compressed = !planes && !padded_applies(c, esz, k.nxact);
   const bool cols = col_chunk<T>(c, k.zhalf) > 0;
   PlaneGP gp;
@@ -1079,7 +1078,7 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
   if (plane_lds(c, esz, maxx) > 160 * 1024)
     return set_error(c, PW_ERR_ARG, "z-plane does not fit in LDS for this precision");
   // the compressed planes run k-point after k-point
-  const bool planes = plane_applies<T>(c, maxx, half);
+  const bool planes = plane_applies<T>(c, maxx);
   size_t plane_bytes = 0;
   const int rl = planes ? 0 : plane_c_rows(c, esz, maxx, PlaneNT<T>::value, &plane_bytes);
   const bool padded = !planes && (padded_applies(c, esz, maxx) || (rl < 1 && plane_lds(c, esz, maxx) <= 160 * 1024));
@@ -1653,7 +1652,7 @@ static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldp
   const int np = c->n1 * c->n2;
   size_t plane_bytes = plane_lds(c, esz, k.nxact);
   int rl = 0;
-  const bool planes = k.half && plane_applies<T>(c, k.nxact, true);
+  const bool planes = plane_applies<T>(c, k.nxact);
   // the padded kernel keeps each thread's share of the plane (<= RHO_REGS points) in registers;
   // planes beyond that take the compressed kernel, which accumulates in HBM
   const bool compressed = !planes && !(padded_applies(c, esz, k.nxact) && np <= RHO_REGS * PlaneNT<T>::value);
@@ -1729,7 +1728,7 @@ static int rhoe_batch_run(pw_ctx* c, int nk, const int* iks, int nb, const cplx<
   }
   const size_t kbytes = (size_t)nb * c->n3 * maxcol * esz;
   const int kc = (int)std::min<size_t>(nk, (256u << 20) / kbytes);
-  if (kc < 2 || !half || !plane_applies<T>(c, maxx, true) || !lanes_ok(c->dim[2])) {
+  if (kc < 2 || !plane_applies<T>(c, maxx) || !lanes_ok(c->dim[2])) {
     for (int kk = 0; kk < nk; ++kk) {
       int rc = rhoe_run<T>(c, iks[kk], nb, psi[kk], ldpsi[kk], d_w + (size_t)kk * nb);
       if (rc) return rc;
@@ -1782,7 +1781,7 @@ static int rhoe_batch_run(pw_ctx* c, int nk, const int* iks, int nb, const cplx<
                          nb, W, C, c->dim[2], twz);
     const int tot = kn * nb, bpg = (tot + std::min(ngroup, tot) - 1) / std::min(ngroup, tot);
     const int ngu = (tot + bpg - 1) / bpg;
-    plane_rho_batch<T>(c, dkb, nb, tot, maxx, W, bpg, ngu, d_w + (size_t)k0 * nb, rpart);
+    plane_rho_batch<T>(c, dkb, nb, tot, maxx, half, W, bpg, ngu, d_w + (size_t)k0 * nb, rpart);
     hipLaunchKernelGGL(k_rho_reduce, dim3(1024), dim3(256), 0, c->stream, c->d_rho, rpart, ngu, c->N, 1.0 / c->omega);
   }
   return hip_check(c, hipGetLastError(), "batched rhoe kernels");
@@ -1800,7 +1799,7 @@ int g2r_apply(pw_ctx* c, KData& k, int nf, const cplx<double>* fG, long ldf, dou
   const int C = cols_per_block(c, esz);
   size_t plane_bytes = plane_lds(c, esz, k.nxact);
   int rl = 0;
-  const bool planes = plane_applies<double>(c, k.nxact, false);
+  const bool planes = plane_applies<double>(c, k.nxact);
   const bool compressed = !planes && !padded_applies(c, esz, k.nxact);
   PlaneGP gp;
   bool global_plane = false;

@@ -556,6 +556,9 @@ template <typename T>
 using PlaneKernel = void (*)(PlaneArgs<T>);
 // The plane kernel of a mode for n1 x n2 planes, null when either length has no plan; half: the
 // k-points' x and y lie in the windows of their plans.  One translation unit defines each.
+// A sphere beyond the window (a grid smaller than twice the sphere) keeps the plane kernels, with
+// every input read: sphere of radius 20 on 72^3, 160 bands, against the padded planes of pw_fft.hip:
+// density 320 us (409) FP64, 200 (242) FP32, FP32 op_V_loc with its column kernels 308 (327).
 template <typename T, int MODE, bool HALF>
 PlaneKernel<T> plane_kernel(int n1, int n2) {
   if (!line_plan_groups(n1) || !line_plan_groups(n2)) return nullptr;
@@ -575,15 +578,18 @@ PlaneKernel<T> plane_kernel(int n1, int n2) {
 extern template PlaneKernel<double> plane_kernel<double, MODE_VLOC, true>(int, int);
 extern template PlaneKernel<double> plane_kernel<double, MODE_VLOC, false>(int, int);
 extern template PlaneKernel<float> plane_kernel<float, MODE_VLOC, true>(int, int);
+extern template PlaneKernel<float> plane_kernel<float, MODE_VLOC, false>(int, int);
 extern template PlaneKernel<double> plane_kernel<double, MODE_RHO, true>(int, int);
+extern template PlaneKernel<double> plane_kernel<double, MODE_RHO, false>(int, int);
 extern template PlaneKernel<float> plane_kernel<float, MODE_RHO, true>(int, int);
+extern template PlaneKernel<float> plane_kernel<float, MODE_RHO, false>(int, int);
 extern template PlaneKernel<double> plane_kernel<double, MODE_REAL, false>(int, int);
 
 // Host side (pw_plane.hip).  plane_applies: whether the plane kernels take planes with at most
-// maxx active x (line lengths with plans, LDS, PW_TUNE_PLANE_COMPRESSED; FP32 half spheres only).
+// maxx active x (line lengths with plans, LDS, PW_TUNE_PLANE_COMPRESSED).
 // The launches go to the context stream and are made only where it holds.
 template <typename T>
-bool plane_applies(const pw_ctx* c, int maxx, bool half);
+bool plane_applies(const pw_ctx* c, int maxx);
 template <typename T>
 void plane_vloc(pw_ctx* c, const KData& k, cplx<T>* W, const T* V, int nb);
 template <typename T>
@@ -593,8 +599,8 @@ void plane_vloc_batch(pw_ctx* c, const KBatch* dkb, int nk, int nb, int maxx, bo
 template <typename T>
 void plane_rho(pw_ctx* c, const KData& k, cplx<T>* W, int nb, int bpg, int ngroup, const double* d_w, double* rpart);
 template <typename T>
-void plane_rho_batch(pw_ctx* c, const KBatch* dkb, int nbk, int nb, int maxx, cplx<T>* W, int bpg, int ngroup,
-                     const double* d_w, double* rpart);
+void plane_rho_batch(pw_ctx* c, const KBatch* dkb, int nbk, int nb, int maxx, bool half, cplx<T>* W, int bpg,
+                     int ngroup, const double* d_w, double* rpart);
 // Workgroups of the density kernel that a CU holds at once, for at most maxx active x.
 template <typename T>
 int plane_rho_resident(const pw_ctx* c, int maxx);

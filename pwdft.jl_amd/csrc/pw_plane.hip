@@ -53,20 +53,16 @@ static int plane_waves(const pw_ctx* c, size_t lds) {
 
 template <typename T>
 static PlaneKernel<T> vloc_kernel(const pw_ctx* c, bool half) {
-  if (half) return plane_kernel<T, MODE_VLOC, true>(c->n1, c->n2);
-  if constexpr (sizeof(T) == 8)
-    return plane_kernel<T, MODE_VLOC, false>(c->n1, c->n2);
-  else
-    return nullptr;
+  return half ? plane_kernel<T, MODE_VLOC, true>(c->n1, c->n2) : plane_kernel<T, MODE_VLOC, false>(c->n1, c->n2);
 }
 
 template <typename T>
-bool plane_applies(const pw_ctx* c, int maxx, bool half) {
+bool plane_applies(const pw_ctx* c, int maxx) {
   PlaneArgs<T> A{};
-  return plane_args<T>(c, maxx, A) != 0 && (sizeof(T) == 8 || half);
+  return plane_args<T>(c, maxx, A) != 0;
 }
-template bool plane_applies<double>(const pw_ctx*, int, bool);
-template bool plane_applies<float>(const pw_ctx*, int, bool);
+template bool plane_applies<double>(const pw_ctx*, int);
+template bool plane_applies<float>(const pw_ctx*, int);
 
 template <typename T>
 void plane_vloc(pw_ctx* c, const KData& k, cplx<T>* W, const T* V, int nb) {
@@ -112,10 +108,12 @@ int plane_rho_resident(const pw_ctx* c, int maxx) {
 }
 
 template <typename T>
-static void rho_launch(pw_ctx* c, PlaneArgs<T>& A, int maxx, cplx<T>* W, int nb, int bpg, int ngroup, const double* d_w,
-                       double* rpart) {
+static void rho_launch(pw_ctx* c, PlaneArgs<T>& A, int maxx, bool half, cplx<T>* W, int nb, int bpg, int ngroup,
+                       const double* d_w, double* rpart) {
   const size_t lds = plane_args<T>(c, maxx, A);
-  const PlaneKernel<T> kern = lds ? plane_kernel<T, MODE_RHO, true>(c->n1, c->n2) : nullptr;
+  if (!lds) return;
+  const PlaneKernel<T> kern =
+      half ? plane_kernel<T, MODE_RHO, true>(c->n1, c->n2) : plane_kernel<T, MODE_RHO, false>(c->n1, c->n2);
   if (!kern) return;
   A.W = W;
   A.nb = nb;
@@ -132,16 +130,16 @@ void plane_rho(pw_ctx* c, const KData& k, cplx<T>* W, int nb, int bpg, int ngrou
   A.apos = k.d_apos;
   A.ncol = k.ncol;
   A.nxact = k.nxact;
-  rho_launch<T>(c, A, k.nxact, W, nb, bpg, ngroup, d_w, rpart);
+  rho_launch<T>(c, A, k.nxact, k.half, W, nb, bpg, ngroup, d_w, rpart);
 }
 
 template <typename T>
-void plane_rho_batch(pw_ctx* c, const KBatch* dkb, int nbk, int nb, int maxx, cplx<T>* W, int bpg, int ngroup,
-                     const double* d_w, double* rpart) {
+void plane_rho_batch(pw_ctx* c, const KBatch* dkb, int nbk, int nb, int maxx, bool half, cplx<T>* W, int bpg,
+                     int ngroup, const double* d_w, double* rpart) {
   PlaneArgs<T> A{};
   A.kb = dkb;
   A.nbk = nbk;
-  rho_launch<T>(c, A, maxx, W, nb, bpg, ngroup, d_w, rpart);
+  rho_launch<T>(c, A, maxx, half, W, nb, bpg, ngroup, d_w, rpart);
 }
 
 void plane_real(pw_ctx* c, const KData& k, cplx<double>* W, int nf, double* out, double scale, int acc) {
@@ -166,8 +164,10 @@ template void plane_vloc_batch<double>(pw_ctx*, const KBatch*, int, int, int, bo
 template void plane_vloc_batch<float>(pw_ctx*, const KBatch*, int, int, int, bool, cplx<float>*, const float*);
 template void plane_rho<double>(pw_ctx*, const KData&, cplx<double>*, int, int, int, const double*, double*);
 template void plane_rho<float>(pw_ctx*, const KData&, cplx<float>*, int, int, int, const double*, double*);
-template void plane_rho_batch<double>(pw_ctx*, const KBatch*, int, int, int, cplx<double>*, int, int, const double*, double*);
-template void plane_rho_batch<float>(pw_ctx*, const KBatch*, int, int, int, cplx<float>*, int, int, const double*, double*);
+template void plane_rho_batch<double>(pw_ctx*, const KBatch*, int, int, int, bool, cplx<double>*, int, int, const double*,
+                                      double*);
+template void plane_rho_batch<float>(pw_ctx*, const KBatch*, int, int, int, bool, cplx<float>*, int, int, const double*,
+                                     double*);
 template int plane_rho_resident<double>(const pw_ctx*, int);
 template int plane_rho_resident<float>(const pw_ctx*, int);
 

@@ -12,8 +12,10 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "csrc")
 SOURCES = ["pw_capi.hip", "pw_fft.hip", "pw_plane.hip", "pw_plane_v64.hip", "pw_plane_v64f.hip", "pw_plane_v32.hip",
-           "pw_plane_r64.hip", "pw_plane_r32.hip", "pw_plane_g64.hip", "pw_col.hip", "pw_col_c64.hip",
-           "pw_col_c64f.hip", "pw_col_c32.hip", "pw_gemm.hip", "pw_forces.hip", "pw_batch.hip", "pw_dense.hip", "pw_scf.hip", "pw_proj.hip", "pw_eig.hip", "pw_lobpcg.hip", "pw_small.hip", "pw_noalloc.hip"]
+           "pw_plane_v32f.hip", "pw_plane_r64.hip", "pw_plane_r64f.hip", "pw_plane_r32.hip", "pw_plane_r32f.hip",
+           "pw_plane_g64.hip", "pw_col.hip", "pw_col_c64.hip", "pw_col_c64f.hip", "pw_col_c32.hip", "pw_col_c32f.hip",
+           "pw_gemm.hip", "pw_forces.hip", "pw_batch.hip", "pw_dense.hip", "pw_scf.hip", "pw_proj.hip", "pw_eig.hip",
+           "pw_lobpcg.hip", "pw_small.hip", "pw_noalloc.hip"]
 OUT = os.path.join(HERE, "libpwdft_hip.so")
 
 # Flags of single sources: the plane and column kernels' pruned butterflies fold their zero inputs away

@@ -55,6 +55,8 @@ VLOC += [((40, 75, 12), "half", m) for m in (False, True)] + [((75, 40, 12), "ha
 VLOC += [((108, 64, 16), "half", False), ((27, 160, 12), "half", True), ((45, 36, 12), "full", False)]
 VLOC += [((16, 15, n), "half", m) for n in PLANS for m in (False, True)]
 VLOC += [((16, 15, n), "full", False) for n in PLANS] + [((16, 15, n), "full", True) for n in (27, 72, 125)]
+VLOC += [((n, n, 12), "full", True) for n in PLANS if n <= 135 and n not in (27, 72)]
+VLOC += [((16, 15, n), "full", True) for n in PLANS if n not in (27, 72)]
 VLOC += [((125, 8, 12), "half", False), ((10, 125, 12), "half", True), ((5, 6, 4), "full", False)]
 
 
@@ -104,10 +106,15 @@ def test_rho_groups(ns, mixed):
 
 # planes long in x (whose compressed form leaves no room for row buffers), lengths without a plan, and
 # spheres beyond the half-sphere window
-@pytest.mark.parametrize("ns,extent,mixed", [
-    ((375, 20, 12), "half", False), ((320, 30, 12), "half", False), ((125, 50, 12), "half", True),
-    ((10, 10, 12), "half", False), ((72, 72, 12), "wide", False), ((72, 72, 12), "wide", True),
-    ((96, 96, 12), "full", False), ((125, 80, 12), "full", False), ((16, 15, 12), "full", True)])
+RHO_GENERAL = [((375, 20, 12), "half", False), ((320, 30, 12), "half", False), ((125, 50, 12), "half", True),
+               ((10, 10, 12), "half", False), ((125, 80, 12), "full", False), ((16, 15, 12), "full", True),
+               ((36, 72, 12), "wide", False), ((72, 36, 12), "wide", True)]
+# (a plane whose active lines LDS cannot hold has no density kernel: 135 in FP64, 192 in FP32)
+RHO_GENERAL += [((n, n, 12), "wide", m) for n in PLANS for m in (False, True) if n <= (180 if m else 128)]
+RHO_GENERAL += [((n, n, 12), "full", False) for n in (12, 27, 45, 96)] + [((n, n, 12), "full", True) for n in (45, 128)]
+
+
+@pytest.mark.parametrize("ns,extent,mixed", RHO_GENERAL)
 def test_rho_general(ns, extent, mixed):
     radius = {"half": [(n - 1) // 4 for n in ns], "wide": [0.28 * n for n in ns],
               "full": [n // 2 - 0.6 for n in ns]}[extent]
@@ -165,15 +172,10 @@ def test_op_H_batch(ns, extent, mixed, acc):
         d.free()
     c.close()
 
-
-@pytest.mark.parametrize("ns,nk,nb,mixed", [((20, 20, 20), 9, 3, False), ((27, 27, 27), 5, 7, True),
-                                            ((36, 24, 45), 3, 5, False), ((24, 36, 20), 4, 40, True),
-                                            ((125, 12, 12), 2, 2, False)])
-def test_rho_batch(ns, nk, nb, mixed):
-    """k-points with different index sets in the same launches (and, without a plan, one by one)."""
+def check_rho_batch(ns, sets, nb, mixed):
     from pwdft_hip._lib import PW_MIXED, DeviceMatrix, ptr
     rng = np.random.default_rng(3)
-    sets = [index_set(ns, [(n - 1) // 4 - (ik % 2) for n in ns], shift=0.2 * ik / nk) for ik in range(nk)]
+    nk = len(sets)
     c = context(ns, sets[0])
     for ik in range(1, nk):
         gk = rng.standard_normal((sets[ik].size, 3))
@@ -202,3 +204,19 @@ def test_rho_batch(ns, nk, nb, mixed):
     for d in dev:
         d.free()
     c.close()
+
+
+@pytest.mark.parametrize("ns,nk,nb,mixed", [((20, 20, 20), 9, 3, False), ((27, 27, 27), 5, 7, True),
+                                            ((36, 24, 45), 3, 5, False), ((24, 36, 20), 4, 40, True),
+                                            ((125, 12, 12), 2, 2, False)])
+def test_rho_batch(ns, nk, nb, mixed):
+    """k-points with different index sets in the same launches (and, without a plan, one by one)."""
+    check_rho_batch(ns, [index_set(ns, [(n - 1) // 4 - (ik % 2) for n in ns], shift=0.2 * ik / nk) for ik in range(nk)],
+                    nb, mixed)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_rho_batch_wide(mixed):
+    """One k-point beyond the half-sphere window among others within it."""
+    ns = (45, 36, 24)
+    check_rho_batch(ns, [index_set(ns, [(0.3 if ik == 1 else 0.22) * n for n in ns]) for ik in range(3)], 4, mixed)
