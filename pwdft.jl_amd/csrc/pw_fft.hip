@@ -1075,8 +1075,6 @@ static int vloc_batch_run(pw_ctx* c, int nk, const int* iks, const T* V, int nb,
     half = half && k.half;
   }
   if (blk > 0x7fffffffL) return set_error(c, PW_ERR_ARG, "op_H batch too large for one launch");
-  if (plane_lds(c, esz, maxx) > 160 * 1024)
-    return set_error(c, PW_ERR_ARG, "z-plane does not fit in LDS for this precision");
   // the compressed planes run k-point after k-point
   const bool planes = plane_applies<T>(c, maxx);
   size_t plane_bytes = 0;

@@ -121,11 +121,12 @@ def test_rho_general(ns, extent, mixed):
     check_rho(ns, index_set(ns, radius), 3, mixed)
 
 
-# the plane passes of the batched op_H: plane kernels, padded planes (one length without a plan, planes
-# long in x, an FP32 sphere beyond the window)
+# the plane passes of the batched op_H: plane kernels (also where LDS holds no padded plane), padded planes
+# (one length without a plan, planes long in x), compressed planes k-point after k-point
 @pytest.mark.parametrize("ns,extent,mixed", [
     ((24, 36, 20), "half", False), ((24, 36, 20), "half", True), ((125, 12, 12), "half", False),
     ((12, 125, 12), "half", True), ((375, 20, 12), "half", False),
+    ((108, 108, 12), "half", False), ((125, 100, 12), "half", False),
     ((45, 45, 12), "wide", True), ((45, 45, 12), "wide", False), ((96, 96, 12), "full", False)])
 @pytest.mark.parametrize("acc", [False, True])
 def test_op_H_batch(ns, extent, mixed, acc):
