@@ -57,7 +57,8 @@ enum {
 int pw_ctx_create(pw_ctx** ctx, int device);
 int pw_ctx_destroy(pw_ctx* ctx);
 const char* pw_last_error(pw_ctx* ctx);
-/* Bands processed per fused FFT launch (intermediates live in HBM/L2 per batch). */
+/* Bands processed per fused FFT launch (intermediates live in HBM/L2 per batch; default 64).
+ * Fewer than the default bound pw_rhoe_accum_batch_dev's work array as well. */
 int pw_set_band_batch(pw_ctx* ctx, int nb);
 
 /* Tuning knobs set by the autotuner (pwdft_hip/autotune.py); no reference counterpart. */
@@ -222,7 +223,8 @@ int pw_rhoe_accum_dev(pw_ctx* ctx, int ik, int nb, const void* psi, int64_t ldps
                       unsigned flags);
 /* pw_rhoe_accum_dev for several k-points (the k loop of calc_rhoe.jl:38-80): k-point iks[i] adds
  * the nb bands psi[i] (Ngw[iks[i]] x nb, leading dimension ldpsi[i]) with weights w[i nb + ist]
- * (host array).  The bands of as many k-points as 256 MiB of transforms hold share each launch. */
+ * (host array).  The bands of as many k-points as 256 MiB of transforms hold share each launch (and at
+ * most as many bands as pw_set_band_batch allows where that is below its default). */
 int pw_rhoe_accum_batch_dev(pw_ctx* ctx, int nk, const int* iks, int nb, void* const* psi, const int64_t* ldpsi,
                             const double* w, unsigned flags);
 int pw_rhoe_get(pw_ctx* ctx, double* rho);

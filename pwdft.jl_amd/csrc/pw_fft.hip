@@ -1708,9 +1708,10 @@ static int rhoe_run(pw_ctx* c, int ik, int nb, const cplx<double>* psi, long ldp
 }
 
 // Every band of the k-points iks: one column launch, one plane launch and one reduction for as
-// many k-points as 256 MiB of W hold (at least two; else k-point after k-point).  A k-point of a
-// metal's mesh is a few bands on a small grid, so its three launches and the wait after them
-// took ~32 us whatever their work (Al fcc, 20^3, 8 bands, 182 k-points: 5.8 -> 0.2 ms).
+// many k-points as 256 MiB of W hold, or as the bands per launch that a caller set below the
+// default to save memory (at least two; else k-point after k-point).  A k-point of a metal's
+// mesh is a few bands on a small grid, so its three launches and the wait after them took
+// ~32 us whatever their work (Al fcc, 20^3, 8 bands, 182 k-points: 5.8 -> 0.2 ms).
 template <typename T>
 static int rhoe_batch_run(pw_ctx* c, int nk, const int* iks, int nb, const cplx<double>* const* psi,
                           const int64_t* ldpsi, const double* d_w) {
@@ -1725,7 +1726,8 @@ static int rhoe_batch_run(pw_ctx* c, int nk, const int* iks, int nb, const cplx<
     zhalf = zhalf && k.zhalf;
   }
   const size_t kbytes = (size_t)nb * c->n3 * maxcol * esz;
-  const int kc = (int)std::min<size_t>(nk, (256u << 20) / kbytes);
+  int kc = (int)std::min<size_t>(nk, (256u << 20) / kbytes);
+  if (c->band_batch < BAND_BATCH_DEFAULT) kc = std::min(kc, c->band_batch / nb);
   if (kc < 2 || !plane_applies<T>(c, maxx) || !lanes_ok(c->dim[2])) {
     for (int kk = 0; kk < nk; ++kk) {
       int rc = rhoe_run<T>(c, iks[kk], nb, psi[kk], ldpsi[kk], d_w + (size_t)kk * nb);

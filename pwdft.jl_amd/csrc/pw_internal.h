@@ -79,6 +79,8 @@ inline void plan_lanes(FftDim& d, int me) {
 // LDS strides: odd line lengths keep strided butterfly reads off a single bank group.
 __host__ __device__ constexpr int odd_stride(int n) { return (n % 2 == 0) ? n + 1 : n; }
 
+constexpr int BAND_BATCH_DEFAULT = 64;   // pw_set_band_batch
+
 // Sphere bookkeeping of one k-point.  Sphere entries are sorted by (column, z);
 // a column is one (x, y) pair that holds at least one entry, columns sorted by (x, y).
 struct KData {
@@ -193,7 +195,7 @@ struct pw_ctx {
   double* d_rho = nullptr;                            // accumulated density [N]
   void* d_tmp = nullptr;   size_t tmp_bytes = 0;      // staging for host-pointer entry points
   void* d_wts = nullptr;   size_t wts_bytes = 0;      // band weights of calc_rhoe
-  int band_batch = 64;
+  int band_batch = pw::BAND_BATCH_DEFAULT;
   // 1: force the compressed plane kernels, 2: the global-plane pass (tuning / tests)
   int plane_compressed = 0;
   int tune_col_chunk = 0;

@@ -221,3 +221,41 @@ def test_rho_batch_wide(mixed):
     """One k-point beyond the half-sphere window among others within it."""
     ns = (45, 36, 24)
     check_rho_batch(ns, [index_set(ns, [(0.3 if ik == 1 else 0.22) * n for n in ns]) for ik in range(3)], 4, mixed)
+
+
+def test_rho_batch_workspace():
+    """Fewer bands per launch than the default bound the batched density's work array: eight k-points of
+    eight bands on 72^3 hold 8 x 8 MiB of transforms, one k-point's 8 MiB where the caller set 8 bands."""
+    import ctypes
+    from pwdft_hip._lib import DeviceMatrix, ptr
+    hip = ctypes.CDLL("libamdhip64.so")
+    ns, nk, nb = (72, 72, 72), 8, 8
+    idx = index_set(ns, [17] * 3)
+    w = np.ones((nk, nb))
+    gk = np.ones((idx.size, 3))
+    iks = np.arange(nk, dtype=np.int32)
+    ld = np.full(nk, idx.size, dtype=np.int64)
+
+    def free_bytes():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    grown, rho = {}, {}
+    for bands in (64, nb):
+        c = context(ns, idx)
+        for ik in range(1, nk):
+            c.call("pw_set_kpoint", ik, idx.size, ptr(idx), 0, ptr(gk))
+        c.call("pw_set_band_batch", bands)
+        dev = DeviceMatrix.from_host(c, rand(np.random.default_rng(9), idx.size, nb))
+        pp = np.full(nk, dev.p.value, dtype=np.uint64)
+        print(f"case rho batch workspace, {bands} bands a launch", flush=True)
+        before = free_bytes()
+        c.call("pw_rhoe_accum_batch_dev", nk, ptr(iks), nb, ptr(pp), ptr(ld), ptr(w), 0)
+        grown[bands] = before - free_bytes()
+        rho[bands] = np.empty(int(np.prod(ns)))
+        c.call("pw_rhoe_get", ptr(rho[bands]))
+        dev.free()
+        c.close()
+    assert np.abs(rho[64] - rho[nb]).max() <= 1e-12 * rho[nb].max()
+    assert grown[nb] <= grown[64] - (40 << 20), grown
