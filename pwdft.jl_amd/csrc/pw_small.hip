@@ -228,9 +228,8 @@ __global__ void __launch_bounds__(SM_NT) k_heev_jacobi(cplx<double>* __restrict_
 //    computes all rotation parameters for itself from the buffer nobody writes;
 //  - a thread keeps one block of A or one pair of V for the whole solve (no index division per
 //    round), A's blocks and V's pairs on different wavefronts side by side;
-//  - tan(theta) only has to annihilate A_pq to about 1e-14 of itself, so it comes from FP32 root
-//    and reciprocal and one Newton step; c = (1 + t^2)^(-1/2) and s = t c, which make the
-//    rotation orthogonal, stay FP64.
+//  - tan(theta) starts from FP32 root and reciprocal; two Newton steps with the residual in FP64
+//    bring it to FP64 accuracy (their slope may be FP32: it scales a correction).
 __device__ inline void jac_pair(int r, int k, int m, int n, int& p, int& q) {
   if (k == 0) {
     p = m - 1;
@@ -319,8 +318,10 @@ __global__ void __launch_bounds__(NT) k_heev_jacobi32(cplx<double>* __restrict__
             const float tf = fabsf((float)tau);
             double t = (double)__builtin_amdgcn_rcpf(tf + __builtin_amdgcn_sqrtf(1.0f + tf * tf));
             const double at = fabs(tau);
-            // t^2 + 2 |tau| t - 1 = 0
-            t -= fma(t, t + 2.0 * at, -1.0) * (double)__builtin_amdgcn_rcpf(2.0f * ((float)t + tf));
+            // t^2 + 2 |tau| t - 1 = 0; 4e-7 -> 1.2e-13 -> 1.7e-16 relative
+            const double h = (double)__builtin_amdgcn_rcpf(2.0f * ((float)t + tf));
+            t -= fma(t, t + 2.0 * at, -1.0) * h;
+            t -= fma(t, t + 2.0 * at, -1.0) * h;
             if (tau < 0.0) t = -t;
             c = rsqrt(1.0 + t * t);
             s = t * c;

@@ -272,3 +272,29 @@ def test_heev_lowest_back_transform(ctx, n, nvec):
     assert np.abs(w[:nvec] - ref[:nvec]).max() < 1e-12 * scale * max(1.0, np.sqrt(n) / 4)
     assert np.abs(X.conj().T @ X - np.eye(nvec)).max() < 1e-12 * max(1.0, np.sqrt(n) / 4)
     assert np.abs(A @ X - X * w[:nvec]).max() < 1e-12 * scale * max(1.0, np.sqrt(n) / 4)
+
+
+def test_heevd_batch_rotation_angle(ctx):
+    """The angle of a rotation in full FP64: 2 x 2 matrices [[0, g], [g*, 1]] whose small eigenvector
+    component is tan(theta) = 1 / (tau + sqrt(tau^2 + 1)), tau = 1 / (2 |g|), over tau = 1 .. 1e12.  |g|^2,
+    its reciprocal root, tau, tan, c, s, the phase and two products round at most twice each: 16 eps."""
+    import ctypes
+    from pwdft_hip._lib import DeviceMatrix
+    rng = np.random.default_rng(17)
+    nb = 600
+    g = 0.5 * 10.0 ** -rng.uniform(0, 12, nb) * np.exp(2j * np.pi * rng.random(nb))
+    A = np.zeros((nb, 2, 2), dtype=complex)   # [batch][column][row]
+    A[:, 1, 0] = g
+    A[:, 0, 1] = g.conj()
+    A[:, 1, 1] = 1.0
+    dA = DeviceMatrix.from_host(ctx, A.reshape(nb, 4).T)
+    w = np.empty((nb, 2))
+    print("case heevd batch 2 x 2", flush=True)
+    ctx.call("pw_heevd_batch_dev", 2, nb, dA.p, 2, 4, w.ctypes.data_as(ctypes.c_void_p))
+    V = dA.download().T.reshape(nb, 2, 2)
+    x, y = g.real.astype(np.longdouble), g.imag.astype(np.longdouble)
+    tau = 0.5 / np.sqrt(x * x + y * y)
+    t = 1 / (tau + np.sqrt(tau * tau + 1))
+    got = np.abs(V[:, 0, 1]) / np.abs(V[:, 0, 0])
+    assert np.max(np.abs(got - t) / t) <= 16 * np.finfo(float).eps
+    dA.free()
