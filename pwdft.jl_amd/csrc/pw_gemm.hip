@@ -71,7 +71,27 @@ template <typename TC, typename TA, typename TB, int TRANSA, int TM, int TN>
 struct WaveTile {
   typedef typename Mfma<TC>::acc_t acc_t;
   static constexpr int RING = TM * TN > 1 ? 4 : 8;   // k-steps in flight
+  // FP32: an accumulator takes the products of RING k-steps only and is then added to a second
+  // one, so that the rounding of a sum over K grows with K / (4 RING) + RING in place of K / 4
+  // (error of A^H B against FP64, 320 x 160 x 23871: 1.5e-7, 5.7e-7 with one chain; 1080 x 480 x
+  // 80797 with a tile per wavefront 4.2e-7, 4.2e-6).  The additions run beside other wavefronts'
+  // MFMAs: 320 x 160 x 23871 170 us (174), 23871 x 160 x 320 128 (126).
+  static constexpr bool WIDE = sizeof(TC) == 4;
   acc_t re[TM][TN], im[TM][TN];
+  acc_t sre[TM][TN], sim[TM][TN];   // WIDE: the second accumulators
+
+  __device__ inline void fold() {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sre[i][j][r] += re[i][j][r];
+          sim[i][j][r] += im[i][j][r];
+          re[i][j][r] = im[i][j][r] = (TC)0;
+        }
+  }
 
   __device__ inline void mma(const cplx<TA> (&a)[TM], const cplx<TB> (&b)[TN]) {
     TC ar[TM], ai[TM], na[TM], br[TN], bi[TN];
@@ -111,7 +131,10 @@ struct WaveTile {
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) re[i][j][r] = im[i][j][r] = (TC)0;
+        for (int r = 0; r < 4; ++r) {
+          re[i][j][r] = im[i][j][r] = (TC)0;
+          if constexpr (WIDE) sre[i][j][r] = sim[i][j][r] = (TC)0;
+        }
     // rows and columns past the matrices take a valid one's data; their outputs are not stored
     const cplx<TA>* pa[TM];
     const cplx<TB>* pb[TN];
@@ -144,6 +167,7 @@ struct WaveTile {
         mma(a[d], b[d]);
         load(d, s + RING + d);
       }
+      if constexpr (WIDE) fold();
     }
     for (; s < n; s += RING) {
 #pragma unroll
@@ -151,6 +175,7 @@ struct WaveTile {
         if (s + d < n) mma(a[d], b[d]);
         if (s + RING + d < n) load(d, s + RING + d);
       }
+      if constexpr (WIDE) fold();
     }
     if (tail && (kend - kbeg) & 3) {
       const bool ok = 4 * full + lg < kend - kbeg;
@@ -161,6 +186,16 @@ struct WaveTile {
 #pragma unroll
       for (int j = 0; j < TN; ++j) tb[j] = ok ? pb[j][4 * full] : mk((TB)0, (TB)0);
       mma(ta, tb);
+    }
+    if constexpr (WIDE) {
+      fold();
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          re[i][j] = sre[i][j];
+          im[i][j] = sim[i][j];
+        }
     }
   }
 };
@@ -188,9 +223,11 @@ __device__ inline void gemm_store(const GemmOut& o, int M, int N, int z, int m, 
   }
 }
 
-// WM x WN wavefronts, each with a 32 x 32 tile of its own.
+// WM x WN wavefronts, each with a 32 x 32 tile of its own.  (FP32: three wavefronts per SIMD in
+// spite of the second accumulators; without the bound the compiler leaves two, A B 5 to 15 %
+// slower.)
 template <typename TC, typename TA, typename TB, int TRANSA, int WM, int WN>
-__global__ void __launch_bounds__(64 * WM * WN)
+__global__ void __launch_bounds__(64 * WM * WN, sizeof(TC) == 4 && WM * WN <= 4 ? 3 : 1)
 k_zgemm(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const cplx<TB>* __restrict__ B,
         long ldb, int kchunk, GemmOut o, int tm, int tn, int nz) {
   int mt, nt, z;
@@ -214,7 +251,7 @@ k_zgemm(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const cpl
 // tiles summed through LDS in wavefront order: products too small to fill the chip with 32 x 32
 // tiles of their own.
 template <typename TC, typename TA, typename TB, int TRANSA, int T, int WK>
-__global__ void __launch_bounds__(64 * WK)
+__global__ void __launch_bounds__(64 * WK, sizeof(TC) == 4 && T == 2 ? 3 : 1)
 k_zgemm_wk(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const cplx<TB>* __restrict__ B,
            long ldb, int kchunk, GemmOut o, int tm, int tn, int nz) {
   __shared__ cplx<TC> red[WK][16][17];
@@ -252,6 +289,9 @@ k_zgemm_wk(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
 // applied (no sign work in the MFMA loop).  Lane l feeds row (or column) l % 16 with the 8
 // consecutive real k of slot block l / 16; the accumulator layout equals that of the FP32
 // 16x16x4 MFMA, so the tiles, split-K and epilogue are those of k_zgemm.
+// As in WaveTile an accumulator takes a short chain (one stage, two for A^H B, whose K is long)
+// and is then added to a second one: error of A B 23871 x 160 x 320 1.0e-7 (3.8e-7 with one
+// chain), of A^H B 1080 x 480 x 80797 3.7e-7 (1.9e-6); 162 us (148) and 2970 (3060).
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 constexpr int HBK = 16;          // complex k per stage = 32 real k = one MFMA k step
 constexpr int HKS = 2 * HBK + 8; // LDS row stride in bf16 (16-byte aligned rows, padded)
@@ -264,12 +304,13 @@ __device__ inline void split3(float x, __bf16& h0, __bf16& h1, __bf16& h2) {
 }
 
 template <typename TA, typename TB, int TRANSA, int WM, int WN>
-__global__ void __launch_bounds__(64 * WM * WN)
+__global__ void __launch_bounds__(64 * WM * WN, 2)
 k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const cplx<TB>* __restrict__ B,
            long ldb, int kchunk, GemmOut o, int tm, int tn, int nz) {
   constexpr int NT = 64 * WM * WN;
   constexpr int BMC = 32 * WM, BNC = 32 * WN;
   constexpr int NA = (BMC * HBK) / NT, NB = (BNC * HBK) / NT;
+  constexpr int CHAIN = TRANSA ? 2 : 1;   // stages whose products one FP32 accumulator takes
   static_assert(NA >= 1 && NB >= 1 && (BMC * HBK) % NT == 0 && (BNC * HBK) % NT == 0, "tile");
   __shared__ __attribute__((aligned(16))) __bf16 As[3][2 * BMC][HKS];  // [part][real row][real k]
   __shared__ __attribute__((aligned(16))) __bf16 Bs[3][BNC][HKS];      // [part][column][real k]
@@ -288,6 +329,13 @@ k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0f;
+  v4f sum[4][2];   // sums of the chains that are finished
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum[i][j][r] = 0.0f;
   const int li = lane & 15, lg = lane >> 4;
 
   cplx<TA> ra[NA];
@@ -370,6 +418,18 @@ k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
     }
   };
 
+  auto fold = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sum[i][j][r] += acc[i][j][r];
+          acc[i][j][r] = 0.0f;
+        }
+  };
+
   if (kbeg < kend) load_stage(kbeg);
   for (int k0 = kbeg; k0 < kend; k0 += HBK) {
     store_stage();
@@ -399,8 +459,10 @@ k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
             acc[rt][ct] =
                 __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[PA[pr]][rt], b[PB[pr]][ct], acc[rt][ct], 0, 0, 0);
     }
+    if ((k0 - kbeg) / HBK % CHAIN == CHAIN - 1) fold();
     __syncthreads();
   }
+  fold();
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
@@ -409,7 +471,7 @@ k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
       for (int p = 0; p < 2; ++p) {
         const int ip = wm * 64 + rt * 16 + 4 * lg + 2 * p;
         gemm_store(o, M, N, z, m0 + (ip >> 1), n0 + wn * 32 + ct * 16 + li,
-                   mk((double)acc[rt][ct][2 * p], (double)acc[rt][ct][2 * p + 1]));
+                   mk((double)sum[rt][ct][2 * p], (double)sum[rt][ct][2 * p + 1]));
       }
 }
 
@@ -428,13 +490,9 @@ __global__ void k_zgemm_reduce(int M, int N, int nz, GemmOut o) {
 // Si64 (1.2e9).
 constexpr double GEMM_SPLIT_MIN = 8589934592.0;
 
-// k-steps that one FP32 accumulator of the shared-tile kernels takes before its sum goes to FP64:
-// as long as the chains of the kernel these replaced (Si64 30 Ha projector products, error of
-// op_H against FP64: 1.3e-8 with 128, 2.2e-8 with 704, 1.7e-8 before).
-constexpr int GEMM_F32_CHAIN = 128;
-
 // Split of K over `nz` chunks for about `slots` workgroups on `tiles` tiles (no chunk shorter
-// than `kmin`), the partial-sum workspace and the epilogue.
+// than `kmin`, none longer than `kmax` where that is set: FP32 sums), the partial-sum workspace
+// and the epilogue.
 struct GemmSplit {
   int nz = 1, kchunk = GBK;
   long nwg = 0;
@@ -485,7 +543,8 @@ static int zgemm_launch(pw_ctx* c, int transa, int M, int N, int K, cplx<double>
   constexpr int BMC = 32 * WM, BNC = 32 * WN;
   const int tm = (M + BMC - 1) / BMC, tn = (N + BNC - 1) / BNC;
   GemmSplit g;
-  int rc = gemm_split(c, M, N, K, (long)tm * tn, target_wg, 128, 0, alpha, beta, C, ldc, kin, g);
+  int rc = gemm_split(c, M, N, K, (long)tm * tn, target_wg, 128, sizeof(TC) == 4 ? 8192 : 0, alpha, beta, C, ldc,
+                      kin, g);
   if (rc) return rc;
   bool split_bf16 = false;
   // the three-part operands of a 128 x 128 tile do not fit in LDS: that shape keeps FP32 MFMA
@@ -526,7 +585,8 @@ static int zgemm_wk_launch(pw_ctx* c, int transa, int M, int N, int K, cplx<doub
                            const GemmKin& kin, int target_wg) {
   const int tm = (M + 16 * T - 1) / (16 * T), tn = (N + 16 * T - 1) / (16 * T);
   GemmSplit g;
-  int rc = gemm_split(c, M, N, K, (long)tm * tn, target_wg, 16 * 4 * WK, sizeof(TC) == 4 ? GEMM_F32_CHAIN * 4 * WK : 0, alpha, beta, C, ldc, kin, g);
+  int rc = gemm_split(c, M, N, K, (long)tm * tn, target_wg, 16 * 4 * WK,
+                      sizeof(TC) == 4 ? 512 * WK : 0, alpha, beta, C, ldc, kin, g);
   if (rc) return rc;
   ProfScope ps(c, transa ? PW_PROF_GEMM_CN : PW_PROF_GEMM_NN,
                (double)M * K * sizeof(cplx<TA>) + (double)K * N * sizeof(cplx<TB>) +
@@ -559,9 +619,10 @@ static int zgemm_t(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alph
   //    share a 32 x 32 tile's K, which quarters the partial sums (FP64 160 x 160 x 23871: 88
   //    against 114 with a tile per wavefront; FP32 320 x 160 x 23871: 136 against 145); from 64
   //    tiles on, in FP64, a tile per wavefront, whose neighbours share its loads in L1 (1080 x
-  //    480 x 80797: 5470 with 8 wavefronts against 8290).  FP32 keeps the shared tile, whose
-  //    chains of FP32 sums are a quarter as long (320 x 243 x 67500: 620 against 585, with half
-  //    the rounding error);
+  //    480 x 80797: 5470 with 8 wavefronts against 8290).  FP32 keeps the shared tile: a tile per
+  //    wavefront is 9 % faster or slower by size (320 x 243 x 67500: 623 against 571, 700 x 400 x
+  //    30000: 1056 against 1152, 500 x 300 x 9000: 213 against 196, 240 x 200 x 30000: 227
+  //    against 242), its error half again as large;
   //  - A B that fills the chip: a tile per wavefront in FP64 (23871 x 160 x 160: 91 against
   //    105), four per tile in FP32, whose shorter MFMAs leave less time per load (23871 x 160 x
   //    320: 108 against 130).

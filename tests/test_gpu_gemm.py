@@ -58,3 +58,37 @@ def test_zgemm_edges(ctx, shape, transa, tile):
     finally:
         for key in (0, 1):
             ctx.call("pw_tune_set", key, -1)
+
+
+# (tile code, split-BF16 switch, transa, (M, N, K)): the kernels of the mixed path over long and short K
+F32_SUMS = [(-1, -1, 1, (500, 300, 9000)), (0, 0, 1, (700, 400, 12000)), (4, 0, 1, (300, 100, 9001)),
+            (5, 1, 1, (700, 400, 12000)), (1, 1, 1, (500, 300, 9000)), (6, 0, 1, (40, 20, 30000)),
+            (-1, -1, 0, (9000, 300, 500)), (0, 0, 0, (9000, 300, 500)), (0, 1, 0, (9000, 300, 500))]
+
+
+@pytest.mark.parametrize("tile,split,transa,shape", F32_SUMS)
+def test_f32_product_error(ctx, tile, split, transa, shape):
+    """The 2-norm error of FP32 products against FP64: operands rounded to FP32 (u / sqrt(3) each, u =
+    2^-24), sums in chains of at most 48 additions and second sums of at most 512: random roundings of
+    the running sum, sqrt(48 / 6) u and sqrt(512 / 6) u at worst, are 10 u in quadrature; 8 u is asked,
+    as no case here has more than 200 second additions (6 u)."""
+    from pwdft_hip._lib import DeviceMatrix, PW_MIXED, ptr
+    M, N, K = shape
+    rng = np.random.default_rng(K)
+    a = rng.standard_normal((K, M) if transa else (M, K)) + 1j * rng.standard_normal((K, M) if transa else (M, K))
+    b = rng.standard_normal((K, N)) + 1j * rng.standard_normal((K, N))
+    ref = (a.conj().T if transa else a) @ b
+    one, zero = np.array([1.0, 0.0]), np.zeros(2)
+    dA, dB, dC = DeviceMatrix.from_host(ctx, a), DeviceMatrix.from_host(ctx, b), DeviceMatrix(ctx, M, N)
+    try:
+        for key, value in ((0, tile), (1, tile), (8, split)):
+            ctx.call("pw_tune_set", key, value)
+        print(f"case zgemm FP32 sums {shape} transa={transa} tile={tile} split={split}", flush=True)
+        ctx.call("pw_zgemm_dev", transa, M, N, K, ptr(one), dA.p, dA.rows, dB.p, dB.rows, ptr(zero), dC.p, M, PW_MIXED)
+        got = dC.download()
+    finally:
+        for key in (0, 1, 8):
+            ctx.call("pw_tune_set", key, -1)
+    assert np.linalg.norm(got - ref) <= 8 * 2.0 ** -24 * np.linalg.norm(ref)
+    for d in (dA, dB, dC):
+        d.free()
