@@ -19,8 +19,8 @@ includes a neighbour's; the result is kept only if the whole op_H beats the sett
 context ran on entry (timed alternately with them, at least 1 % faster).
 
 The chosen settings are applied with pw_tune_set and cached in a JSON file keyed by the
-shape (grid, plane waves, projectors, bands, precision), so a later Hamiltonian of the same
-shape applies them without timing (Hamiltonian(..., autotune=True)).  Settings change the
+shape (grid, plane waves, projectors, bands, precision), with the generation of the kernels they
+were timed on, so a later Hamiltonian of the same shape applies them without timing (Hamiltonian(..., autotune=True)).  Settings change the
 order of floating-point operations only; the tests check that a tuned op_H equals the
 default one to rounding."""
 import json
@@ -35,6 +35,11 @@ from ._lib import DeviceMatrix, PW_MIXED, PW_TERM_ALL
  TUNE_PLANE_COMPRESSED, TUNE_OVERLAP, TUNE_COL_CHUNK, TUNE_GEMM_SPLIT_BF16) = range(9)
 TUNE_FFT_ORDER = 15
 SHAPES = {-1: "auto", 0: "64x64", 1: "128x64", 2: "64x128", 3: "128x128", 4: "128x32", 5: "64x32"}
+
+# Generation of the kernels that the settings name: raised whenever a code means another kernel than
+# before (2: the plane and column kernels, which a column chunk, a radix mode or a plane mode of the
+# general kernels switches off, and GEMM tiles without LDS).  An entry of another generation is timed anew.
+KERNELS = 2
 
 # the library's defaults (what a fresh context runs)
 DEFAULTS = {"fft_order": 0, "plane_compressed": 0, "col_chunk": 0, "band_batch": 64,
@@ -242,10 +247,10 @@ def autotune(H, nbands=None, mixed=None, cache=True, path=None, **kw):
     key = shape_key(H.pw.Ns, H.pw.Ngw[ik], H.pspotNL.NbetaNL, nb, mixed)
     if cache:
         hit = load_cache(path).get(key)
-        if isinstance(hit, dict):
+        if isinstance(hit, dict) and hit.get("kernels") == KERNELS:
             apply_settings(H.ctx, hit)
             return hit, "cache"
     settings, _ = tune_op_H(H, nbands=nb, mixed=mixed, **kw)
     if cache:
-        save_cache({key: settings}, path)
+        save_cache({key: dict(settings, kernels=KERNELS)}, path)
     return settings, "tuned"

@@ -310,3 +310,26 @@ def test_calc_rhoe_batch_arguments():
     H, ctx, psi, block = _rhoe_stub()
     calc_rhoe_(H, psi[:3] + [block(2)], out, np.full((3, 4), 2.0))
     assert [n for n, _ in ctx.calls].count("pw_rhoe_accum_dev") == 4
+
+
+def test_autotune_cache_of_other_kernels(tmp_path, monkeypatch):
+    """Settings timed on another generation of kernels (or before entries named one) are timed anew, not
+    applied: their codes may mean other kernels.  Host logic only, on a stand-in Hamiltonian."""
+    from types import SimpleNamespace
+    from pwdft_hip import autotune as at
+    calls = []
+    ctx = SimpleNamespace(call=lambda name, *a: calls.append((name, a)))
+    H = SimpleNamespace(ctx=ctx, mixed=False, pw=SimpleNamespace(Ns=(20, 20, 20), Ngw=[316]),
+                        pspotNL=SimpleNamespace(NbetaNL=4), electrons=SimpleNamespace(Nstates=8))
+    monkeypatch.setattr(at, "tune_op_H", lambda H, **kw: (dict(at.DEFAULTS, op_H_ms=1.0), []))
+    path = str(tmp_path / "tune.json")
+    key = at.shape_key((20, 20, 20), 316, 4, 8, False)
+    for stale in ({"fft_order": 2, "col_chunk": 16}, {"fft_order": 2, "kernels": at.KERNELS - 1}):
+        at.save_cache({key: stale}, path)
+        calls.clear()
+        settings, source = at.autotune(H, path=path)
+        assert source == "tuned" and settings["fft_order"] == 0
+        assert ("pw_tune_set", (at.TUNE_FFT_ORDER, 2)) not in calls
+        settings, source = at.autotune(H, path=path)
+        assert source == "cache" and settings["fft_order"] == 0
+        assert ("pw_tune_set", (at.TUNE_FFT_ORDER, 0)) in calls
