@@ -4,15 +4,18 @@ Every candidate is timed on the device with the library's own per-kernel events
 (pw_profile_*) on the Hamiltonian's largest k-point and its band count, in four stages, each
 keeping the best setting of the previous ones:
 
-1. FFT plans: the radix mode of the line FFTs (PW_TUNE_FFT_ORDER: 9 x 8 as compiled, the
-   same radices reversed, or radices 5/4/3/2 only) x the z-plane kernel (padded plane, or
-   the compressed plane of the active x lines) x the z-columns per workgroup of the column
-   passes, scored by the three FFT kernels' time;
+1. FFT plans: the radix mode of the line FFTs (PW_TUNE_FFT_ORDER: 0, the plane and column
+   kernels' two-pass plans with the largest radices first elsewhere; the general column
+   kernels with the same radices reversed, or with radices 5/4/3/2 only) x the z-plane kernel
+   (as sizes choose it, or the general compressed plane of the active x lines) x the z-columns
+   per workgroup of the general column kernels (0: as sizes choose), scored by the three FFT
+   kernels' time;
 2. the band split: bands per FFT launch (PW_TUNE_BAND_BATCH), same score;
-3. the projector GEMMs: tile shape and split-K workgroup target of beta^H psi and of
-   beta (D B), each scored by its own kernel time;
-4. whole-op_H choices scored by wall time: the nonlocal products on a second stream or
-   not, and (mixed precision) the BF16-split MFMA GEMM.
+3. the projector GEMMs: tile shape (a tile per wavefront, or one that four or eight
+   wavefronts share along K) and split-K workgroup target of beta^H psi and of beta (D B),
+   each scored by its own kernel time;
+4. whole-op_H choices scored by wall time: beta^H psi on a second stream where the sizes
+   make that pay or not, and (mixed precision) the BF16-split MFMA GEMM.
 
 Stages 1-3 score kernels run one at a time (no second stream), so that no kernel's time
 includes a neighbour's; the result is kept only if the whole op_H beats the settings the
@@ -34,7 +37,8 @@ from ._lib import DeviceMatrix, PW_MIXED, PW_TERM_ALL
 (TUNE_GEMM_CN_SHAPE, TUNE_GEMM_NN_SHAPE, TUNE_GEMM_CN_WG, TUNE_GEMM_NN_WG, TUNE_BAND_BATCH,
  TUNE_PLANE_COMPRESSED, TUNE_OVERLAP, TUNE_COL_CHUNK, TUNE_GEMM_SPLIT_BF16) = range(9)
 TUNE_FFT_ORDER = 15
-SHAPES = {-1: "auto", 0: "64x64", 1: "128x64", 2: "64x128", 3: "128x128", 4: "128x32", 5: "64x32"}
+SHAPES = {-1: "auto", 0: "64x64", 1: "128x64", 2: "64x128", 3: "128x128", 4: "128x32", 5: "64x32",
+          6: "16x16 by eight", 7: "32x32 by four"}
 
 # Generation of the kernels that the settings name: raised whenever a code means another kernel than
 # before (2: the plane and column kernels, which a column chunk, a radix mode or a plane mode of the
@@ -189,7 +193,7 @@ def tune_op_H(H, nbands=None, mixed=None, steps=3, quick=False):
         # 3. projector GEMMs (both products timed in one run per candidate)
         if H.pspotNL.NbetaNL > 0:
             bcn = bnn = None
-            shapes = (-1, 0, 5) if quick else (-1, 0, 1, 2, 4, 5)
+            shapes = (-1, 0, 5, 6, 7) if quick else (-1, 0, 1, 2, 4, 5, 6, 7)
             targets = (0, 512) if quick else (0, 256, 512, 1024, 2048)
             for shape in shapes:
                 for wg in targets:
