@@ -2,10 +2,12 @@
 oracle, through the C ABI.  Tolerances: FP64 path <= 1e-12 relative to max|ref| (FFT
 order and FMA contraction differ from numpy's; the arithmetic is the same); mixed path
 (FP32 FFT, FP32 MFMA projectors) <= 2e-5 relative."""
+import os
+
 import numpy as np
 import pytest
 
-from _systems import A_SI, oracle_ham, product_ham, rand_psi, rel, si_fcc_structure
+from _systems import A_SI, ROOT, oracle_ham, product_ham, rand_psi, rel, si_fcc_structure
 
 pytestmark = pytest.mark.gpu
 
@@ -270,9 +272,9 @@ def test_other_grids(case):
 
 @pytest.mark.parametrize("mixed", [False, True])
 def test_overlapped_nonlocal_stream(mixed):
-    """op_H with the nonlocal products on the second stream (default) against the
-    single-stream order, with and without accumulation, over several band batches; and a
-    captured op_H (fork and join inside the graph) replayed against the eager result."""
+    """op_H with the second stream allowed (default) and not, with and without accumulation, over
+    several band batches, and captured.  Si8 with 20 bands lies below the size from which op_H forks
+    (test_forked_projector_product has sizes on both sides): either setting runs one stream."""
     import pwdft_hip as ph
     from pwdft_hip._lib import PW_ACCUMULATE, PW_MIXED, PW_TERM_ALL
     atoms = ph.Atoms(["Si"] * 8, ph.diamond_supercell(1.0, 1), ph.gen_lattice_sc(10.2631))
@@ -303,3 +305,115 @@ def test_overlapped_nonlocal_stream(mixed):
         H.ctx.call("pw_synchronize")
         assert np.array_equal(out.download(), res[(1, 0)]), rep
     g.free()
+
+
+@pytest.fixture(scope="module")
+def si64():
+    """Si64, 15 Ha: 23 871 plane waves, 320 projectors."""
+    import pwdft_hip as ph
+    frac = np.array(ph.diamond_supercell(1.0, 2), dtype=float)
+    H = ph.Hamiltonian(ph.Atoms(["Si"] * 64, frac, ph.gen_lattice_sc(20.5262)), ["Si-q4.lda.gth"], 15.0,
+                       Ns_=(72, 72, 72), Nstates=160, use_symmetry=False)
+    H.update(H.guess_rhoe())
+    return H
+
+
+# bands on either side of the window in which op_H forks (beta^H psi beside the FFT passes), and in it
+@pytest.mark.parametrize("nb,forks", [(10, False), (12, True), (40, True), (78, True), (79, False)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_forked_projector_product(si64, nb, forks, mixed):
+    """op_H with beta^H psi on the second stream against one stream: bit for bit, with and without
+    accumulation, after another psi has filled the shared buffers (so a missing wait shows), and captured."""
+    import re
+    import pwdft_hip as ph
+    from pwdft_hip._lib import PW_ACCUMULATE, PW_MIXED, PW_TERM_ALL
+    H = si64
+    n, nbeta = int(H.pw.Ngw[0]), H.pspotNL.NbetaNL
+    # the window itself, from the rule in the source
+    src = open(os.path.join(ROOT, "pwdft.jl_amd", "csrc", "pw_capi.hip")).read()
+    lo = 1 << int(re.search(r"k\.ngw \* nb >= \(1L << (\d+)\)", src).group(1))
+    hi = float(re.search(r"\(double\)k\.ngw \* nb \* k\.nbeta < ([0-9.e+]+);", src).group(1))
+    assert forks == (n * nb >= lo and n * nb * nbeta < hi)
+    rng = np.random.default_rng(nb)
+    psi = ph.DeviceMatrix.from_host(H.ctx, rand_psi(rng, n, nb))
+    other = ph.DeviceMatrix.from_host(H.ctx, rand_psi(rng, n, nb))
+    scratch = ph.DeviceMatrix(H.ctx, n, nb)
+    h0 = rand_psi(rng, n, nb)
+    flags = PW_TERM_ALL | (PW_MIXED if mixed else 0)
+    print(f"case fork nb={nb} forks={forks} mixed={mixed}", flush=True)
+    res = {}
+    try:
+        for ov in (0, 1):
+            H.ctx.call("pw_tune_set", 6, ov)
+            for acc in (0, PW_ACCUMULATE):
+                H.ctx.call("pw_op_H_dev", 0, 0, nb, other.p, n, scratch.p, n, flags)
+                out = ph.DeviceMatrix.from_host(H.ctx, h0 if acc else np.full((n, nb), np.nan + 0j))
+                H.ctx.call("pw_op_H_dev", 0, 0, nb, psi.p, n, out.p, n, flags | acc)
+                res[(ov, acc)] = out.download()
+                out.free()
+    finally:
+        H.ctx.call("pw_tune_set", 6, 1)
+    for acc in (0, PW_ACCUMULATE):
+        assert np.array_equal(res[(1, acc)], res[(0, acc)]), acc
+    out = ph.DeviceMatrix(H.ctx, n, nb)
+    with ph.Graph(H.ctx) as g:
+        H.ctx.call("pw_op_H_dev", 0, 0, nb, psi.p, n, out.p, n, flags)
+    for rep in range(3):
+        H.ctx.call("pw_op_H_dev", 0, 0, nb, other.p, n, scratch.p, n, flags)
+        out.upload(np.full((n, nb), np.nan + 0j))
+        g.launch()
+        H.ctx.call("pw_synchronize")
+        assert np.array_equal(out.download(), res[(1, 0)]), rep
+    g.free()
+    for d in (psi, other, scratch, out):
+        d.free()
+
+
+# product kernels that add the kinetic term: the rule's own, an explicit tile, K split over workgroups (the
+# reduction adds it), and the split-BF16 kernel with and without that split
+KIN_GEMM = [((), False), ((), True), (((1, 0),), False), (((1, 0), (3, 2048)), False), (((1, 0), (3, 2048)), True),
+            (((8, 1), (1, 0)), True), (((8, 1), (1, 0), (3, 2048)), True)]
+
+
+@pytest.mark.parametrize("tune,mixed", KIN_GEMM)
+@pytest.mark.parametrize("acc", [False, True])
+def test_op_H_term_subsets(si64, tune, mixed, acc):
+    """Every subset of the terms, psi and Hpsi in larger arrays, against the sum of the terms applied one by
+    one; what Hpsi held is added to or (NaN) never read."""
+    import pwdft_hip as ph
+    from pwdft_hip._lib import PW_ACCUMULATE, PW_MIXED, PW_TERM_K, PW_TERM_NLOC, PW_TERM_VLOC
+    H = si64
+    n, nb, ldp, ldh = int(H.pw.Ngw[0]), 6, int(H.pw.Ngw[0]) + 5, int(H.pw.Ngw[0]) + 2
+    rng = np.random.default_rng(3)
+    full = np.full((ldp, nb), np.nan + 0j, order="F")
+    full[:n] = rand_psi(rng, n, nb)
+    psi = ph.DeviceMatrix.from_host(H.ctx, full)
+    old = np.full((ldh, nb), np.nan + 0j, order="F")
+    if acc:
+        old[:n] = rand_psi(rng, n, nb)
+    m = PW_MIXED if mixed else 0
+
+    def apply(terms, start, flags):
+        out = ph.DeviceMatrix.from_host(H.ctx, start)
+        H.ctx.call("pw_op_H_dev", 0, 0, nb, psi.p, ldp, out.p, ldh, terms | flags)
+        got = out.download()
+        out.free()
+        assert np.all(np.isnan(got[n:])), "rows past Hpsi were written"
+        return got[:n]
+
+    blank = np.full((ldh, nb), np.nan + 0j, order="F")
+    one = {t: apply(t, blank, m) for t in (PW_TERM_K, PW_TERM_VLOC, PW_TERM_NLOC)}
+    assert np.abs(one[PW_TERM_K] - 0.5 * H.pw.gk2(0)[:, None] * full[:n]).max() <= 1e-14 * np.abs(one[PW_TERM_K]).max()
+    try:
+        for key, value in tune:
+            H.ctx.call("pw_tune_set", key, value)
+        for bits in range(1, 8):
+            terms = [t for i, t in enumerate(one) if bits >> i & 1]
+            print(f"case op_H terms={terms} tune={tune} mixed={mixed} acc={acc}", flush=True)
+            got = apply(sum(terms), old, m | (PW_ACCUMULATE if acc else 0))
+            ref = sum(one[t] for t in terms) + (old[:n] if acc else 0)
+            assert rel(got, ref) <= (2e-6 if mixed else 1e-13), terms
+    finally:
+        for key, value in ((1, -1), (3, 0), (8, -1)):
+            H.ctx.call("pw_tune_set", key, value)
+    psi.free()
