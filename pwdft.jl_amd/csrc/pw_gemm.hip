@@ -291,7 +291,9 @@ k_zgemm_wk(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
 // 16x16x4 MFMA, so the tiles, split-K and epilogue are those of k_zgemm.
 // As in WaveTile an accumulator takes a short chain (one stage, two for A^H B, whose K is long)
 // and is then added to a second one: error of A B 23871 x 160 x 320 1.0e-7 (3.8e-7 with one
-// chain), of A^H B 1080 x 480 x 80797 3.7e-7 (1.9e-6); 162 us (148) and 2970 (3060).
+// chain), of A^H B 1080 x 480 x 80797 3.7e-7 (1.9e-6), 67500 x 320 x 480 912 us (892).  A B in
+// tiles of eight wavefronts keeps one chain over its short K: two of its workgroups share a CU at
+// 128 registers, and with second accumulators one does (67500 x 480 x 320: 1103 us, 1489).
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 constexpr int HBK = 16;          // complex k per stage = 32 real k = one MFMA k step
 constexpr int HKS = 2 * HBK + 8; // LDS row stride in bf16 (16-byte aligned rows, padded)
@@ -304,13 +306,14 @@ __device__ inline void split3(float x, __bf16& h0, __bf16& h1, __bf16& h2) {
 }
 
 template <typename TA, typename TB, int TRANSA, int WM, int WN>
-__global__ void __launch_bounds__(64 * WM * WN, 2)
+__global__ void __launch_bounds__(64 * WM * WN, WM * WN == 8 && !TRANSA ? 4 : 2)
 k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const cplx<TB>* __restrict__ B,
            long ldb, int kchunk, GemmOut o, int tm, int tn, int nz) {
   constexpr int NT = 64 * WM * WN;
   constexpr int BMC = 32 * WM, BNC = 32 * WN;
   constexpr int NA = (BMC * HBK) / NT, NB = (BNC * HBK) / NT;
-  constexpr int CHAIN = TRANSA ? 2 : 1;   // stages whose products one FP32 accumulator takes
+  constexpr bool WIDE = TRANSA || WM * WN < 8;
+  constexpr int CHAIN = TRANSA ? 2 : 1;   // WIDE: stages whose products one FP32 accumulator takes
   static_assert(NA >= 1 && NB >= 1 && (BMC * HBK) % NT == 0 && (BNC * HBK) % NT == 0, "tile");
   __shared__ __attribute__((aligned(16))) __bf16 As[3][2 * BMC][HKS];  // [part][real row][real k]
   __shared__ __attribute__((aligned(16))) __bf16 Bs[3][BNC][HKS];      // [part][column][real k]
@@ -329,7 +332,7 @@ k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0f;
-  v4f sum[4][2];   // sums of the chains that are finished
+  v4f sum[4][2];   // WIDE: sums of the chains that are finished
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -459,7 +462,8 @@ k_zgemm_b3(int M, int N, int K, const cplx<TA>* __restrict__ A, long lda, const 
             acc[rt][ct] =
                 __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[PA[pr]][rt], b[PB[pr]][ct], acc[rt][ct], 0, 0, 0);
     }
-    if ((k0 - kbeg) / HBK % CHAIN == CHAIN - 1) fold();
+    if constexpr (WIDE)
+      if ((k0 - kbeg) / HBK % CHAIN == CHAIN - 1) fold();
     __syncthreads();
   }
   fold();
