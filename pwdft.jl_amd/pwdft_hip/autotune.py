@@ -15,7 +15,8 @@ keeping the best setting of the previous ones:
    wavefronts share along K) and split-K workgroup target of beta^H psi and of beta (D B),
    each scored by its own kernel time;
 4. whole-op_H choices scored by wall time: beta^H psi on a second stream where the sizes
-   make that pay or not, and (mixed precision) the BF16-split MFMA GEMM.
+   make that pay or not, and (mixed precision) the BF16-split MFMA GEMM off or on, each with
+   the tiles of stage 3 timed under it.
 
 Stages 1-3 score kernels run one at a time (no second stream), so that no kernel's time
 includes a neighbour's; the result is kept only if the whole op_H beats the settings the
@@ -191,36 +192,44 @@ def tune_op_H(H, nbands=None, mixed=None, steps=3, quick=False):
                 best["band_batch"] = bb
         apply_settings(c, {"band_batch": best["band_batch"]})
         # 3. projector GEMMs (both products timed in one run per candidate)
-        if H.pspotNL.NbetaNL > 0:
-            bcn = bnn = None
+        def products(split):
+            """The best tiles and targets of both products under one split-BF16 setting.  Codes 6 and 7 run
+            FP32 MFMA under any, so with it on either product can still go without."""
             shapes = (-1, 0, 5, 6, 7) if quick else (-1, 0, 1, 2, 4, 5, 6, 7)
             targets = (0, 512) if quick else (0, 256, 512, 1024, 2048)
+            bcn = bnn = None
+            apply_settings(c, {"gemm_split_bf16": split, "overlap": 0})
             for shape in shapes:
                 for wg in targets:
                     apply_settings(c, {"gemm_cn_shape": shape, "gemm_nn_shape": shape, "gemm_cn_wg": wg,
                                        "gemm_nn_wg": wg})
                     t = _profiled(H, X, Y, flags, steps)
-                    table.append({"gemm_shape": SHAPES[shape], "gemm_wg": wg, "gemm_cn_ms": t["gemm_cn"],
-                                  "gemm_nn_ms": t["gemm_nn"]})
+                    table.append({"gemm_shape": SHAPES[shape], "gemm_wg": wg, "gemm_split_bf16": split,
+                                  "gemm_cn_ms": t["gemm_cn"], "gemm_nn_ms": t["gemm_nn"]})
                     if bcn is None or t["gemm_cn"] < bcn[0]:
                         bcn = (t["gemm_cn"], shape, wg)
                     if bnn is None or t["gemm_nn"] < bnn[0]:
                         bnn = (t["gemm_nn"], shape, wg)
-            best.update(gemm_cn_shape=bcn[1], gemm_cn_wg=bcn[2], gemm_nn_shape=bnn[1], gemm_nn_wg=bnn[2])
+            return {"gemm_cn_shape": bcn[1], "gemm_cn_wg": bcn[2], "gemm_nn_shape": bnn[1], "gemm_nn_wg": bnn[2],
+                    "gemm_split_bf16": split}
+        nonlocal_term = H.pspotNL.NbetaNL > 0
+        if nonlocal_term:
+            best.update(products(best["gemm_split_bf16"]))
         apply_settings(c, best)
         # 4. whole op_H: second stream, BF16-split GEMMs (mixed only), by wall time
         wall = _wall(H, X, Y, flags, 3 * steps)
-        for key, vals in (("overlap", (1, 0)), ("gemm_split_bf16", (-1, 0, 1) if mixed else ())):
-            for v in vals:
-                if v == best[key]:
-                    continue
-                apply_settings(c, {key: v})
-                w = _wall(H, X, Y, flags, 3 * steps)
-                table.append({key: v, "op_H_ms": w})
-                if w < wall:
-                    wall = w
-                    best[key] = v
-            apply_settings(c, best)
+        cands = [lambda: {"overlap": 1 - best["overlap"]}]
+        if mixed and nonlocal_term:
+            cands += [lambda: products(0), lambda: products(1)]
+        for cand in cands:
+            new = cand()
+            apply_settings(c, dict(best, **new))
+            w = _wall(H, X, Y, flags, 3 * steps)
+            table.append(dict(new, op_H_ms=w))
+            if w < wall:
+                wall = w
+                best.update(new)
+        apply_settings(c, best)
         # final check, entry and tuned settings timed alternately (drift and noise hit both):
         # the tuned ones are kept only if at least 1 % faster
         t_entry, t_best = float("inf"), float("inf")
