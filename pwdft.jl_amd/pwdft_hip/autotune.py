@@ -206,10 +206,14 @@ def tune_op_H(H, nbands=None, mixed=None, steps=3, quick=False):
                     t = _profiled(H, X, Y, flags, steps)
                     table.append({"gemm_shape": SHAPES[shape], "gemm_wg": wg, "gemm_split_bf16": split,
                                   "gemm_cn_ms": t["gemm_cn"], "gemm_nn_ms": t["gemm_nn"]})
-                    if bcn is None or t["gemm_cn"] < bcn[0]:
-                        bcn = (t["gemm_cn"], shape, wg)
-                    if bnn is None or t["gemm_nn"] < bnn[0]:
-                        bnn = (t["gemm_nn"], shape, wg)
+                    # the solvers' own products run under these settings too: a tile other than the
+                    # rules' (-1, 7) must be a tenth faster, or a smaller product loses what op_H gains
+                    # (mixed LOBPCG at Si64, A^H B in 64 x 64 tiles: 7.7 against 7.4 ms an iteration)
+                    f = 1.0 if shape in (-1, 7) else 1.1
+                    if bcn is None or f * t["gemm_cn"] < bcn[0]:
+                        bcn = (f * t["gemm_cn"], shape, wg)
+                    if bnn is None or f * t["gemm_nn"] < bnn[0]:
+                        bnn = (f * t["gemm_nn"], shape, wg)
             return {"gemm_cn_shape": bcn[1], "gemm_cn_wg": bcn[2], "gemm_nn_shape": bnn[1], "gemm_nn_wg": bnn[2],
                     "gemm_split_bf16": split}
         nonlocal_term = H.pspotNL.NbetaNL > 0
