@@ -74,15 +74,18 @@ enum {
   PW_TUNE_GEMM_NN_WG = 3,     /* A B split-K target workgroup count (0 = default, the same) */
   PW_TUNE_BAND_BATCH = 4,     /* bands per fused FFT launch (same as pw_set_band_batch) */
   PW_TUNE_PLANE_COMPRESSED = 5, /* 1: always use the general compressed z-plane kernels (they are
-                                   used anyway for line lengths without a two-pass plan); 2:
-                                   always the global-plane pass (compressed planes in HBM, used
-                                   anyway when even the compressed plane exceeds LDS) */
+                                   used anyway for line lengths without a two-pass plan whose
+                                   padded plane exceeds LDS); 2: always the global-plane pass
+                                   (compressed planes in HBM, used anyway when even the
+                                   compressed plane exceeds LDS) */
   PW_TUNE_OVERLAP = 6,          /* 1 (default): op_H runs beta^H psi on a second stream
                                    beside the FFT passes where the sizes make that pay (2^18
                                    sphere entries to 6e8 multiply-adds); 0: one stream, in
                                    sequence */
-  PW_TUNE_COL_CHUNK = 7,        /* z-columns per workgroup of the column FFT kernels (0: the
-                                   default, as many as 48 KiB of LDS hold) */
+  PW_TUNE_COL_CHUNK = 7,        /* 0 (default): the column FFT kernels with two-pass plans, or where
+                                   the length has none the general ones with as many z-columns
+                                   per workgroup as 48 KiB of LDS hold; > 0: the general ones
+                                   with that many */
   PW_TUNE_GEMM_SPLIT_BF16 = 8,  /* the mixed path's complex GEMMs on BF16 MFMA with each operand
                                    split in three BF16 parts (FP32-level accuracy): 1 always,
                                    0 never, -1 (default) for products of >= 2^33 complex
@@ -111,16 +114,18 @@ enum {
                                    2 one exchange per column (the owner of the next
                                    column publishes it with its p segments and every
                                    workgroup forms the next reflector itself), each value
-                                   its own arrival flag (n = 480: 2.2 ms,
-                                   n = 960: 6.3 ms); 1 two exchanges per column (the owner
-                                   publishes the next reflector), device-coherent atomic
-                                   accesses, each producer waiting for its stores before the
-                                   flag (n = 480: 10.8 ms, n = 960: 21.4 ms); 0 two exchanges
-                                   ordered by agent-scope fences (12.2, 33.4 ms) */
+                                   its own arrival flag (eigenvalues of n = 480: 4.4 ms,
+                                   n = 960: 10.4 ms, of which the reduction 2.2 and 6.3); 1 two
+                                   exchanges per column (the owner publishes the next reflector),
+                                   device-coherent atomic accesses, each producer waiting for its
+                                   stores before the flag (5.5, 12.7 ms); 0 two exchanges ordered
+                                   by agent-scope fences (9.3, 28.5 ms) */
   PW_TUNE_FFT_ORDER = 15,       /* radix plan of the FFT lines outside the plane kernels, which
-                                   have their own plans: 0 (default) largest radices
-                                   first (72 = 9 x 8, compile-time specialised); 1 the same
-                                   radices in reverse order; 2 radices 5, 4, 3, 2 only */
+                                   have their own plans: 0 (default) the column kernels' two-pass
+                                   plans, elsewhere largest radices first (72 = 9 x 8,
+                                   compile-time specialised); 1 the general column kernels, the
+                                   same radices in reverse order; 2 the same with radices 5, 4,
+                                   3, 2 only */
   PW_TUNE_BATCH_GEMM_SMALL = 16, /* pw_zgemm_batch_dev and the batched solvers: 1 (default) the
                                    small-product kernels (A B with k <= 64 and n <= 32: one
                                    thread per row; A^H B with m, n <= 32: one workgroup per

@@ -489,9 +489,12 @@ __global__ void k_zgemm_reduce(int M, int N, int nz, GemmOut o) {
   }
 }
 
-// Complex multiply-adds from which the split-BF16 kernel takes FP32 products by default: it pays
-// off on large ones (Si216's projector and Gram products, 4e10), not beside the FFT passes at
-// Si64 (1.2e9).
+// Complex multiply-adds from which the split-BF16 kernel takes FP32 products by default: Si216's
+// projector and Gram products (4e10).  Where it pays depends on both columns and size; op_H with FP32
+// products / with split ones, one after the other, us: 72^3, 320 projectors, 80 bands (6e8) 277 /
+// 299, 120 bands 394 / 386, 160 bands (1.2e9) 520 / 495, 240 bands 796 / 723, 480 bands (3.7e9)
+// 1618 / 1753; 108^3, 243 bands (5.3e9) 2562 / 2230, 480 bands (1e10) 4966 / 5097.  Its error on
+// long sums is up to twice the FP32 kernels', so below the line it is left to the autotuner.
 constexpr double GEMM_SPLIT_MIN = 8589934592.0;
 
 // Split of K over `nz` chunks for about `slots` workgroups on `tiles` tiles (no chunk shorter
@@ -629,7 +632,7 @@ static int zgemm_t(pw_ctx* c, int transa, int M, int N, int K, cplx<double> alph
   //    against 242), its error half again as large;
   //  - A B that fills the chip: a tile per wavefront in FP64 (23871 x 160 x 160: 91 against
   //    105), four per tile in FP32, whose shorter MFMAs leave less time per load (23871 x 160 x
-  //    320: 108 against 130).
+  //    320: 128 against 148).
   if constexpr (sizeof(TC) == 4) {
     if (shape < 0 && (c->gemm_split_bf16 > 0 || (c->gemm_split_bf16 < 0 && work >= GEMM_SPLIT_MIN))) {
       // the split-BF16 kernel's tiles

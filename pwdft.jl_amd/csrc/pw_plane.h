@@ -14,9 +14,9 @@
 // it in registers where the inverse transform ends and the forward one begins.  The plane needs
 // two workgroup barriers.
 //
-// What bounds it: FP32 VALU issue (72^2: ~6 400 vector instructions per plane and SIMD, 70 % of
-// them butterflies), FP64 LDS bandwidth and the two wavefronts per SIMD that its registers
-// leave.  Per launch of 160 bands at 72^3 (a kernel with the whole padded plane in LDS, radix 9 x
+// What bounds it (counters, 72^3, 160 bands): the LDS pipes, active for 65 % of the cycles in FP64
+// and 71 % in FP32, about half of that bank conflicts; FP32 vector issue too (67 %; FP64 36 %), and
+// in FP64 the two wavefronts per SIMD that its registers leave.  Per launch of 160 bands at 72^3 (a kernel with the whole padded plane in LDS, radix 9 x
 // 8, before): FP64 338 us (498), FP32 176 us (203); 108^3, 243 bands: FP32 1.0 ms (3.4 ms with
 // three radix passes), FP64 86 ns per plane.
 #pragma once

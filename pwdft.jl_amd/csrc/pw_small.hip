@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(SM_NT) k_heev_jacobi(cplx<double>* __restrict_
 
 // The same solver for n <= 32, built for the length of a round, which the rotation parameters'
 // serial chain, the barriers and the instructions around them set (mean per solve over an SCF of
-// Si2, n = 24: 184 us, 16: 76, 8: 17; 110 over the three orders with the kernel above, 78 now):
+// Si2, n = 24: 186 us, 16: 76, 8: 17; 110 over the three orders with the kernel above, 78 now):
 //  - A is updated from one buffer into another, so a round has one barrier: every wavefront
 //    computes all rotation parameters for itself from the buffer nobody writes;
 //  - a thread keeps one block of A or one pair of V for the whole solve (no index division per
